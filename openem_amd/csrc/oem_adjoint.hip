@@ -57,7 +57,7 @@ struct AdjDev {
     GridDev g;
     MatDev mat;
     float ch;
-    size_t ncell;
+    size_t ncell;                // cells of a component, row padding included
     int chunk;                   // x planes per block of the transposes
 };
 
@@ -128,7 +128,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_e1(AdjDev d)
     }
     const GridDev &g = d.g;
     const AxisDev &X = g.ax[0], &Y = g.ax[1], &Z = g.ax[2];
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const int nx = g.nx, ny = g.ny, nz = g.nz, pz = g.pz;
     // one (j, k) column per thread, numbered along the plane: no idle lanes when nz is not a
     // multiple of 64 (a 48-cell-thick slab leaves a quarter of (k, j) tiles empty).  Threads
     // past the last column take the last one and store nothing: every thread reaches the
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_e1(AdjDev d)
     const int q = act ? base + tid : ny * nz - 1;
     const int j = q / nz, k = q - j * nz;
     const int i0 = blockIdx.z * d.chunk, i1 = min(i0 + d.chunk, nx);
-    const uint32_t nc = (uint32_t)d.ncell, plane = (uint32_t)(ny * nz);
+    const uint32_t nc = (uint32_t)d.ncell, plane = (uint32_t)(ny * pz);
     const int wy = Y.lo + Y.hi, wz = Z.lo + Z.hi;
     const uint32_t *off = d.psl.off;
     // buffer resources (the x march's per-plane offsets go in SGPRs): the three components of
@@ -167,10 +167,10 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_e1(AdjDev d)
     const bool y_lds = y_nb && ly >= 0 && ly < OEM_ADJ_TK * OEM_ADJ_TJ;
     const bool z_lds = z_nb && lz >= 0 && lz < OEM_ADJ_TK * OEM_ADJ_TJ;
     // per-thread byte offsets within a plane: the cell, its y and z neighbours, their psi rows
-    const uint32_t vo = (uint32_t)(j * nz + k) * EB, vyn = (uint32_t)(jn * nz + k) * EB,
-                   vzn = (uint32_t)(j * nz + kn) * EB;
-    const uint32_t vpy = (uint32_t)(max(yc.s, 0) * nz + k) * EB;
-    const uint32_t vpyn = (uint32_t)(max(yn.s, 0) * nz + k) * EB;
+    const uint32_t vo = (uint32_t)(j * pz + k) * EB, vyn = (uint32_t)(jn * pz + k) * EB,
+                   vzn = (uint32_t)(j * pz + kn) * EB;
+    const uint32_t vpy = (uint32_t)(max(yc.s, 0) * pz + k) * EB;
+    const uint32_t vpyn = (uint32_t)(max(yn.s, 0) * pz + k) * EB;
     const uint32_t vpz = (uint32_t)(j * wz + max(zc.s, 0)) * EB;
     const uint32_t vpzn = (uint32_t)(j * wz + max(zn.s, 0)) * EB;
     int buf = 0;
@@ -197,7 +197,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_e1(AdjDev d)
         const uint32_t sp = (uint32_t)i * plane * EB;
         const AxAt xc = ax_at_row(X, nx, i, AX_AE, AX_KE, AX_IDLD, AX_MPV);
         float bx, by, bz;
-        cbs(cls_at(vo, sp), (uint32_t)i * plane + (uint32_t)(j * nz + k), bx, by, bz);
+        cbs(cls_at(vo, sp), (uint32_t)i * plane + (uint32_t)(j * pz + k), bx, by, bz);
         const F nu1 = by * (zc.pec * xc.pec) * T::ld(rE, vo, sp + cB);
         const F nu2 = bz * (xc.pec * yc.pec) * T::ld(rE, vo, sp + 2u * cB);
         F p0 = T::zero(), p1 = T::zero();
@@ -224,9 +224,9 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_e1(AdjDev d)
         if (x_nb_top) qx(inb, q3n, q4n);
     }
     for (int i = i1 - 1; i >= i0; --i) {
-        const uint32_t id = (uint32_t)i * plane + (uint32_t)(j * nz + k);
+        const uint32_t id = (uint32_t)i * plane + (uint32_t)(j * pz + k);
         const uint32_t sp = (uint32_t)i * plane * EB;
-        const uint32_t sy = (uint32_t)i * (uint32_t)(wy * nz) * EB;
+        const uint32_t sy = (uint32_t)i * (uint32_t)(wy * pz) * EB;
         const uint32_t sz = (uint32_t)i * (uint32_t)(ny * wz) * EB;
         const AxAt xc = ax_at_row(X, nx, i, AX_AE, AX_KE, AX_IDLD, AX_MPV);
         const uint32_t sx = (uint32_t)max(xc.s, 0) * plane * EB;
@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_e1(AdjDev d)
         F q0n = T::zero(), q5n = T::zero(), q1n = T::zero(), q2n = T::zero();
         if (!y_lds && y_nb) {
             float b0, b1, b2;
-            cbs(cls_at(vyn, sp), (uint32_t)i * plane + (uint32_t)(jn * nz + k), b0, b1, b2);
+            cbs(cls_at(vyn, sp), (uint32_t)i * plane + (uint32_t)(jn * pz + k), b0, b1, b2);
             const F n0 = b0 * (yn.pec * zc.pec) * T::ld(rE, vyn, sp);
             const F n2 = b2 * (xc.pec * yn.pec) * T::ld(rE, vyn, sp + 2u * cB);
             F a0 = T::zero(), a1 = T::zero();
@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_e1(AdjDev d)
         }
         if (!z_lds && z_nb) {
             float b0, b1, b2;
-            cbs(cls_at(vzn, sp), (uint32_t)i * plane + (uint32_t)(j * nz + kn), b0, b1, b2);
+            cbs(cls_at(vzn, sp), (uint32_t)i * plane + (uint32_t)(j * pz + kn), b0, b1, b2);
             const F n0 = b0 * (yc.pec * zn.pec) * T::ld(rE, vzn, sp);
             const F n1 = b1 * (zn.pec * xc.pec) * T::ld(rE, vzn, sp + cB);
             F a0 = T::zero(), a1 = T::zero();
@@ -367,7 +367,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_h1(AdjDev d)
     }
     const GridDev &g = d.g;
     const AxisDev &X = g.ax[0], &Y = g.ax[1], &Z = g.ax[2];
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const int nx = g.nx, ny = g.ny, nz = g.nz, pz = g.pz;
     // one (j, k) column per thread, numbered along the plane (threads past the last column take
     // the last one and store nothing, so every thread reaches the per-plane barrier)
     const int tid = threadIdx.y * OEM_ADJ_TK + threadIdx.x;
@@ -376,7 +376,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_h1(AdjDev d)
     const int q = act ? base + tid : ny * nz - 1;
     const int j = q / nz, k = q - j * nz;
     const int i0 = blockIdx.z * d.chunk, i1 = min(i0 + d.chunk, nx);
-    const uint32_t nc = (uint32_t)d.ncell, plane = (uint32_t)(ny * nz);
+    const uint32_t nc = (uint32_t)d.ncell, plane = (uint32_t)(ny * pz);
     const int wy = Y.lo + Y.hi, wz = Z.lo + Z.hi;
     const uint32_t *off = d.psl.off;
     const float mch = -d.ch;
@@ -412,10 +412,10 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_h1(AdjDev d)
     const bool y_lds = y_nb && ly >= 0 && ly < OEM_ADJ_TK * OEM_ADJ_TJ;
     const bool z_lds = z_nb && lz >= 0 && lz < OEM_ADJ_TK * OEM_ADJ_TJ;
     // per-thread byte offsets within a plane: the cell, its y and z neighbours, their psi rows
-    const uint32_t vo = (uint32_t)(j * nz + k) * EB, vyp = (uint32_t)(jp * nz + k) * EB,
-                   vzp = (uint32_t)(j * nz + kp) * EB;
-    const uint32_t vpy = (uint32_t)(max(yc.s, 0) * nz + k) * EB;
-    const uint32_t vpyp = (uint32_t)(max(yp.s, 0) * nz + k) * EB;
+    const uint32_t vo = (uint32_t)(j * pz + k) * EB, vyp = (uint32_t)(jp * pz + k) * EB,
+                   vzp = (uint32_t)(j * pz + kp) * EB;
+    const uint32_t vpy = (uint32_t)(max(yc.s, 0) * pz + k) * EB;
+    const uint32_t vpyp = (uint32_t)(max(yp.s, 0) * pz + k) * EB;
     const uint32_t vpz = (uint32_t)(j * wz + max(zc.s, 0)) * EB;
     const uint32_t vpzp = (uint32_t)(j * wz + max(zp.s, 0)) * EB;
     int buf = 0;
@@ -449,7 +449,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_h1(AdjDev d)
     }
     for (int i = i0; i < i1; ++i) {
         const uint32_t sp = (uint32_t)i * plane * EB;
-        const uint32_t sy = (uint32_t)i * (uint32_t)(wy * nz) * EB;
+        const uint32_t sy = (uint32_t)i * (uint32_t)(wy * pz) * EB;
         const uint32_t sz = (uint32_t)i * (uint32_t)(ny * wz) * EB;
         const AxAt xc = ax_at_row(X, nx, i, AX_AH, AX_KH, AX_IDLP, AX_MNX);
         const uint32_t sx = (uint32_t)max(xc.s, 0) * plane * EB;
@@ -472,7 +472,7 @@ __global__ void __launch_bounds__(OEM_ADJ_TK * OEM_ADJ_TJ) k_adj_h1(AdjDev d)
         float ax_ = 0.f, ay_ = 0.f, az_ = 0.f;
         F el0 = T::zero(), el1 = T::zero(), el2 = T::zero();
         if (act) {
-            cas(vo, sp, (uint32_t)i * plane + (uint32_t)(j * nz + k), ax_, ay_, az_);
+            cas(vo, sp, (uint32_t)i * plane + (uint32_t)(j * pz + k), ax_, ay_, az_);
             el0 = T::ld(rE, vo, sp);
             el1 = T::ld(rE, vo, sp + cB);
             el2 = T::ld(rE, vo, sp + 2u * cB);
@@ -653,8 +653,8 @@ k_adj_disp_setup(DispDev d, MatDev mat, GridDev g, float cw, size_t ncell, float
     uint32_t c, id;
     int t0, t1;
     adj_entry(d, e, c, id, t0, t1);
-    const int pl = g.ny * g.nz;
-    const int i = (int)id / pl, r = (int)id - i * pl, j = r / g.nz, k = r - j * g.nz;
+    const int pl = g.ny * g.pz;
+    const int i = (int)id / pl, r = (int)id - i * pl, j = r / g.pz, k = r - j * g.pz;
     const float cb = mat.mode == 0 ? mat.lut[8 * (size_t)mat.cls[id] + 2 * c + 1]
                                    : mat.cb[(size_t)c * ncell + id];
     const float px = axv(g.ax[0], i, AX_PEC), py = axv(g.ax[1], j, AX_PEC),
@@ -769,10 +769,10 @@ static void gather_design(oem_ctx *ctx, oem_adjoint_state *a, size_t row) {
     if (ctx->cplx)
         hipLaunchKernelGGL((k_adj_gather<cf2>), g, b, 0, ctx->stream,
                            reinterpret_cast<const cf2 *>(ctx->cur_E()), a->d_comp, a->d_cell,
-                           a->n_design, ctx->ncell, reinterpret_cast<cf2 *>(a->rec) + o);
+                           a->n_design, ctx->nst, reinterpret_cast<cf2 *>(a->rec) + o);
     else
         hipLaunchKernelGGL((k_adj_gather<float>), g, b, 0, ctx->stream, ctx->cur_E(), a->d_comp,
-                           a->d_cell, a->n_design, ctx->ncell, a->rec + o);
+                           a->d_cell, a->n_design, ctx->nst, a->rec + o);
 }
 
 static int adj_check(oem_ctx *ctx) {
@@ -783,7 +783,7 @@ static int adj_check(oem_ctx *ctx) {
     // the transposed sweeps address the three components of an adjoint field, and the psi
     // adjoints of one side, through buffer resources with 32-bit byte offsets
     const uint64_t eb = 4ull * ctx->esz;
-    if (3ull * eb * ctx->ncell >= (1ull << 32) || eb * ctx->psi.total >= (1ull << 32))
+    if (3ull * eb * ctx->nst >= (1ull << 32) || eb * ctx->psi.total >= (1ull << 32))
         return fail(OEM_ENOTSUP, "the adjoint covers up to 2^32 / %llu cells",
                     (unsigned long long)(3ull * eb));
     if (!ctx->adj) ctx->adj = new oem_adjoint_state();
@@ -796,7 +796,7 @@ static size_t pole_floats(oem_ctx *c) {
     return c->has_disp ? 2 * (size_t)c->disp_n_pole * (c->cplx ? 2 : 1) : 0;
 }
 static size_t state_floats(oem_ctx *c) {
-    return (6 * c->ncell + 2 * (size_t)c->psi.total) * c->esz + pole_floats(c);
+    return (6 * c->nst + 2 * (size_t)c->psi.total) * c->esz + pole_floats(c);
 }
 
 extern "C" int oem_checkpoint_alloc(oem_ctx *ctx, int32_t n_slots) {
@@ -811,7 +811,7 @@ extern "C" int oem_checkpoint_alloc(oem_ctx *ctx, int32_t n_slots) {
 }
 
 static int copy_state(oem_ctx *c, float *dst_base, bool save) {
-    const size_t nc = c->ncell, pt = c->psi.total;
+    const size_t nc = c->nst, pt = c->psi.total;
     const bool odd = c->fused && (c->step & 1);
     float *E = odd ? c->E2 : c->E, *H = odd ? c->H2 : c->H;
     const PsiDev &ps = odd ? c->psi2 : c->psi;
@@ -881,7 +881,7 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
             return fail(OEM_EINVAL, "design entry %d out of range", q);
         if (cb[q] == 0.f) return fail(OEM_EINVAL, "design entry %d has cb = 0 (PEC)", q);
     }
-    const size_t nc = ctx->ncell, es = ctx->esz;
+    const size_t nc = ctx->nst, es = ctx->esz;
     TRY(ctx->alloc(&a->lE, 3 * nc * es, true));
     TRY(ctx->alloc(&a->lH, 3 * nc * es, true));
     TRY(ctx->alloc(&a->lpe, (size_t)ctx->psi.total * es, true));
@@ -889,7 +889,9 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
     TRY(ctx->alloc(&a->lpe2, (size_t)ctx->psi.total * es, true));
     TRY(ctx->alloc(&a->lph2, (size_t)ctx->psi.total * es, true));
     TRY(ctx->upload(&a->d_comp, (const int *)comp, (size_t)n_design));
-    TRY(ctx->upload(&a->d_cell, (const int *)cell, (size_t)n_design));
+    std::vector<int> dcell(n_design);
+    for (int q = 0; q < n_design; ++q) dcell[q] = (int)ctx->dev_cell(cell[q]);
+    TRY(ctx->upload(&a->d_cell, (const int *)dcell.data(), dcell.size()));
     TRY(ctx->upload(&a->dca, dca, (size_t)n_design));
     TRY(ctx->upload(&a->dcb, dcb, (size_t)n_design));
     TRY(ctx->upload(&a->ca, ca, (size_t)n_design));
@@ -903,7 +905,7 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
         TRY(ctx->alloc(&a->pend, (size_t)ne * es, true));
         TRY(ctx->alloc(&a->wnu, (size_t)ne, true));
         hipLaunchKernelGGL(k_adj_disp_setup, dim3((ne + 255) / 256), dim3(256), 0, ctx->stream,
-                           ctx->disp, ctx->mat, ctx->g, ctx->dims.cw, ctx->ncell, a->wnu);
+                           ctx->disp, ctx->mat, ctx->g, ctx->dims.cw, ctx->nst, a->wnu);
         HIP_OK(hipGetLastError());
     }
     a->n_design = n_design;
@@ -1010,19 +1012,19 @@ static void back_steps(oem_ctx *ctx, oem_adjoint_state *a, AdjDev &d, const ObjD
         if (all) {
             if (od.ofs[od.n] > 0)
                 hipLaunchKernelGGL((k_adj_obj_all<F>), dim3((od.ofs[od.n] + 255) / 256), dim3(256),
-                                   0, ctx->stream, lE, lH, od, ctx->mat, ctx->ncell, n);
+                                   0, ctx->stream, lE, lH, od, ctx->mat, ctx->nst, n);
         } else {
             for (auto &P : a->obj)
                 hipLaunchKernelGGL((k_adj_obj<F>), dim3((P.d.n_groups + 255) / 256), dim3(256), 0,
-                                   ctx->stream, P.magnetic ? lH : lE, P.d, ctx->mat, ctx->ncell, n);
+                                   ctx->stream, P.magnetic ? lH : lE, P.d, ctx->mat, ctx->nst, n);
         }
         if (ctx->has_disp)
             hipLaunchKernelGGL((k_adj_disp<F>), dim3((ctx->disp.n_entry + 255) / 256), dim3(256), 0,
                                ctx->stream, lE, ctx->disp, a->lP, a->lQ,
-                               reinterpret_cast<F *>(a->pend), a->wnu, ctx->ncell);
+                               reinterpret_cast<F *>(a->pend), a->wnu, ctx->nst);
         hipLaunchKernelGGL((k_adj_grad<F>), gg, gb, 0, ctx->stream, lE, a->d_comp, a->d_cell,
                            a->dca, a->dcb, a->ca, a->cb, rec + (size_t)s * a->n_design,
-                           rec + (size_t)(s + 1) * a->n_design, a->n_design, ctx->ncell, a->grad);
+                           rec + (size_t)(s + 1) * a->n_design, a->n_design, ctx->nst, a->grad);
         // E transpose: reads lE and lpe, adds to lH, writes the new lpe to the other buffer;
         // then the H transpose: reads lH and lph, rewrites lE in place as ca pec lE + its
         // sum, writes the new lph to the other buffer
@@ -1047,7 +1049,7 @@ extern "C" int oem_adjoint_back(oem_ctx *ctx, int64_t n_steps) {
     d.g = ctx->g;
     d.mat = ctx->mat;
     d.ch = ctx->dims.ch;
-    d.ncell = ctx->ncell;
+    d.ncell = ctx->nst;
     d.chunk = adj_chunk();
     const dim3 tb(OEM_ADJ_TK, OEM_ADJ_TJ);
     const int cols = ctx->dims.ny * ctx->dims.nz;

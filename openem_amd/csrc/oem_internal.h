@@ -128,7 +128,10 @@ struct oem_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     oem_dims dims{};
-    size_t ncell = 0;
+    size_t ncell = 0;           // cells of the grid (the ABI's flat index space)
+    int pz = 0;                 // row pitch of the device arrays (row_pitch)
+    size_t nst = 0;             // cells of one device component, nx*ny*pz
+    float *stage = nullptr;     // dense rows of a padded field on their way to or from the host
     bool cplx = false;          // Bloch: complex fields, (re, im) interleaved
     size_t esz = 1;             // floats per field element
     float *E = nullptr, *H = nullptr;
@@ -211,6 +214,22 @@ struct oem_ctx {
         return OEM_OK;
     }
 
+    // flat cell of the ABI -> flat cell of the pitched device arrays
+    size_t dev_cell(size_t id) const {
+        const size_t nz = (size_t)dims.nz;
+        return id / nz * (size_t)pz + id % nz;
+    }
+
+    // `rows` rows of nz elements of a caller's array -> the pitched rows of an uploaded one
+    template <typename T>
+    int upload_rows(T **out, const T *host, size_t rows) {
+        const size_t nz = (size_t)dims.nz;
+        if (pz == dims.nz) return upload(out, host, rows * nz);
+        std::vector<T> v(rows * (size_t)pz, T(0));
+        for (size_t r = 0; r < rows; ++r) std::memcpy(&v[r * pz], host + r * nz, nz * sizeof(T));
+        return upload(out, (const T *)v.data(), v.size());
+    }
+
     template <typename T>
     int upload(T **out, const T *host, size_t n) {
         int rc = alloc(out, n, false);
@@ -226,6 +245,9 @@ struct oem_ctx {
         if (!(c)) return fail(OEM_EINVAL, "null context");                     \
         HIP_OK(hipSetDevice((c)->device));                                     \
     } while (0)
+
+// Row pitch (cells) of a context's device arrays, chosen from the dimensions alone.
+int row_pitch(const oem_dims *d, bool pooled);
 
 // Shared by oem_ctx_create and oem_pool_ctx_create: validate dims and allocate the fields,
 // psi slabs and counters of a context (through the pool's arena when ctx->pool is set).

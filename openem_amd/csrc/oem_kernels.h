@@ -135,7 +135,10 @@ __device__ __forceinline__ int cidx_at(const int *p, int i) {
 struct GridDev {
     AxisDev ax[3];
     int nx, ny, nz;
-    int plane;          // ny*nz
+    // row pitch (cells): rows of a field, class, x- or y-slab psi plane start pz cells apart
+    // (row_pitch); the step neither reads nor writes the pad cells
+    int pz;
+    int plane;          // ny*pz
     int tiles;          // k-tiles * j-tiles of the (ny, nz) plane (flat: blocks of the plane)
     int chunk;          // i-planes per block
     int nblocks;        // tiles * ceil(nx / chunk)
@@ -202,7 +205,7 @@ __device__ __forceinline__ TileCoord tile_coord(const GridDev &g, int lb) {
     TileCoord t;
     if (g.flat) {
         const int q = tile * (OEM_TK * OEM_TJ) + (int)threadIdx.y * OEM_TK + (int)threadIdx.x;
-        t.ok = q < g.plane;
+        t.ok = q < g.ny * g.nz;
         t.j = t.ok ? q / g.nz : 0;
         t.k = t.ok ? q - t.j * g.nz : 0;
     } else {
@@ -237,7 +240,7 @@ __device__ __forceinline__ void update_h_tile(F *__restrict__ H, const F *__rest
 {
     typedef FT<F> T;
     const int j = tc.j, k = tc.k;
-    const int nz = g.nz, ny = g.ny, nx = g.nx;
+    const int nz = g.nz, pz = g.pz, ny = g.ny, nx = g.nx;
     const AxisDev &X = g.ax[0], &Y = g.ax[1], &Z = g.ax[2];
     const size_t ncell = (size_t)g.plane * nx;
     const uint32_t cb = (uint32_t)(ncell * T::B);
@@ -245,9 +248,9 @@ __device__ __forceinline__ void update_h_tile(F *__restrict__ H, const F *__rest
     const rsrc_t rHx = mk_rsrc(H, cb), rHy = mk_rsrc(H + ncell, cb), rHz = mk_rsrc(H + 2 * ncell, cb);
     const rsrc_t rP = mk_rsrc(ps.h, ps.total * T::B);
 
-    const uint32_t op = (uint32_t)(j * nz + k) * T::B;            // own cell in the plane
-    const uint32_t oj = (uint32_t)(Y.nxt[j] * nz + k) * T::B;     // (j+1, k)
-    const uint32_t ok = (uint32_t)(j * nz + Z.nxt[k]) * T::B;     // (j, k+1)
+    const uint32_t op = (uint32_t)(j * pz + k) * T::B;            // own cell in the plane
+    const uint32_t oj = (uint32_t)(Y.nxt[j] * pz + k) * T::B;     // (j+1, k)
+    const uint32_t ok = (uint32_t)(j * pz + Z.nxt[k]) * T::B;     // (j, k+1)
     const float mj = axv(Y, j, AX_MNX), mk = axv(Z, k, AX_MNX);
     const float mji = axv(Y, j, AX_MNXI), mki = axv(Z, k, AX_MNXI);
     const float idy = axv(Y, j, AX_IDLP), idz = axv(Z, k, AX_IDLP);
@@ -257,7 +260,7 @@ __device__ __forceinline__ void update_h_tile(F *__restrict__ H, const F *__rest
     float ay = 0.f, by = 1.f, ky = 1.f, az = 0.f, bz = 1.f, kz = 1.f;
     if (sy >= 0) { ay = axv(Y, j, AX_AH); by = axv(Y, j, AX_BH); ky = axv(Y, j, AX_KH); }
     if (sz >= 0) { az = axv(Z, k, AX_AH); bz = axv(Z, k, AX_BH); kz = axv(Z, k, AX_KH); }
-    const uint32_t oy = (uint32_t)(max(sy, 0) * nz + k) * T::B;   // psi y-slab, within plane i
+    const uint32_t oy = (uint32_t)(max(sy, 0) * pz + k) * T::B;   // psi y-slab, within plane i
     const uint32_t oz = (uint32_t)(j * wz + max(sz, 0)) * T::B;   // psi z-slab, within plane i
 
     float inj_hx = 0.f, inj_hy = 0.f;
@@ -285,8 +288,8 @@ __device__ __forceinline__ void update_h_tile(F *__restrict__ H, const F *__rest
         const int sx = slab_of(i, nx, X.lo, X.hi);
         const uint32_t sx0 = (ps.off[0] + (uint32_t)max(sx, 0) * (uint32_t)g.plane) * T::B;
         const uint32_t sx1 = (ps.off[1] + (uint32_t)max(sx, 0) * (uint32_t)g.plane) * T::B;
-        const uint32_t sy0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * nz)) * T::B;
-        const uint32_t sy1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * nz)) * T::B;
+        const uint32_t sy0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * pz)) * T::B;
+        const uint32_t sy1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * pz)) * T::B;
         const uint32_t sz0 = (ps.off[4] + (uint32_t)i * (uint32_t)(ny * wz)) * T::B;
         const uint32_t sz1 = (ps.off[5] + (uint32_t)i * (uint32_t)(ny * wz)) * T::B;
         F psx0 = T::zero(), psx1 = T::zero(), psy0 = T::zero(), psy1 = T::zero(),
@@ -372,7 +375,7 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
 {
     typedef FT<F> T;
     const int j = tc.j, k = tc.k;
-    const int nz = g.nz, ny = g.ny, nx = g.nx;
+    const int nz = g.nz, pz = g.pz, ny = g.ny, nx = g.nx;
     const AxisDev &X = g.ax[0], &Y = g.ax[1], &Z = g.ax[2];
     const size_t ncell = (size_t)g.plane * nx;
     const uint32_t cbytes = (uint32_t)(ncell * T::B);
@@ -383,9 +386,9 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
     const rsrc_t rP = mk_rsrc(ps.e, ps.total * T::B);
     const rsrc_t rC = mk_rsrc(mat.cls, (uint32_t)(ncell * 2));
 
-    const uint32_t op = (uint32_t)(j * nz + k) * T::B;
-    const uint32_t oj = (uint32_t)(Y.prv[j] * nz + k) * T::B;     // (j-1, k)
-    const uint32_t ok = (uint32_t)(j * nz + Z.prv[k]) * T::B;     // (j, k-1)
+    const uint32_t op = (uint32_t)(j * pz + k) * T::B;
+    const uint32_t oj = (uint32_t)(Y.prv[j] * pz + k) * T::B;     // (j-1, k)
+    const uint32_t ok = (uint32_t)(j * pz + Z.prv[k]) * T::B;     // (j, k-1)
     const float mj = axv(Y, j, AX_MPV), mk = axv(Z, k, AX_MPV);
     const float mji = axv(Y, j, AX_MPVI), mki = axv(Z, k, AX_MPVI);
     const float idy = axv(Y, j, AX_IDLD), idz = axv(Z, k, AX_IDLD);
@@ -396,7 +399,7 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
     float ay = 0.f, by = 1.f, ky = 1.f, az = 0.f, bz = 1.f, kz = 1.f;
     if (sy >= 0) { ay = axv(Y, j, AX_AE); by = axv(Y, j, AX_BE); ky = axv(Y, j, AX_KE); }
     if (sz >= 0) { az = axv(Z, k, AX_AE); bz = axv(Z, k, AX_BE); kz = axv(Z, k, AX_KE); }
-    const uint32_t oy = (uint32_t)(max(sy, 0) * nz + k) * T::B;
+    const uint32_t oy = (uint32_t)(max(sy, 0) * pz + k) * T::B;
     const uint32_t oz = (uint32_t)(j * wz + max(sz, 0)) * T::B;
 
     float inj_ex = 0.f, inj_ey = 0.f;
@@ -418,7 +421,7 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
     const uint32_t hcomp = (uint32_t)(hbx * hby * hbz);
     const rsrc_t rHist = mk_rsrc(mat.hist, 3u * hcomp * T::B);
     const uint32_t oh = hrow ? (uint32_t)((j - mat.hb[2]) * hbz + (k - mat.hb[4])) * T::B : 0u;
-    const uint32_t oc = (uint32_t)(j * nz + k) * 2u;               // uint16 class index
+    const uint32_t oc = (uint32_t)(j * pz + k) * 2u;               // uint16 class index
 
     const uint32_t planeB = (uint32_t)g.plane * T::B, plane2 = (uint32_t)g.plane * 2u;
     const uint32_t sp0 = (uint32_t)__builtin_amdgcn_readfirstlane(X.prv[tc.i0]) * planeB;
@@ -435,8 +438,8 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
         const int sx = slab_of(i, nx, X.lo, X.hi);
         const uint32_t sx0 = (ps.off[0] + (uint32_t)max(sx, 0) * (uint32_t)g.plane) * T::B;
         const uint32_t sx1 = (ps.off[1] + (uint32_t)max(sx, 0) * (uint32_t)g.plane) * T::B;
-        const uint32_t sy0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * nz)) * T::B;
-        const uint32_t sy1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * nz)) * T::B;
+        const uint32_t sy0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * pz)) * T::B;
+        const uint32_t sy1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * pz)) * T::B;
         const uint32_t sz0 = (ps.off[4] + (uint32_t)i * (uint32_t)(ny * wz)) * T::B;
         const uint32_t sz1 = (ps.off[5] + (uint32_t)i * (uint32_t)(ny * wz)) * T::B;
         F psx0 = T::zero(), psx1 = T::zero(), psy0 = T::zero(), psy1 = T::zero(),
@@ -457,7 +460,7 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
             cax = r0.x; cbx = r0.y; cay = r0.z; cby = r0.w; caz = r1.x; cbz = r1.y;
             fl = __float_as_uint(r1.z);
         } else {
-            const size_t id = (size_t)i * g.plane + (size_t)j * nz + k;
+            const size_t id = (size_t)i * g.plane + (size_t)j * pz + k;
             cax = mat.ca[id]; cay = mat.ca[ncell + id]; caz = mat.ca[2 * ncell + id];
             cbx = mat.cb[id]; cby = mat.cb[ncell + id]; cbz = mat.cb[2 * ncell + id];
             fl = (hrow && i >= mat.hb[0] && i < mat.hb[1]) ? 7u : 0u;
@@ -593,13 +596,13 @@ __device__ __forceinline__ void hcolumn_init(HColumn<F> &c, const GridDev &g,
                                              int jn, int kn) {
     typedef FT<F> T;
     const AxisDev &Y = g.ax[1], &Z = g.ax[2];
-    const int nz = g.nz, wz = Z.lo + Z.hi;
-    c.op = (uint32_t)(j * nz + k) * T::B;
-    c.oj = (uint32_t)(jn * nz + k) * T::B;
-    c.ok = (uint32_t)(j * nz + kn) * T::B;
+    const int nz = g.nz, pz = g.pz, wz = Z.lo + Z.hi;
+    c.op = (uint32_t)(j * pz + k) * T::B;
+    c.oj = (uint32_t)(jn * pz + k) * T::B;
+    c.ok = (uint32_t)(j * pz + kn) * T::B;
     c.sy = slab_of(j, g.ny, Y.lo, Y.hi);
     c.sz = slab_of(k, nz, Z.lo, Z.hi);
-    c.oy = (uint32_t)(max(c.sy, 0) * nz + k) * T::B;
+    c.oy = (uint32_t)(max(c.sy, 0) * pz + k) * T::B;
     c.oz = (uint32_t)(j * wz + max(c.sz, 0)) * T::B;
     c.mj = axv(Y, j, AX_MNX); c.mji = axv(Y, j, AX_MNXI); c.idy = axv(Y, j, AX_IDLP);
     c.mk = axv(Z, k, AX_MNX); c.mki = axv(Z, k, AX_MNXI); c.idz = axv(Z, k, AX_IDLP);
@@ -642,8 +645,8 @@ __device__ __forceinline__ PsiOffH psi_off_h(const GridDev &g, const PsiDev &ps,
     o.sx = slab_of(i, g.nx, X.lo, X.hi);
     o.x0 = (ps.off[0] + (uint32_t)max(o.sx, 0) * (uint32_t)g.plane) * T::B;
     o.x1 = (ps.off[1] + (uint32_t)max(o.sx, 0) * (uint32_t)g.plane) * T::B;
-    o.y0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * g.nz)) * T::B;
-    o.y1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * g.nz)) * T::B;
+    o.y0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * g.pz)) * T::B;
+    o.y1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * g.pz)) * T::B;
     o.z0 = (ps.off[4] + (uint32_t)i * (uint32_t)(g.ny * wz)) * T::B;
     o.z1 = (ps.off[5] + (uint32_t)i * (uint32_t)(g.ny * wz)) * T::B;
     return o;
@@ -888,7 +891,7 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
     __shared__ int s_fq[64];
     __shared__ int s_fcnt[OEM_CR];
     const AxisDev &X = g.ax[0], &Y = g.ax[1], &Z = g.ax[2];
-    const int nx = g.nx, ny = g.ny, nz = g.nz;
+    const int nx = g.nx, ny = g.ny, nz = g.nz, pz = g.pz;
     const int nkt = (nz + 63) / 64;
     // per-work-group quantities through readfirstlane: the compiler then keeps them in SGPRs
     const int lb = xcd_remap(blockIdx.x, g.nblocks);
@@ -1033,7 +1036,7 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
     const bool hrow = mat.hist && own && j >= mat.hb[2] && j < mat.hb[3] && k >= mat.hb[4] &&
                       k < mat.hb[5];
     const uint32_t oh = hrow ? (uint32_t)((j - mat.hb[2]) * hbz + (k - mat.hb[4])) * T::B : 0u;
-    const uint32_t oc = (uint32_t)(j * nz + k) * 2u;
+    const uint32_t oc = (uint32_t)(j * pz + k) * 2u;
 
     // the new Hy, Hz of the plane before i0 (the x neighbours of E at i0), not stored
     F hy_m, hz_m;
@@ -1059,8 +1062,8 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         const int wy = Y.lo + Y.hi, wz = Z.lo + Z.hi;
         const uint32_t sx0 = (ps.off[0] + (uint32_t)max(sx, 0) * (uint32_t)g.plane) * T::B;
         const uint32_t sx1 = (ps.off[1] + (uint32_t)max(sx, 0) * (uint32_t)g.plane) * T::B;
-        const uint32_t sy0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * nz)) * T::B;
-        const uint32_t sy1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * nz)) * T::B;
+        const uint32_t sy0 = (ps.off[2] + (uint32_t)i * (uint32_t)(wy * pz)) * T::B;
+        const uint32_t sy1 = (ps.off[3] + (uint32_t)i * (uint32_t)(wy * pz)) * T::B;
         const uint32_t sz0 = (ps.off[4] + (uint32_t)i * (uint32_t)(ny * wz)) * T::B;
         const uint32_t sz1 = (ps.off[5] + (uint32_t)i * (uint32_t)(ny * wz)) * T::B;
         const bool hin = hrow && i >= mat.hb[0] && i < mat.hb[1];
@@ -1080,7 +1083,7 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
             cax = r0.x; cbx = r0.y; cay = r0.z; cby = r0.w; caz = r1.x; cbz = r1.y;
             fl = __float_as_uint(r1.z);
         } else {
-            const size_t id = (size_t)i * g.plane + (size_t)j * nz + k;
+            const size_t id = (size_t)i * g.plane + (size_t)j * pz + k;
             cax = mat.ca[id]; cay = mat.ca[ncell + id]; caz = mat.ca[2 * ncell + id];
             cbx = mat.cb[id]; cby = mat.cb[ncell + id]; cbz = mat.cb[2 * ncell + id];
             fl = 7u;
@@ -1282,8 +1285,8 @@ struct DispDev {
     float2 *sp, *sq;        // pole state driven by Re E / by Im E (complex fields only)
 };
 
-__device__ __forceinline__ size_t hist_index(const DispDev &d, int c, int cell, int ny, int nz) {
-    const int i = cell / (ny * nz), r = cell - i * ny * nz, j = r / nz, k = r - j * nz;
+__device__ __forceinline__ size_t hist_index(const DispDev &d, int c, int cell, int ny, int pz) {
+    const int i = cell / (ny * pz), r = cell - i * ny * pz, j = r / pz, k = r - j * pz;
     const int bx = d.hb[1] - d.hb[0], by = d.hb[3] - d.hb[2], bz = d.hb[5] - d.hb[4];
     return (((size_t)c * bx + (i - d.hb[0])) * by + (j - d.hb[2])) * bz + (k - d.hb[4]);
 }
@@ -1377,7 +1380,7 @@ __device__ __forceinline__ void disp_entry_np(const DispDev &d, const F *__restr
 // Entry e: mode 0 = pre, 1 = post, 2 = fused post + pre.
 template <typename F>
 __device__ __forceinline__ void disp_entry(const DispDev &d, const F *__restrict__ E,
-                                           size_t ncell, int ny, int nz, int mode, int e)
+                                           size_t ncell, int ny, int pz, int mode, int e)
 {
     switch (d.np) {
     case 1: disp_entry_np<F, 1>(d, E, ncell, mode, e); return;
@@ -1392,24 +1395,24 @@ __device__ __forceinline__ void disp_entry(const DispDev &d, const F *__restrict
         float w = 0.f;
         for (int t = d.ofs[e]; t < d.ofs[e + 1]; ++t)
             w += pole_update(d.p_re, d.p_im, t, d.cidx[t], d, en, mode);
-        if (mode != 1) static_cast<float *>(d.hist)[hist_index(d, c, id, ny, nz)] = w;
+        if (mode != 1) static_cast<float *>(d.hist)[hist_index(d, c, id, ny, pz)] = w;
     } else {
         float wr = 0.f, wi = 0.f;
         for (int t = d.ofs[e]; t < d.ofs[e + 1]; ++t) {
             wr += pole_update(d.p_re, d.p_im, t, d.cidx[t], d, en.r, mode);
             wi += pole_update(d.q_re, d.q_im, t, d.cidx[t], d, en.i, mode);
         }
-        if (mode != 1) static_cast<cf2 *>(d.hist)[hist_index(d, c, id, ny, nz)] = cf2{wr, wi};
+        if (mode != 1) static_cast<cf2 *>(d.hist)[hist_index(d, c, id, ny, pz)] = cf2{wr, wi};
     }
 }
 
 template <typename F>
 __global__ void __launch_bounds__(256)
-k_disp(DispDev d, const F *__restrict__ E, size_t ncell, int ny, int nz, int mode)
+k_disp(DispDev d, const F *__restrict__ E, size_t ncell, int ny, int pz, int mode)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= d.n_entry) return;
-    disp_entry<F>(d, E, ncell, ny, nz, mode, e);
+    disp_entry<F>(d, E, ncell, ny, pz, mode, e);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1430,7 +1433,7 @@ struct TimeMonDev {
 template <typename F>
 __global__ void __launch_bounds__(256)
 k_time_sample(TimeMonDev d, const F *__restrict__ E, const F *__restrict__ H, size_t ncell,
-              int ny, int nz, const int *__restrict__ stp, int shot)
+              int ny, int pz, const int *__restrict__ stp, int shot)
 {
     const int m = step_now(stp) + 1 - shot;
     const int off = m - d.beg;
@@ -1441,7 +1444,7 @@ k_time_sample(TimeMonDev d, const F *__restrict__ E, const F *__restrict__ H, si
     if (q >= d.cells) return;
     const int a = q / (d.b[1] * d.b[2]), r = q - a * d.b[1] * d.b[2];
     const int b = r / d.b[2], c = r - b * d.b[2];
-    const size_t id = ((size_t)(d.o[0] + a) * ny + (d.o[1] + b)) * nz + (d.o[2] + c);
+    const size_t id = ((size_t)(d.o[0] + a) * ny + (d.o[1] + b)) * pz + (d.o[2] + c);
     F *out = static_cast<F *>(d.buf);
     for (int t = 0; t < d.nc; ++t) {
         const int comp = d.comps[t];
@@ -1487,12 +1490,12 @@ __device__ __forceinline__ int ft_slot(const FluxTimeDev &d, int m) {
 }
 
 __device__ __forceinline__ size_t ft_cell(const FluxTimeDev &d, int k, int i1, int i2, int ny,
-                                          int nz) {
+                                          int pz) {
     int c[3];
     c[d.axis] = k;
     c[d.t1] = i1;
     c[d.t2] = i2;
-    return ((size_t)c[0] * ny + c[1]) * nz + c[2];
+    return ((size_t)c[0] * ny + c[1]) * pz + c[2];
 }
 
 // Sum of a double over the block (fixed tree), valid in thread 0.
@@ -1510,7 +1513,7 @@ __device__ __forceinline__ double ft_block_sum(double v, double *sh) {
 template <typename F>
 __global__ void __launch_bounds__(OEM_FT_BLK)
 k_flux_time_partial(FluxTimeDev d, const F *__restrict__ E, const F *__restrict__ H,
-                    size_t ncell, int ny, int nz, const int *__restrict__ stp)
+                    size_t ncell, int ny, int pz, const int *__restrict__ stp)
 {
     static_assert(sizeof(F) == 4, "flux-time monitors sample real fields");
     const int n = step_now(stp);
@@ -1530,26 +1533,26 @@ k_flux_time_partial(FluxTimeDev d, const F *__restrict__ E, const F *__restrict_
             const int ke = d.ke[p], kh = d.kh[p];
             const float lo = d.wh_lo[p], hi = d.wh_hi[p];
             // H_u: on the edge along t1, centre -> edge along t2, coordinate weights along the normal
-            const float hu_l = lo * Hu[ft_cell(d, kh, d.e1[a], d.l2[b], ny, nz)] +
-                               hi * Hu[ft_cell(d, kh + 1, d.e1[a], d.l2[b], ny, nz)];
-            const float hu_h = lo * Hu[ft_cell(d, kh, d.e1[a], d.h2[b], ny, nz)] +
-                               hi * Hu[ft_cell(d, kh + 1, d.e1[a], d.h2[b], ny, nz)];
+            const float hu_l = lo * Hu[ft_cell(d, kh, d.e1[a], d.l2[b], ny, pz)] +
+                               hi * Hu[ft_cell(d, kh + 1, d.e1[a], d.l2[b], ny, pz)];
+            const float hu_h = lo * Hu[ft_cell(d, kh, d.e1[a], d.h2[b], ny, pz)] +
+                               hi * Hu[ft_cell(d, kh + 1, d.e1[a], d.h2[b], ny, pz)];
             const float hu = w2 * hu_l + (1.0f - w2) * hu_h;
             // H_v: centre -> edge along t1, on the edge along t2
-            const float hv_l = lo * Hv[ft_cell(d, kh, d.l1[a], d.e2[b], ny, nz)] +
-                               hi * Hv[ft_cell(d, kh + 1, d.l1[a], d.e2[b], ny, nz)];
-            const float hv_h = lo * Hv[ft_cell(d, kh, d.h1[a], d.e2[b], ny, nz)] +
-                               hi * Hv[ft_cell(d, kh + 1, d.h1[a], d.e2[b], ny, nz)];
+            const float hv_l = lo * Hv[ft_cell(d, kh, d.l1[a], d.e2[b], ny, pz)] +
+                               hi * Hv[ft_cell(d, kh + 1, d.l1[a], d.e2[b], ny, pz)];
+            const float hv_h = lo * Hv[ft_cell(d, kh, d.h1[a], d.e2[b], ny, pz)] +
+                               hi * Hv[ft_cell(d, kh + 1, d.h1[a], d.e2[b], ny, pz)];
             const float hv = w1 * hv_l + (1.0f - w1) * hv_h;
             float *keep = d.ep + (size_t)(2 * p) * np;
             const double wp = 0.5 * d.plane_w[p] * dS;
             if (s1 >= 0)
                 v1 += wp * ((double)(keep[q] * hv) - (double)(keep[np + q] * hu));
             if (s0 >= 0) {
-                const float eu = w1 * Eu[ft_cell(d, ke, d.l1[a], d.e2[b], ny, nz)] +
-                                 (1.0f - w1) * Eu[ft_cell(d, ke, d.h1[a], d.e2[b], ny, nz)];
-                const float ev = w2 * Ev[ft_cell(d, ke, d.e1[a], d.l2[b], ny, nz)] +
-                                 (1.0f - w2) * Ev[ft_cell(d, ke, d.e1[a], d.h2[b], ny, nz)];
+                const float eu = w1 * Eu[ft_cell(d, ke, d.l1[a], d.e2[b], ny, pz)] +
+                                 (1.0f - w1) * Eu[ft_cell(d, ke, d.h1[a], d.e2[b], ny, pz)];
+                const float ev = w2 * Ev[ft_cell(d, ke, d.e1[a], d.l2[b], ny, pz)] +
+                                 (1.0f - w2) * Ev[ft_cell(d, ke, d.e1[a], d.h2[b], ny, pz)];
                 v0 += wp * ((double)(eu * hv) - (double)(ev * hu));
                 keep[q] = eu;
                 keep[np + q] = ev;
@@ -1608,7 +1611,7 @@ struct MonDev {
 // Point q of a monitor into ring row `slot`.
 template <typename F>
 __device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict__ E,
-                                           const F *__restrict__ H, size_t ncell, int ny, int nz,
+                                           const F *__restrict__ H, size_t ncell, int ny, int pz,
                                            int slot, int q)
 {
     F *row = static_cast<F *>(m.snap) + (size_t)slot * m.ncomp * m.npts;
@@ -1617,9 +1620,9 @@ __device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict_
         int c[3];
         const int t1 = m.axis == 0 ? 1 : 0, t2 = m.axis == 2 ? 1 : 2;
         c[m.axis] = m.km; c[t1] = a; c[t2] = b;
-        const size_t id = ((size_t)c[0] * ny + c[1]) * nz + c[2];
+        const size_t id = ((size_t)c[0] * ny + c[1]) * pz + c[2];
         c[m.axis] = m.km - 1;
-        const size_t idm = ((size_t)c[0] * ny + c[1]) * nz + c[2];
+        const size_t idm = ((size_t)c[0] * ny + c[1]) * pz + c[2];
         row[q] = E[(size_t)t1 * ncell + id];
         row[m.npts + q] = E[(size_t)t2 * ncell + id];
         row[2 * m.npts + q] = 0.5f * (H[(size_t)t1 * ncell + id] + H[(size_t)t1 * ncell + idm]);
@@ -1627,7 +1630,7 @@ __device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict_
     } else {
         const int bjk = m.b[1] * m.b[2];
         const int a = q / bjk, r = q - a * bjk, b = r / m.b[2], cc = r - b * m.b[2];
-        const size_t id = ((size_t)(m.o[0] + a) * ny + (m.o[1] + b)) * nz + (m.o[2] + cc);
+        const size_t id = ((size_t)(m.o[0] + a) * ny + (m.o[1] + b)) * pz + (m.o[2] + cc);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             row[(size_t)c * m.npts + q] = E[(size_t)c * ncell + id];
@@ -1639,11 +1642,11 @@ __device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict_
 template <typename F>
 __global__ void __launch_bounds__(256)
 k_dft_snap(MonDev m, const F *__restrict__ E, const F *__restrict__ H, size_t ncell, int ny,
-           int nz, const int *__restrict__ stp)
+           int pz, const int *__restrict__ stp)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= m.npts) return;
-    snap_point<F>(m, E, H, ncell, ny, nz, step_now(stp) % m.T, q);
+    snap_point<F>(m, E, H, ncell, ny, pz, step_now(stp) % m.T, q);
 }
 
 // The end of a step as one single-block launch, where three small launches would otherwise
@@ -1663,7 +1666,7 @@ struct TailDev {
 template <typename F>
 __global__ void __launch_bounds__(OEM_TAIL_THREADS)
 k_step_tail(F *__restrict__ E, const F *__restrict__ H, TailDev t, MatDev mat, float ch,
-            size_t ncell, int ny, int nz, int *__restrict__ stp)
+            size_t ncell, int ny, int pz, int *__restrict__ stp)
 {
     const int n = step_now(stp);
     const int tid = threadIdx.x;
@@ -1672,7 +1675,7 @@ k_step_tail(F *__restrict__ E, const F *__restrict__ H, TailDev t, MatDev mat, f
         __syncthreads();
     }
     for (int m = 0; m < t.n_snap; ++m)
-        if (tid < t.nq[m]) snap_point<F>(t.mon[m], E, H, ncell, ny, nz, n % t.mon[m].T, t.qs[m][tid]);
+        if (tid < t.nq[m]) snap_point<F>(t.mon[m], E, H, ncell, ny, pz, n % t.mon[m].T, t.qs[m][tid]);
     __syncthreads();
     if (tid == 0) *stp = n + 1;
 }
@@ -1681,11 +1684,11 @@ k_step_tail(F *__restrict__ E, const F *__restrict__ H, TailDev t, MatDev mat, f
 template <typename F>
 __global__ void __launch_bounds__(256)
 k_dft_snap_list(MonDev m, const F *__restrict__ E, const F *__restrict__ H, size_t ncell, int ny,
-                int nz, const int *__restrict__ stp, const int *__restrict__ qs, int nq)
+                int pz, const int *__restrict__ stp, const int *__restrict__ qs, int nq)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nq) return;
-    snap_point<F>(m, E, H, ncell, ny, nz, step_now(stp) % m.T, qs[t]);
+    snap_point<F>(m, E, H, ncell, ny, pz, step_now(stp) % m.T, qs[t]);
 }
 
 __device__ __forceinline__ void dft_acc(double &sr, double &si, float v, double c, double s) {

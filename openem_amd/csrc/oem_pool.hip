@@ -49,8 +49,8 @@ struct SceneDev {
     float ch, cw;
     int *stp;           // [0] steps taken, [1] steps flushed
     int n_total;
-    int ny, nz;
-    size_t ncell;
+    int ny, pz;
+    size_t ncell;       // cells of a component, row padding included
 };
 
 struct PtSeg {
@@ -180,7 +180,7 @@ k_pool_disp(const PoolDev *__restrict__ P, int phase)
             mode = n == S.n_total - 1 ? 1 : 2;
         }
         const int e = base - P->disp_ofs[s] + (int)threadIdx.x;
-        if (e < S.disp.n_entry) disp_entry<float>(S.disp, S.E, S.ncell, S.ny, S.nz, mode, e);
+        if (e < S.disp.n_entry) disp_entry<float>(S.disp, S.E, S.ncell, S.ny, S.pz, mode, e);
     }
 }
 
@@ -197,7 +197,7 @@ k_pool_snap(const PoolDev *__restrict__ P)
         int n;
         if (!scene_live(S, &n)) continue;
         const int q = base - P->snap_ofs[g] + (int)threadIdx.x;
-        if (q < M.d.npts) snap_point<float>(M.d, S.E, S.H, S.ncell, S.ny, S.nz, n % M.d.T, q);
+        if (q < M.d.npts) snap_point<float>(M.d, S.E, S.H, S.ncell, S.ny, S.pz, n % M.d.T, q);
     }
 }
 
@@ -381,8 +381,8 @@ int build_desc(oem_pool *pool, PoolDev *h) {
         S.stp = c->d_step;
         S.n_total = c->dims.n_steps;
         S.ny = c->dims.ny;
-        S.nz = c->dims.nz;
-        S.ncell = c->ncell;
+        S.pz = c->pz;
+        S.ncell = c->nst;
         h->item_ofs[ns] = items;
         items += c->g.nblocks;
         h->disp_ofs[ns] = dsp;

@@ -60,14 +60,16 @@ template <> __device__ __forceinline__ float wsq<cf2>(float w, cf2 x) {
 template <typename F>
 __global__ void __launch_bounds__(OEM_RED_THREADS)
 k_energy(const F *__restrict__ E, const F *__restrict__ H, EnergyDev d, int nx, int ny, int nz,
-         double *__restrict__ partial)
+         int pz, double *__restrict__ partial)
 {
-    const size_t ncell = (size_t)nx * ny * nz;
+    // the fields and the classes have rows of pz cells, the dense eps rows of nz
+    const size_t ncell = (size_t)nx * ny * pz;
     double acc[3] = {0.0, 0.0, 0.0};
     for (size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x; id < ncell;
          id += (size_t)gridDim.x * blockDim.x) {
-        const int k = (int)(id % nz);
-        const size_t r = id / nz;
+        const int k = (int)(id % pz);
+        const size_t r = id / pz;
+        if (k >= nz) continue;
         const int j = (int)(r % ny), i = (int)(r / ny);
         const double xp = d.dl[0][i], yp = d.dl[1][j], zp = d.dl[2][k];
         const double xd = d.dd[0][i], yd = d.dd[1][j], zd = d.dd[2][k];
@@ -77,7 +79,8 @@ k_energy(const F *__restrict__ E, const F *__restrict__ H, EnergyDev d, int nx, 
             const float *row = d.eps + 4 * (size_t)d.cls[id];
             ep[0] = row[0]; ep[1] = row[1]; ep[2] = row[2];
         } else {
-            ep[0] = d.eps[id]; ep[1] = d.eps[ncell + id]; ep[2] = d.eps[2 * ncell + id];
+            const size_t q = r * nz + k, n = (size_t)nx * ny * nz;
+            ep[0] = d.eps[q]; ep[1] = d.eps[n + q]; ep[2] = d.eps[2 * n + q];
         }
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -243,11 +246,11 @@ extern "C" int oem_energy(oem_ctx *ctx, double *out) {
     if (ctx->cplx)
         hipLaunchKernelGGL((k_energy<cf2>), g, b, 0, ctx->stream, (const cf2 *)ctx->cur_E(),
                            (const cf2 *)ctx->cur_H(), r->ed, ctx->dims.nx, ctx->dims.ny, ctx->dims.nz,
-                           r->partial);
+                           ctx->pz, r->partial);
     else
         hipLaunchKernelGGL((k_energy<float>), g, b, 0, ctx->stream, (const float *)ctx->cur_E(),
                            (const float *)ctx->cur_H(), r->ed, ctx->dims.nx, ctx->dims.ny, ctx->dims.nz,
-                           r->partial);
+                           ctx->pz, r->partial);
     hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(64), 0, ctx->stream, r->partial,
                        OEM_RED_BLOCKS, 3, r->out);
     HIP_OK(hipGetLastError());
