@@ -53,7 +53,7 @@ struct FluxTimeMonitor {
 // One grouped point list (dipoles or TF/SF face corrections) and which field it updates.
 enum { PT_DIPOLE = 0, PT_TFSF = 1, PT_MODE = 2 };
 
-// Smallest scene (cells) that takes the fused H+E step by default.
+// From this size (cells) on every scene takes the fused H+E step by default (march_pays).
 #define OEM_FUSE_MIN_CELLS (10u << 20)
 
 struct Points {
@@ -144,6 +144,7 @@ struct oem_ctx {
     float *cur_H() const { return (fused && (step & 1)) ? H2 : H; }
     GridDev g{};
     GridDev fg{};               // launch geometry of the fused H+E step
+    bool fuse_plain = false;    // its stores keep their lines in the caches (march_bytes)
     FuseSnap fsnap{};           // the DFT monitors the fused step snaps
     bool fsnap_multi = false;   // some work-group meets more than one of them
     bool axis_set[3] = {false, false, false};
@@ -217,7 +218,7 @@ struct oem_ctx {
     // flat cell of the ABI -> flat cell of the pitched device arrays
     size_t dev_cell(size_t id) const {
         const size_t nz = (size_t)dims.nz;
-        return id / nz * (size_t)pz + id % nz;
+        return pz == dims.nz ? id : id / nz * (size_t)pz + id % nz;
     }
 
     // `rows` rows of nz elements of a caller's array -> the pitched rows of an uploaded one

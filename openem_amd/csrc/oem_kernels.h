@@ -60,14 +60,12 @@ __device__ __forceinline__ uint32_t bld_u16(rsrc_t r, uint32_t voff, uint32_t so
 // __builtin_bit_cast.
 typedef unsigned int oem_u32x2 __attribute__((vector_size(8)));
 
-// Cache policy of every buffer store: non-temporal (cache-policy bit 1).  Nothing a kernel
-// stores is read again in the same launch, so the stored lines need not displace, in L2, the
-// lines that neighbouring work-groups read again (the fused march's halo and neighbour lines):
-// on the 512^3 step its reads fell from 2.29 to 2.17 M KiB per launch and the march from 1.729
-// to 1.703 ms; the Bloch step from 1.105 to 1.053 ms.
-#ifndef OEM_ST_AUX
-#define OEM_ST_AUX 2
-#endif
+// Cache policy of the buffer stores: non-temporal (cache-policy bit 1) unless a kernel asks for
+// plain ones.  Nothing a kernel stores is read again in the same launch, so the stored lines need
+// not displace, in L2, the lines that neighbouring work-groups read again (the fused march's
+// halo and neighbour lines): on the 512^3 step its reads fell from 2.29 to 2.17 M KiB per launch
+// and the march from 1.729 to 1.703 ms; the Bloch step from 1.105 to 1.053 ms.
+#define OEM_ST_NT 2
 
 template <typename F> struct FT;
 template <> struct FT<float> {
@@ -75,8 +73,9 @@ template <> struct FT<float> {
     static __device__ __forceinline__ float ld(rsrc_t r, uint32_t v, uint32_t s) {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0));
     }
+    template <int AUX = OEM_ST_NT>
     static __device__ __forceinline__ void st(rsrc_t r, float x, uint32_t v, uint32_t s) {
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, x), r, v, s, OEM_ST_AUX);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, x), r, v, s, AUX);
     }
     static __device__ __forceinline__ float mmul(float x, float mr, float) { return x * mr; }
     static __device__ __forceinline__ float zero() { return 0.f; }
@@ -92,8 +91,9 @@ template <> struct FT<cf2> {
         const oem_u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(r, v, s, 0);
         return __builtin_bit_cast(cf2, q);
     }
+    template <int AUX = OEM_ST_NT>
     static __device__ __forceinline__ void st(rsrc_t r, cf2 x, uint32_t v, uint32_t s) {
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(oem_u32x2, x), r, v, s, OEM_ST_AUX);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(oem_u32x2, x), r, v, s, AUX);
     }
     static __device__ __forceinline__ cf2 mmul(cf2 x, float mr, float mi) {
         return {x.r * mr - x.i * mi, x.r * mi + x.i * mr};
@@ -142,6 +142,8 @@ struct GridDev {
     int tiles;          // k-tiles * j-tiles of the (ny, nz) plane (flat: blocks of the plane)
     int chunk;          // i-planes per block
     int nblocks;        // tiles * ceil(nx / chunk)
+    // fused step: the k extent in kt64 strips of 64 lanes (t64 tiles), then perhaps one of 32
+    int kt64, t64;
     int flat;           // the sweeps number the (j, k) columns along the plane (nz % 64 != 0)
 };
 
@@ -355,9 +357,12 @@ k_update_h(F *__restrict__ H, const F *__restrict__ E, PsiDev ps, GridDev g, flo
 // next plane's class index is prefetched, so the per-cell coefficient gather never waits on a
 // global load issued in the same iteration.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ bool lut_in_lds(const MatDev &mat) {
-    return mat.mode == 0 && mat.n_classes <= OEM_LDS_CLASSES;
+// How a kernel reads the material coefficients: 0 the class LUT staged in LDS, 1 the class LUT
+// in global memory (more classes than LDS holds), 2 dense per-cell arrays.
+__host__ __device__ __forceinline__ int mat_kind(const MatDev &mat) {
+    return mat.mode != 0 ? 2 : mat.n_classes <= OEM_LDS_CLASSES ? 0 : 1;
 }
+__device__ __forceinline__ bool lut_in_lds(const MatDev &mat) { return mat_kind(mat) == 0; }
 
 // Stage the class LUT (2 float4 per class) in LDS; the caller brackets it with barriers.
 __device__ __forceinline__ void stage_lut(float4 *s_lut, const MatDev &mat) {
@@ -547,7 +552,8 @@ __device__ __forceinline__ void pw_h_inj(const PlaneSrcDev &pw, int k, const int
 }
 
 // ------------------------------------------------------------------------------------------
-// Fused H + E step.  A work-group owns a tile of OEM_CR rows (j) x 64 cells (k)
+// Fused H + E step.  A work-group owns a tile of OEM_CR rows (j) x 64 cells (k) (or 2 OEM_CR x 32
+// at the end of a row whose last strip holds at most 32 cells)
 // and marches it along x; every thread of the OEM_CR row waves keeps one (j, k) column, as in
 // the separate sweeps, and computes H^{n+1/2} and then E^{n+1} of each plane:
 //   * the old Ey, Ez of the plane and the new Hy, Hz of the plane before are carried in
@@ -563,19 +569,40 @@ __device__ __forceinline__ void pw_h_inj(const PlaneSrcDev &pw, int k, const int
 #ifndef OEM_CR
 #define OEM_CR 7            // owned rows (waves) per work-group; one halo wave more
 #endif
+#define OEM_CT (64 * OEM_CR)    // columns of a work-group: OEM_CR rows x 64 or 2 OEM_CR x 32
 // s_waitcnt vmcnt(0) with the other counters left alone (gfx9 encoding: vmcnt bits 3:0 and
 // 15:14, expcnt 6:4, lgkmcnt 11:8)
 #define OEM_WAIT_VM0 0x0F70
 
-// Buffer descriptors of the fused step: a field set is E then H in one allocation, a psi set
-// the H side then the E side; one descriptor each keeps the SGPRs the march needs low.
+// Buffer descriptors of the fused step: a field set is E then H in one allocation; one
+// descriptor each keeps the SGPRs the march needs low.  The H-side psi ping-pongs with the
+// fields (a halo recompute reads the old one of its neighbours' cells); the E-side psi is read
+// and written by its own thread alone and stays in place.
 struct ColIO {
     rsrc_t fo, fn;              // old / new field set
-    rsrc_t po, pn;              // old / new psi set
+    rsrc_t po, pn;              // old / new H-side psi
+    rsrc_t pe;                  // E-side psi
     uint32_t cb;                // bytes per field component
     uint32_t hof;               // bytes from E to H in a field set (3 * cb)
-    uint32_t pef;               // bytes from the H-side to the E-side psi in a psi set
 };
+
+// CPML coefficients of a tile's rows and cells in LDS: the rows (then the halo row) and the cells
+// (then the halo column), a, b, 1/kappa at H and at E.  Only the lanes of a slab read them; kept
+// in registers they held 12 of every thread.
+struct TileCpml {
+    float y[6][2 * OEM_CR + 1], z[6][65];
+};
+__device__ __forceinline__ void stage_cpml(TileCpml &t, const GridDev &g, int j0, int k0, int nr,
+                                           int kw, int jh, int kh, int tid, int nthr) {
+    const int fld[6] = {AX_AH, AX_BH, AX_KH, AX_AE, AX_BE, AX_KE};
+    for (int q = tid; q < nr + 1 + kw + 1; q += nthr) {
+        const bool row = q <= nr;
+        const int u = row ? q : q - nr - 1;
+        const int p = row ? (u < nr ? min(j0 + u, g.ny - 1) : jh) : (u < kw ? min(k0 + u, g.nz - 1) : kh);
+#pragma unroll
+        for (int f = 0; f < 6; ++f) (row ? t.y[f] : t.z[f])[u] = axv(g.ax[row ? 1 : 2], p, fld[f]);
+    }
+}
 
 // The H update at one (j, k) column: its per-column constants and the old Ey, Ez of the
 // current plane.
@@ -584,8 +611,8 @@ struct HColumn {
     uint32_t op, oj, ok;        // byte offsets in the plane: (j, k), (Y.nxt[j], k), (j, Z.nxt[k])
     uint32_t oy, oz;            // psi offsets in the y / z slab planes
     int sy, sz;                 // slab indices (-1 outside)
+    int ly, lz;                 // the row's and the cell's slot in the tile's CPML coefficients
     float mj, mji, idy, mk, mki, idz;
-    float ay, by, ky, az, bz, kz;
     float ihx, ihy;             // plane-wave H corrections at k
     F ey, ez;
 };
@@ -593,7 +620,7 @@ struct HColumn {
 template <typename F>
 __device__ __forceinline__ void hcolumn_init(HColumn<F> &c, const GridDev &g,
                                              const PlaneSrcDev &pw, const int *stp, int j, int k,
-                                             int jn, int kn) {
+                                             int jn, int kn, int ly, int lz) {
     typedef FT<F> T;
     const AxisDev &Y = g.ax[1], &Z = g.ax[2];
     const int nz = g.nz, pz = g.pz, wz = Z.lo + Z.hi;
@@ -606,9 +633,8 @@ __device__ __forceinline__ void hcolumn_init(HColumn<F> &c, const GridDev &g,
     c.oz = (uint32_t)(j * wz + max(c.sz, 0)) * T::B;
     c.mj = axv(Y, j, AX_MNX); c.mji = axv(Y, j, AX_MNXI); c.idy = axv(Y, j, AX_IDLP);
     c.mk = axv(Z, k, AX_MNX); c.mki = axv(Z, k, AX_MNXI); c.idz = axv(Z, k, AX_IDLP);
-    c.ay = 0.f; c.by = 1.f; c.ky = 1.f; c.az = 0.f; c.bz = 1.f; c.kz = 1.f;
-    if (c.sy >= 0) { c.ay = axv(Y, j, AX_AH); c.by = axv(Y, j, AX_BH); c.ky = axv(Y, j, AX_KH); }
-    if (c.sz >= 0) { c.az = axv(Z, k, AX_AH); c.bz = axv(Z, k, AX_BH); c.kz = axv(Z, k, AX_KH); }
+    c.ly = ly;
+    c.lz = lz;
     pw_h_inj(pw, k, stp, c.ihx, c.ihy);
     c.ey = c.ez = T::zero();
 }
@@ -679,11 +705,11 @@ __device__ __forceinline__ void hcolumn_load(HLoads<F> &v, const HColumn<F> &c, 
 // H^{n+1/2} of the column at plane i from its loaded inputs (the arithmetic of update_h_tile);
 // `xr` is the x-axis table row of plane i.  The column's Ey, Ez move on to plane X.nxt[i].  With
 // `store` the new H and H-side psi are written.
-template <typename F>
+template <typename F, int AUX>
 __device__ __forceinline__ void hcolumn_do(HColumn<F> &c, const HLoads<F> &v, const ColIO &io,
-                                           const GridDev &g, const PsiDev &ps, int i,
-                                           ctab_t xr, float ch, bool store, F &hx, F &hy,
-                                           F &hz) {
+                                           const GridDev &g, const PsiDev &ps,
+                                           const TileCpml &tc, int i, ctab_t xr, float ch,
+                                           bool store, F &hx, F &hy, F &hz) {
     typedef FT<F> T;
     const uint32_t so = (uint32_t)i * ((uint32_t)g.plane * T::B), sh = so + io.hof;
     const uint32_t c1 = io.cb, c2 = 2u * io.cb;
@@ -704,25 +730,27 @@ __device__ __forceinline__ void hcolumn_do(HColumn<F> &c, const HLoads<F> &v, co
         const float a_ = xr[AX_AH], b_ = xr[AX_BH], k_ = xr[AX_KH];
         s_hy_x = stretch_v(psx0, dzx, a_, b_, k_);
         s_hz_x = stretch_v(psx1, dyx, a_, b_, k_);
-        if (store) { T::st(io.pn, psx0, c.op, sx0); T::st(io.pn, psx1, c.op, sx1); }
+        if (store) { T::template st<AUX>(io.pn, psx0, c.op, sx0); T::template st<AUX>(io.pn, psx1, c.op, sx1); }
     }
     if (c.sy >= 0) {
-        s_hx_y = stretch_v(psy0, dzy, c.ay, c.by, c.ky);
-        s_hz_y = stretch_v(psy1, dxy, c.ay, c.by, c.ky);
-        if (store) { T::st(io.pn, psy0, c.oy, sy0); T::st(io.pn, psy1, c.oy, sy1); }
+        const float a_ = tc.y[0][c.ly], b_ = tc.y[1][c.ly], k_ = tc.y[2][c.ly];
+        s_hx_y = stretch_v(psy0, dzy, a_, b_, k_);
+        s_hz_y = stretch_v(psy1, dxy, a_, b_, k_);
+        if (store) { T::template st<AUX>(io.pn, psy0, c.oy, sy0); T::template st<AUX>(io.pn, psy1, c.oy, sy1); }
     }
     if (c.sz >= 0) {
-        s_hx_z = stretch_v(psz0, dyz, c.az, c.bz, c.kz);
-        s_hy_z = stretch_v(psz1, dxz, c.az, c.bz, c.kz);
-        if (store) { T::st(io.pn, psz0, c.oz, sz0); T::st(io.pn, psz1, c.oz, sz1); }
+        const float a_ = tc.z[0][c.lz], b_ = tc.z[1][c.lz], k_ = tc.z[2][c.lz];
+        s_hx_z = stretch_v(psz0, dyz, a_, b_, k_);
+        s_hy_z = stretch_v(psz1, dxz, a_, b_, k_);
+        if (store) { T::template st<AUX>(io.pn, psz0, c.oz, sz0); T::template st<AUX>(io.pn, psz1, c.oz, sz1); }
     }
     hx = T::addre(v.h0 - ch * (s_hx_y - s_hx_z), c.ihx);
     hy = T::addre(v.h1 - ch * (s_hy_z - s_hy_x), c.ihy);
     hz = v.h2 - ch * (s_hz_x - s_hz_y);
     if (store) {
-        T::st(io.fn, hx, c.op, sh);
-        T::st(io.fn, hy, c.op, sh + c1);
-        T::st(io.fn, hz, c.op, sh + c2);
+        T::template st<AUX>(io.fn, hx, c.op, sh);
+        T::template st<AUX>(io.fn, hy, c.op, sh + c1);
+        T::template st<AUX>(io.fn, hz, c.op, sh + c2);
     }
     c.ey = v.ey_n;
     c.ez = v.ez_n;
@@ -863,28 +891,29 @@ __device__ __forceinline__ void snap_flush(const SnapPlan<F> &p, const F *stage,
 // LDS, 1 the class LUT in global memory (more classes than LDS holds), 2 dense per-cell arrays.
 // MULTI: up to three fused monitors meet a work-group (else at most one, and the kernel holds
 // no registers for the others).
-template <typename F, int MK, bool MULTI>
+// AUX: the cache policy of its stores, plain while both field sets fit the memory-side cache.
+template <typename F, int MK, bool MULTI, int AUX>
 __global__ void __launch_bounds__(64 * (OEM_CR + 1))
 k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ En,
                 F *__restrict__ Hn, PsiDev ps, PsiDev pn, GridDev g, MatDev mat, float ch,
                 float cw, PlaneSrcDev pw, const int *__restrict__ stp, FuseSnap fs)
 {
     typedef FT<F> T;
-    // Ho = Eo + 3 components and ps.e = ps.h + ps.total (the host allocates them so)
+    // Ho = Eo + 3 components (the host allocates them so)
     ColIO io;
     {
         const size_t nc = (size_t)g.plane * g.nx;
         io.cb = (uint32_t)(nc * T::B);
         io.hof = 3u * io.cb;
-        io.pef = ps.total * T::B;
+        const uint32_t pb = ps.total * T::B;
         io.fo = mk_rsrc(Eo, 2u * io.hof); io.fn = mk_rsrc(En, 2u * io.hof);
-        io.po = mk_rsrc(ps.h, 2u * io.pef); io.pn = mk_rsrc(pn.h, 2u * io.pef);
+        io.po = mk_rsrc(ps.h, pb); io.pn = mk_rsrc(pn.h, pb); io.pe = mk_rsrc(ps.e, pb);
     }
     __shared__ float4 s_lut[2 * OEM_LDS_CLASSES];
-    // new H per row slot (0: the halo row, 1 + w: row wave w) and of the halo column, by
-    // plane parity
-    __shared__ F s_row[2][3][OEM_CR + 1][64];
-    __shared__ F s_col[2][2][OEM_CR];
+    // new H by plane parity: the halo row (kw lanes), then the tile's columns row by row, so a
+    // column's own slot is kw + q and the row above it is slot q; and of the halo column
+    __shared__ F s_row[2][3][OEM_CT + 64];
+    __shared__ F s_col[2][2][2 * OEM_CR];
     // snapshot stage by plane parity ([component][point]), the points' ring offsets, and the
     // row waves' point counts
     __shared__ F s_fsn[2][6 * 64];
@@ -892,19 +921,35 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
     __shared__ int s_fcnt[OEM_CR];
     const AxisDev &X = g.ax[0], &Y = g.ax[1], &Z = g.ax[2];
     const int nx = g.nx, ny = g.ny, nz = g.nz, pz = g.pz;
-    const int nkt = (nz + 63) / 64;
     // per-work-group quantities through readfirstlane: the compiler then keeps them in SGPRs
     const int lb = xcd_remap(blockIdx.x, g.nblocks);
     const int tile = __builtin_amdgcn_readfirstlane(lb % g.tiles);
     const int chunk = __builtin_amdgcn_readfirstlane(lb / g.tiles);
-    const int j0 = __builtin_amdgcn_readfirstlane((tile / nkt) * OEM_CR);
-    const int k0 = __builtin_amdgcn_readfirstlane((tile % nkt) * 64);
+    // the tile: nr rows x kw = 1 << lw lanes from (j0, k0)
+    int lw = 6, jt, k0;
+    if (tile < g.t64) {
+        jt = tile / g.kt64;
+        k0 = (tile - jt * g.kt64) * 64;
+    } else {
+        lw = 5;
+        jt = tile - g.t64;
+        k0 = g.kt64 * 64;
+    }
+    lw = __builtin_amdgcn_readfirstlane(lw);
+    k0 = __builtin_amdgcn_readfirstlane(k0);
+    const int kw = 1 << lw, nr = OEM_CT >> lw;
+    const int j0 = __builtin_amdgcn_readfirstlane(jt * nr);
     const int i0 = chunk * g.chunk, i1 = min(i0 + g.chunk, nx);
-    constexpr bool lds_lut = MK == 0;
-    if constexpr (lds_lut) {
+    const int jh = __builtin_amdgcn_readfirstlane(Y.prv[j0]);       // halo row and column
+    const int kh = __builtin_amdgcn_readfirstlane(Z.prv[k0]);
+    __shared__ TileCpml s_pml;
+    {
         const int tid = threadIdx.y * 64 + threadIdx.x;
-        const float4 *src = reinterpret_cast<const float4 *>(mat.lut);
-        for (int q = tid; q < 2 * mat.n_classes; q += 64 * (OEM_CR + 1)) s_lut[q] = src[q];
+        if constexpr (MK == 0) {
+            const float4 *src = reinterpret_cast<const float4 *>(mat.lut);
+            for (int q = tid; q < 2 * mat.n_classes; q += 64 * (OEM_CR + 1)) s_lut[q] = src[q];
+        }
+        stage_cpml(s_pml, g, j0, k0, nr, kw, jh, kh, tid, 64 * (OEM_CR + 1));
         __syncthreads();
     }
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
@@ -916,7 +961,9 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
     const size_t ncell = (size_t)g.plane * nx;
 
     // Threads outside the grid work on a clamped in-range column and store nothing.
-    const int kl = min(k0 + lane, nz - 1);
+    const int tq = min(w, OEM_CR - 1) * 64 + lane;      // the column of a row wave's thread
+    const int rr = tq >> lw, kk = tq & (kw - 1);
+    const int kl = min(k0 + kk, nz - 1);
     const int xp0 = __builtin_amdgcn_readfirstlane(X.prv[i0]);
     // the fused DFT monitor that meets this work-group's tile and chunk (the host fuses monitors
     // whose work-groups are disjoint; most work-groups meet none), set up here so that the march
@@ -933,10 +980,10 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
     fp3.ilo = fp3.ihi = 0;
     if (fs.n) {
         uint32_t fmask = __builtin_amdgcn_readfirstlane(
-            fuse_snap_mask(fs, nx, ny, nz, i0, i1, j0, j0 + OEM_CR, k0, k0 + 64));
+            fuse_snap_mask(fs, nx, ny, nz, i0, i1, j0, j0 + nr, k0, k0 + kw));
         if (fmask) {
             const int fstep = __builtin_amdgcn_readfirstlane(step_now(stp));
-            const int jr = min(j0 + min(w, OEM_CR - 1), ny - 1);
+            const int jr = min(j0 + rr, ny - 1);
             // all but qjk are the same across the work-group
             auto uniform = [](SnapPlan<F> &p) {
                 const uint64_t rp = reinterpret_cast<uint64_t>(p.row);
@@ -965,17 +1012,25 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         }
     }
     if (w == OEM_CR) {
-        // the halo wave: the new H of (Y.prv[j0], k0 + lane) and of (j0 + lane, Z.prv[k0]) for
-        // lane < OEM_CR, into LDS slot 0 and the column slots; one barrier per plane, as the
-        // row waves
-        const int jh = __builtin_amdgcn_readfirstlane(Y.prv[j0]);
-        const int kh = __builtin_amdgcn_readfirstlane(Z.prv[k0]);
-        const int jc = min(j0 + min(lane, OEM_CR - 1), ny - 1);
+        // the halo wave: the new H of the halo row (Y.prv[j0], k0 + 0 .. kw - 1) into the first
+        // slots and of the halo column (j0 + 0 .. nr - 1, Z.prv[k0]) into the column slots, one
+        // barrier per plane as the row waves.  A 32-wide tile's row and column (32 + 14 lanes)
+        // fit the wave together; a 64-wide one takes two passes
+        const bool two = lw == 6;
+        const int cl = two ? lane : lane - kw;              // this lane's row of the halo column
+        const bool in_row = lane < kw, in_col = cl >= 0 && cl < nr;
+        const int cs = max(min(cl, nr - 1), 0), ks = lane & (kw - 1);
+        const int jc = min(j0 + cs, ny - 1), kr = min(k0 + ks, nz - 1);
+        const int ja = in_row ? jh : jc, ka = in_row ? kr : kh;
         HColumn<F> cr, cc;
-        hcolumn_init<F>(cr, g, pw, stp, jh, kl, next_of(jh, ny, yn_last), next_of(kl, nz, zn_last));
-        hcolumn_init<F>(cc, g, pw, stp, jc, kh, next_of(jc, ny, yn_last), next_of(kh, nz, zn_last));
+        hcolumn_init<F>(cr, g, pw, stp, ja, ka, next_of(ja, ny, yn_last), next_of(ka, nz, zn_last),
+                        in_row ? nr : cs, in_row ? ks : kw);
         hcolumn_load_e<F>(cr, io, g, i0);
-        hcolumn_load_e<F>(cc, io, g, i0);
+        if (two) {
+            hcolumn_init<F>(cc, g, pw, stp, jc, kh, next_of(jc, ny, yn_last), next_of(kh, nz, zn_last), cs,
+                            kw);
+            hcolumn_load_e<F>(cc, io, g, i0);
+        }
         if (fplan) fcnt = snap_rank(false, w, lane, 0, s_fcnt, s_fq, fslot);
 #pragma unroll 1
         for (int i = i0; i < i1; ++i) {
@@ -984,15 +1039,17 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
             F hx, hy, hz;
             HLoads<F> vr, vc;
             hcolumn_load<F>(vr, cr, io, g, ps, i, in_);
-            hcolumn_load<F>(vc, cc, io, g, ps, i, in_);
+            if (two) hcolumn_load<F>(vc, cc, io, g, ps, i, in_);
             const ctab_t xr = ctab_row(X, i);
-            hcolumn_do<F>(cr, vr, io, g, ps, i, xr, ch, false, hx, hy, hz);
-            s_row[buf][0][0][lane] = hx;
-            s_row[buf][2][0][lane] = hz;
-            hcolumn_do<F>(cc, vc, io, g, ps, i, xr, ch, false, hx, hy, hz);
-            if (lane < OEM_CR) {
-                s_col[buf][0][lane] = hx;
-                s_col[buf][1][lane] = hy;
+            hcolumn_do<F, AUX>(cr, vr, io, g, ps, s_pml, i, xr, ch, false, hx, hy, hz);
+            if (in_row) {
+                s_row[buf][0][lane] = hx;
+                s_row[buf][2][lane] = hz;
+            }
+            if (two) hcolumn_do<F, AUX>(cc, vc, io, g, ps, s_pml, i, xr, ch, false, hx, hy, hz);
+            if (in_col) {
+                s_col[buf][0][cl] = hx;
+                s_col[buf][1][cl] = hy;
             }
             __syncthreads();
             // the row waves staged plane i - 1 before this barrier
@@ -1007,18 +1064,15 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         return;
     }
 
-    // a row wave: column (j0 + w, k0 + lane)
-    const int j = min(j0 + w, ny - 1), k = kl;
-    const bool own = j0 + w < ny && k0 + lane < nz;
+    // a row wave's thread: column (j0 + rr, k0 + kk)
+    const int j = min(j0 + rr, ny - 1), k = kl;
+    const bool own = j0 + rr < ny && k0 + kk < nz;
     HColumn<F> ca;
-    hcolumn_init<F>(ca, g, pw, stp, j, k, next_of(j, ny, yn_last), next_of(k, nz, zn_last));
+    hcolumn_init<F>(ca, g, pw, stp, j, k, next_of(j, ny, yn_last), next_of(k, nz, zn_last), rr, kk);
     const float mjE = axv(Y, j, AX_MPV), mjEi = axv(Y, j, AX_MPVI);
     const float idyE = axv(Y, j, AX_IDLD), pecy = axv(Y, j, AX_PEC);
     const float mkE = axv(Z, k, AX_MPV), mkEi = axv(Z, k, AX_MPVI);
     const float idzE = axv(Z, k, AX_IDLD), pecz = axv(Z, k, AX_PEC);
-    float ayE = 0.f, byE = 1.f, kyE = 1.f, azE = 0.f, bzE = 1.f, kzE = 1.f;
-    if (ca.sy >= 0) { ayE = axv(Y, j, AX_AE); byE = axv(Y, j, AX_BE); kyE = axv(Y, j, AX_KE); }
-    if (ca.sz >= 0) { azE = axv(Z, k, AX_AE); bzE = axv(Z, k, AX_BE); kzE = axv(Z, k, AX_KE); }
     float inj_ex = 0.f, inj_ey = 0.f;
     bool inj_x = false, inj_y = false;
     if (pw.n) {
@@ -1046,7 +1100,7 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         HLoads<F> vp;
         hcolumn_load<F>(vp, cp, io, g, ps, xp0, next_of(xp0, nx, xn_last));
         F hx_;
-        hcolumn_do<F>(cp, vp, io, g, ps, xp0, ctab_row(X, xp0), ch, false, hx_, hy_m,
+        hcolumn_do<F, AUX>(cp, vp, io, g, ps, s_pml, xp0, ctab_row(X, xp0), ch, false, hx_, hy_m,
                       hz_m);
     }
     hcolumn_load_e<F>(ca, io, g, i0);
@@ -1097,9 +1151,9 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         }
         F pe0 = T::zero(), pe1 = T::zero(), pe2 = T::zero(), pe3 = T::zero(), pe4 = T::zero(),
           pe5 = T::zero();
-        if (sx >= 0) { pe0 = T::ld(io.po, ca.op, sx0 + io.pef); pe1 = T::ld(io.po, ca.op, sx1 + io.pef); }
-        if (ca.sy >= 0) { pe2 = T::ld(io.po, ca.oy, sy0 + io.pef); pe3 = T::ld(io.po, ca.oy, sy1 + io.pef); }
-        if (ca.sz >= 0) { pe4 = T::ld(io.po, ca.oz, sz0 + io.pef); pe5 = T::ld(io.po, ca.oz, sz1 + io.pef); }
+        if (sx >= 0) { pe0 = T::ld(io.pe, ca.op, sx0); pe1 = T::ld(io.pe, ca.op, sx1); }
+        if (ca.sy >= 0) { pe2 = T::ld(io.pe, ca.oy, sy0); pe3 = T::ld(io.pe, ca.oy, sy1); }
+        if (ca.sz >= 0) { pe4 = T::ld(io.pe, ca.oz, sz0); pe5 = T::ld(io.pe, ca.oz, sz1); }
         HLoads<F> cv;
         hcolumn_load<F>(cv, ca, io, g, ps, i, in_);
         if (MK != 2 && i + 1 < i1) cls_c = bld_u16(rC, oc, (uint32_t)(i + 1) * plane2);
@@ -1111,14 +1165,14 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         F hx, hy, hz;
         const ctab_t xr = ctab_row(X, i);
         const F ex0 = cv.ex;
-        hcolumn_do<F>(ca, cv, io, g, ps, i, xr, ch, own, hx, hy, hz);
-        s_row[buf][0][w + 1][lane] = hx;
-        s_row[buf][1][w + 1][lane] = hy;
-        s_row[buf][2][w + 1][lane] = hz;
+        hcolumn_do<F, AUX>(ca, cv, io, g, ps, s_pml, i, xr, ch, own, hx, hy, hz);
+        s_row[buf][0][kw + tq] = hx;
+        s_row[buf][1][kw + tq] = hy;
+        s_row[buf][2][kw + tq] = hz;
         __syncthreads();
-        const F hx_j = s_row[buf][0][w][lane], hz_j = s_row[buf][2][w][lane];
-        const F hx_k = lane ? s_row[buf][0][w + 1][lane - 1] : s_col[buf][0][w];
-        const F hy_k = lane ? s_row[buf][1][w + 1][lane - 1] : s_col[buf][1][w];
+        const F hx_j = s_row[buf][0][tq], hz_j = s_row[buf][2][tq];
+        const F hx_k = kk ? s_row[buf][0][kw + tq - 1] : s_col[buf][0][rr];
+        const F hy_k = kk ? s_row[buf][1][kw + tq - 1] : s_col[buf][1][rr];
         const F hpx = phx, hpy = phy, hpz = phz;
         const float mi = xr[AX_MPV], mii = xr[AX_MPVI];
         const float idx = xr[AX_IDLD], pecx = xr[AX_PEC];
@@ -1133,17 +1187,19 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
             const float a_ = xr[AX_AE], b_ = xr[AX_BE], k_ = xr[AX_KE];
             s_ey_x = stretch_v(pe0, dzx, a_, b_, k_);
             s_ez_x = stretch_v(pe1, dyx, a_, b_, k_);
-            if (own) { T::st(io.pn, pe0, ca.op, sx0 + io.pef); T::st(io.pn, pe1, ca.op, sx1 + io.pef); }
+            if (own) { T::template st<AUX>(io.pe, pe0, ca.op, sx0); T::template st<AUX>(io.pe, pe1, ca.op, sx1); }
         }
         if (ca.sy >= 0) {
-            s_ex_y = stretch_v(pe2, dzy, ayE, byE, kyE);
-            s_ez_y = stretch_v(pe3, dxy, ayE, byE, kyE);
-            if (own) { T::st(io.pn, pe2, ca.oy, sy0 + io.pef); T::st(io.pn, pe3, ca.oy, sy1 + io.pef); }
+            const float a_ = s_pml.y[3][rr], b_ = s_pml.y[4][rr], k_ = s_pml.y[5][rr];
+            s_ex_y = stretch_v(pe2, dzy, a_, b_, k_);
+            s_ez_y = stretch_v(pe3, dxy, a_, b_, k_);
+            if (own) { T::template st<AUX>(io.pe, pe2, ca.oy, sy0); T::template st<AUX>(io.pe, pe3, ca.oy, sy1); }
         }
         if (ca.sz >= 0) {
-            s_ex_z = stretch_v(pe4, dyz, azE, bzE, kzE);
-            s_ey_z = stretch_v(pe5, dxz, azE, bzE, kzE);
-            if (own) { T::st(io.pn, pe4, ca.oz, sz0 + io.pef); T::st(io.pn, pe5, ca.oz, sz1 + io.pef); }
+            const float a_ = s_pml.z[3][kk], b_ = s_pml.z[4][kk], k_ = s_pml.z[5][kk];
+            s_ex_z = stretch_v(pe4, dyz, a_, b_, k_);
+            s_ey_z = stretch_v(pe5, dxz, a_, b_, k_);
+            if (own) { T::template st<AUX>(io.pe, pe4, ca.oz, sz0); T::template st<AUX>(io.pe, pe5, ca.oz, sz1); }
         }
         F nex = (cax * ex0 + cbx * (s_ex_y - s_ex_z - cw * hpx)) * pecy * pecz;
         F ney = (cay * ey0 + cby * (s_ey_z - s_ey_x - cw * hpy)) * pecz * pecx;
@@ -1151,9 +1207,9 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         if (inj_x) nex = T::addre(nex, cbx * inj_ex);
         if (inj_y) ney = T::addre(ney, cby * inj_ey);
         if (own) {
-            T::st(io.fn, nex, ca.op, so);
-            T::st(io.fn, ney, ca.op, so + io.cb);
-            T::st(io.fn, nez, ca.op, so + 2u * io.cb);
+            T::template st<AUX>(io.fn, nex, ca.op, so);
+            T::template st<AUX>(io.fn, ney, ca.op, so + io.cb);
+            T::template st<AUX>(io.fn, nez, ca.op, so + 2u * io.cb);
             if (i >= fp.ilo && i < fp.ihi && fp.qjk >= 0)
                 snap_planned<F>(fp, i, fcnt >= 0 ? s_fsn[buf] : nullptr, fslot, nex, ney, nez, hx,
                                 hy, hz, hy_m, hz_m, hx_j, hz_j, hx_k, hy_k);

@@ -121,8 +121,8 @@ int ctx_init(oem_ctx *c, const oem_dims *d, int32_t device) {
         }
     if (total * 4 * c->esz > 0xffffffffull) return fail(OEM_ENOTSUP, "CPML slabs exceed 4 GiB per side");
     c->psi.total = (uint32_t)(total ? total : 1);
-    // E and H in one allocation (H right after E), and the H- and E-side psi in one: a kernel
-    // then reaches a whole field set, or a whole psi set, through one buffer descriptor
+    // E and H in one allocation (H right after E): a kernel then reaches a whole field set
+    // through one buffer descriptor
     TRY(c->alloc(&c->E, 6 * nc * c->esz, true));
     c->H = c->E + 3 * nc * c->esz;
     float *pp = nullptr;
@@ -723,7 +723,8 @@ extern "C" int oem_read_flux_time_monitor(oem_ctx *ctx, int32_t mon_id, double *
 // after the corrections, so every snapshot holds the final fields).
 static int plan_fused_snaps(oem_ctx *ctx) {
     const int nx = ctx->dims.nx, ny = ctx->dims.ny, nz = ctx->dims.nz;
-    const int tile[3] = {ctx->fg.chunk, OEM_CR, 64};
+    // the rows of the taller, 32-wide tiles where there are any
+    const int tile[3] = {ctx->fg.chunk, ctx->fg.tiles > ctx->fg.t64 ? 2 * OEM_CR : OEM_CR, 64};
     std::vector<std::array<int, 6>> taken;   // fused footprints: first, last tile per axis
     auto footprint = [&](const MonDev &m) {
         int lo[3] = {0, 0, 0}, hi[3] = {nx, ny, nz};
@@ -803,6 +804,47 @@ static int plan_fused_snaps(oem_ctx *ctx) {
     return OEM_OK;
 }
 
+// The fused step's tiles of the (ny, nz) plane: 64-wide strips and, when at most 32 cells of a
+// row are left, one 32-wide strip of twice the rows, which idles fewer lanes (step times with and
+// without it: 200^3 186 / 201 us, 144^3 57.5 / 59.8, 80^3 23.6 / 25.6, 250 x 230 x 210 233 / 241).
+// Not with dense coefficients, whose 24 bytes a cell cost more lines in it: 150 x 133 x 141 took
+// 57.1 us with and 53.4 without.
+static void march_tiles(GridDev &g, bool dense) {
+    const int n32 = (g.nz + 31) / 32;
+    g.kt64 = dense ? (n32 + 1) / 2 : n32 / 2;
+    g.t64 = g.kt64 * ((g.ny + OEM_CR - 1) / OEM_CR);
+    g.tiles = g.t64;
+    if (!dense && (n32 & 1)) g.tiles += (g.ny + 2 * OEM_CR - 1) / (2 * OEM_CR);
+}
+
+// Bytes of the state a fused march goes through over two steps: both field sets, both H-side psi
+// and the E-side psi.
+static uint64_t march_bytes(const oem_ctx *c) {
+    const uint64_t f = 4ull * c->esz;
+    return 12 * f * c->nst + 3 * f * c->psi.total;
+}
+// With at most this much of it the memory-side cache (256 MiB) still holds a step's result when the
+// next step reads it, and the march's stores are plain; past it they are non-temporal (step times
+// plain / non-temporal: 128^3, 126 MiB, 45.6 / 61 us; 144^3, 171 MiB, 58 / 83; 160^3, 230 MiB,
+// 99 / 93; 512^3 1.74 / 1.70 ms).
+#define OEM_MARCH_CACHED (200ull << 20)
+
+// Whether the fused H+E step is the faster form.  It moves two thirds of the sweeps' bytes but
+// alternates between two field sets.  From OEM_FUSE_MIN_CELLS on the bytes decide: 320^3 516 us
+// against 677 with the two sweeps, 512^3 1.70 ms against 2.53.  While its state stays in the
+// memory-side cache it wins as well, and takes the monitors' snapshots and the step's end with it
+// (about 4.6 us a launch): with three flux planes 128^3 55.5 us against 69.9, 64^3 24.2 / 32.8,
+// 97 x 89 x 103 35 / 43; without monitors 45.6 / 55.0, 17.3 / 20.5, 27.9 / 29.2.  In between one
+// set fits the cache and two do not: 160^3 with the planes 108 us against 90.6, 200^3 203 / 191.
+// Smaller scenes with an H-side point list keep the sweeps: the march adds it to H before the
+// update, the sweeps after it, and their results keep that rounding.
+static bool march_pays(const oem_ctx *c) {
+    if (c->ncell >= OEM_FUSE_MIN_CELLS) return true;
+    for (const auto &p : c->points)
+        if (p.magnetic) return false;
+    return march_bytes(c) <= OEM_MARCH_CACHED;
+}
+
 extern "C" int oem_prepare(oem_ctx *ctx) {
     CHECK_CTX(ctx);
     if (ctx->prepared) return OEM_OK;
@@ -867,15 +909,11 @@ extern "C" int oem_prepare(oem_ctx *ctx) {
     const long long nb = (long long)g.tiles * ((g.nx + g.chunk - 1) / g.chunk);
     if (nb > 0x7fffffffLL) return fail(OEM_EINVAL, "launch too large");
     g.nblocks = (int)nb;
-    // the fused H+E step for scenes of OEM_FUSE_MIN_CELLS and more (OEM_FUSE=1: any size, 0:
-    // never), outside a serving pool.  Measured step times (box soup, two sweeps / fused):
-    // 64^3 30 / 29-55 us, 128^3 69 / 65-83 us, 160^3 98 / 132 us, 200^3 241 / 240 us, 256^3
-    // 393 / 355-361 us, 320^3 677 / 596 us, 512^3 2.54 / 1.99 ms: below ~8 M cells a fused
-    // work-group marches too few tiles to fill the GPU
+    // OEM_FUSE=1: the fused H+E step at any size, 0: never, outside a serving pool
     // (oem_set_step_form overrides the rule and OEM_FUSE)
     const char *fe = std::getenv("OEM_FUSE");
     bool fuse = !ctx->pool && !(fe && fe[0] == '0');
-    if (!(fe && fe[0] == '1')) fuse &= ctx->ncell >= OEM_FUSE_MIN_CELLS;
+    if (!(fe && fe[0] == '1')) fuse &= march_pays(ctx);
     if (ctx->form_req) fuse = ctx->form_req == 2;
     // it addresses a whole field set (E and H, six components) and a whole psi set (both sides)
     // with 32-bit offsets
@@ -889,18 +927,20 @@ extern "C" int oem_prepare(oem_ctx *ctx) {
         TRY(ctx->alloc(&ctx->E2, 6 * nc * ctx->esz, true));
         ctx->H2 = ctx->E2 + 3 * nc * ctx->esz;
         float *pp = nullptr;
-        TRY(ctx->alloc(&pp, 2 * (size_t)ctx->psi.total * ctx->esz, true));
-        ctx->psi2 = ctx->psi;
+        TRY(ctx->alloc(&pp, (size_t)ctx->psi.total * ctx->esz, true));
+        ctx->psi2 = ctx->psi;       // the E-side psi stays in place
         ctx->psi2.h = pp;
-        ctx->psi2.e = pp + (size_t)ctx->psi.total * ctx->esz;
         HIP_OK(hipStreamSynchronize(ctx->stream));
-        // one work-group per (OEM_CR rows x 64 k) tile and x chunk.  Measured step times:
-        // real fields at 512^3 (3 work-groups per CU), chunks 8 / 10 / 12 / 16 / 24 / 32: 2.00 /
-        // 1.96 / 1.93 / 1.94 / 1.93 / 1.94 ms; the complex Bloch cell (2 per CU), chunks 12 / 16
-        // / 24 / 32: 1.24 / 1.20 / 1.22 / 1.20 ms
         ctx->fg = g;
-        ctx->fg.tiles = ((g.nz + 63) / 64) * ((g.ny + OEM_CR - 1) / OEM_CR);
-        int fchunk = ctx->cplx ? 16 : 12;
+        march_tiles(ctx->fg, mat_kind(ctx->mat) == 2);
+        // x planes a work-group marches: enough work-groups for the chip in a small scene, few
+        // prologue planes in a large one.  Step times by chunk (us): 64^3 2 / 4 / 8: 17.6 / 18.5 /
+        // 24.9; 128^3 2 / 4 / 6 / 8: 49 / 45.6 / 49 / 50; 200^3 6 / 8 / 12: 187 / 186 / 194; 256^3
+        // 8 / 12: 271 / 278; 512^3 8 / 12 / 16 / 24: 2000 / 1930 / 1940 / 1930; complex 64 x 64 x
+        // 200 2 / 4 / 8: 38 / 35 / 41, 256 x 256 x 600 12 / 16 / 24: 1240 / 1200 / 1220
+        const int64_t planes = (int64_t)ctx->fg.tiles * g.nx;
+        const int per = ctx->cplx ? 650 : 1300, most = ctx->cplx ? 16 : planes < 100000 ? 8 : 12;
+        int fchunk = (int)std::min<int64_t>(most, std::max<int64_t>(2, (planes + per / 2) / per));
         if (ctx->chunk_req > 0) fchunk = ctx->chunk_req;
         else if (env && std::atoi(env) > 0) fchunk = std::atoi(env);
         ctx->fg.chunk = std::min(fchunk, g.nx);
@@ -908,6 +948,7 @@ extern "C" int oem_prepare(oem_ctx *ctx) {
         if (fb > 0x7fffffffLL) return fail(OEM_EINVAL, "launch too large");
         ctx->fg.nblocks = (int)fb;
         ctx->fused = true;
+        ctx->fuse_plain = march_bytes(ctx) <= OEM_MARCH_CACHED;
         const char *fsn = std::getenv("OEM_FUSE_SNAP");
         if (!(fsn && fsn[0] == '0')) TRY(plan_fused_snaps(ctx));
     }
@@ -1017,20 +1058,22 @@ int launch_step_t(oem_ctx *c, int flush_after, Prof *pr, bool last) {
         TRY(mark(OEM_K_UPDATE_HE, true));
         const FuseSnap fsn = c->mons_off ? FuseSnap{} : c->fsnap;
         const dim3 hg(c->fg.nblocks), hb(64, OEM_CR + 1);
-        const int mk = c->mat.mode != 0 ? 2 : c->mat.n_classes <= OEM_LDS_CLASSES ? 0 : 1;
-#define OEM_HE_LAUNCH(MKV, MULTIV)                                                        \
-        hipLaunchKernelGGL((k_update_he<F, MKV, MULTIV>), hg, hb, 0, c->stream,            \
+        const int mk = mat_kind(c->mat);
+#define OEM_HE_LAUNCH(MKV, MULTIV, AUXV)                                                  \
+        hipLaunchKernelGGL((k_update_he<F, MKV, MULTIV, AUXV>), hg, hb, 0, c->stream,      \
                            (const F *)Eo, (const F *)Ho, E, H, po, pn, c->fg, c->mat,       \
                            c->dims.ch, c->dims.cw, c->pw, c->d_step, fsn)
-        if (!c->mons_off && c->fsnap_multi) {
-            if (mk == 0) OEM_HE_LAUNCH(0, true);
-            else if (mk == 1) OEM_HE_LAUNCH(1, true);
-            else OEM_HE_LAUNCH(2, true);
+#define OEM_HE_KIND(MULTIV, AUXV)                                                         \
+        if (mk == 0) OEM_HE_LAUNCH(0, MULTIV, AUXV);                                       \
+        else if (mk == 1) OEM_HE_LAUNCH(1, MULTIV, AUXV);                                  \
+        else OEM_HE_LAUNCH(2, MULTIV, AUXV)
+        const bool multi = !c->mons_off && c->fsnap_multi;
+        if (c->fuse_plain) {
+            if (multi) { OEM_HE_KIND(true, 0); } else { OEM_HE_KIND(false, 0); }
         } else {
-            if (mk == 0) OEM_HE_LAUNCH(0, false);
-            else if (mk == 1) OEM_HE_LAUNCH(1, false);
-            else OEM_HE_LAUNCH(2, false);
+            if (multi) { OEM_HE_KIND(true, OEM_ST_NT); } else { OEM_HE_KIND(false, OEM_ST_NT); }
         }
+#undef OEM_HE_KIND
 #undef OEM_HE_LAUNCH
         TRY(mark(OEM_K_UPDATE_HE, false));
     } else {
