@@ -1756,66 +1756,97 @@ __device__ __forceinline__ void dft_acc(double &sr, double &si, cf2 v, double c,
     si += (double)v.r * s + (double)v.i * c;
 }
 
-// Replay the snapshots of steps first..last (in step order) for point q at frequency f; NC
-// components of which the first NC/2 are E (whole-step phase).
-template <typename F, int NC>
-__device__ __forceinline__ void flush_point(const MonDev &m, int first, int last, int f, int q)
+// Replay of one (component, frequency group) of a monitor for the 256 points of a block: a
+// thread per point forms the group's sums over the cnt snapshots from step `first` in step order
+// and adds them to the accumulators.  The time of a small monitor was the chain of a load and a
+// scalar phase read per step (22-29 us for 16 steps whatever its size, once per monitor), so the
+// phases are staged in LDS and 16 snapshots are in flight before the first is used: three flux
+// planes of 64^3 went from 47 to 8.5 us a batch in one launch, of 256^3 from 65 to 34.
+#define OEM_FLUSH_FG 8          // frequencies of a group: each snapshot is read once per group
+#define OEM_FLUSH_BLK 256
+// G: the group's frequencies, rounded up to 1, 2, 4 or 8 (the phases past nfl are zero)
+template <typename F, int G>
+__device__ __forceinline__ void flush_sums(const MonDev &m, int c, int f0, int nfl, int q,
+                                           int first, int cnt,
+                                           const double2 (*__restrict__ ph)[OEM_FLUSH_FG])
 {
-    double sre[NC], sim[NC];
+    double sre[G], sim[G];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) { sre[c] = 0.0; sim[c] = 0.0; }
-    for (int s = first; s <= last; ++s) {
-        const F *row = static_cast<const F *>(m.snap) + (size_t)(s % m.T) * NC * m.npts;
-        const double *ph = m.phase + ((size_t)s * m.nf + f) * 4;
-        const double ce = ph[0], se = ph[1], chh = ph[2], shh = ph[3];
+    for (int u = 0; u < G; ++u) { sre[u] = 0.0; sim[u] = 0.0; }
+    const size_t row = (size_t)m.ncomp * m.npts;
+    const F *col = static_cast<const F *>(m.snap) + (size_t)c * m.npts + q;
+    int slot = first % m.T, s = 0;
+    for (; s + 16 <= cnt; s += 16) {
+        F v[16];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const F v = row[(size_t)c * m.npts + q];
-            dft_acc(sre[c], sim[c], v, c < NC / 2 ? ce : chh, c < NC / 2 ? se : shh);
+        for (int e = 0; e < 16; ++e) {
+            v[e] = col[(size_t)slot * row];
+            slot = slot + 1 == m.T ? 0 : slot + 1;
         }
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+#pragma unroll
+            for (int u = 0; u < G; ++u) dft_acc(sre[u], sim[u], v[e], ph[s + e][u].x, ph[s + e][u].y);
+    }
+    for (; s < cnt; ++s) {
+        const F v = col[(size_t)slot * row];
+        slot = slot + 1 == m.T ? 0 : slot + 1;
+#pragma unroll
+        for (int u = 0; u < G; ++u) dft_acc(sre[u], sim[u], v, ph[s][u].x, ph[s][u].y);
     }
 #pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        const size_t o = ((size_t)c * m.nf + f) * m.npts + q;
-        m.re[o] += sre[c];
-        m.im[o] += sim[c];
-    }
-}
-
-// Replay of a single-scene monitor: a thread per (point, component) and group of up to
-// OEM_FLUSH_FG frequencies, so each snapshot value is read once per group, not once per
-// frequency (the phase rows are the same for the whole block and come through scalar loads).
-// Each (point, component, frequency) sum is formed in the order flush_point forms it, so both
-// give the same bits.  grid: x over points, y over (component, frequency group).  Launched after
-// the step counter advanced past the last snapshot: the cnt snapshots ending at step *stp - 1
-// are replayed.
-#define OEM_FLUSH_FG 8
-template <typename F>
-__global__ void __launch_bounds__(256)
-k_dft_flush(MonDev m, int cnt, const int *__restrict__ stp)
-{
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    const int ngrp = (m.nf + OEM_FLUSH_FG - 1) / OEM_FLUSH_FG;
-    const int c = blockIdx.y / ngrp, f0 = (blockIdx.y - c * ngrp) * OEM_FLUSH_FG;
-    if (q >= m.npts || c >= m.ncomp) return;
-    const int nfl = min(OEM_FLUSH_FG, m.nf - f0);
-    const int last = step_now(stp) - 1, first = last - cnt + 1;
-    const int po = c < m.ncomp / 2 ? 0 : 2;        // E: whole-step phase, H: half-step phase
-    double sre[OEM_FLUSH_FG], sim[OEM_FLUSH_FG];
-#pragma unroll
-    for (int u = 0; u < OEM_FLUSH_FG; ++u) { sre[u] = 0.0; sim[u] = 0.0; }
-    for (int s = first; s <= last; ++s) {
-        const F v = static_cast<const F *>(m.snap)[((size_t)(s % m.T) * m.ncomp + c) * m.npts + q];
-        const double *ph = m.phase + ((size_t)s * m.nf + f0) * 4 + po;
-#pragma unroll
-        for (int u = 0; u < OEM_FLUSH_FG; ++u)
-            if (u < nfl) dft_acc(sre[u], sim[u], v, ph[4 * u], ph[4 * u + 1]);
-    }
-#pragma unroll
-    for (int u = 0; u < OEM_FLUSH_FG; ++u)
+    for (int u = 0; u < G; ++u)
         if (u < nfl) {
             const size_t o = ((size_t)c * m.nf + f0 + u) * m.npts + q;
             m.re[o] += sre[u];
             m.im[o] += sim[u];
         }
+}
+
+// Block `b` of monitor m: its points (b mod the point blocks) of one component and group.
+template <typename F>
+__device__ __forceinline__ void flush_block(const MonDev &m, int b, int first, int cnt,
+                                            double2 (*s_ph)[OEM_FLUSH_FG])
+{
+    const int npb = (m.npts + OEM_FLUSH_BLK - 1) / OEM_FLUSH_BLK;
+    const int cg = b / npb, ngrp = (m.nf + OEM_FLUSH_FG - 1) / OEM_FLUSH_FG;
+    const int c = cg / ngrp, f0 = (cg - c * ngrp) * OEM_FLUSH_FG;
+    const int q = (b - cg * npb) * OEM_FLUSH_BLK + (int)threadIdx.x;
+    const int nfl = min(OEM_FLUSH_FG, m.nf - f0);
+    const int g = nfl > 4 ? 8 : nfl > 2 ? 4 : nfl;
+    const int po = c < m.ncomp / 2 ? 0 : 2;        // E: whole-step phase, H: half-step phase
+    for (int t = threadIdx.x; t < cnt * g; t += OEM_FLUSH_BLK) {
+        const int s = t / g, u = t - s * g;
+        const double *p = m.phase + ((size_t)(first + s) * m.nf + f0 + u) * 4 + po;
+        s_ph[s][u] = u < nfl ? make_double2(p[0], p[1]) : make_double2(0.0, 0.0);
+    }
+    __syncthreads();
+    if (q < m.npts) {
+        if (g == 8) flush_sums<F, 8>(m, c, f0, nfl, q, first, cnt, s_ph);
+        else if (g == 4) flush_sums<F, 4>(m, c, f0, nfl, q, first, cnt, s_ph);
+        else if (g == 2) flush_sums<F, 2>(m, c, f0, nfl, q, first, cnt, s_ph);
+        else flush_sums<F, 1>(m, c, f0, nfl, q, first, cnt, s_ph);
+    }
+}
+__host__ __device__ __forceinline__ int flush_blocks(const MonDev &m) {
+    return (m.npts + OEM_FLUSH_BLK - 1) / OEM_FLUSH_BLK * m.ncomp *
+           ((m.nf + OEM_FLUSH_FG - 1) / OEM_FLUSH_FG);
+}
+
+// The monitors of a scene (up to OEM_FLUSH_MONS a launch) replayed together: ofs[t] is the first
+// block of monitor t.  Launched after the step counter advanced past the last snapshot: the cnt
+// snapshots ending at step *stp - 1 are replayed.
+#define OEM_FLUSH_MONS 8
+struct FlushDev {
+    int n, ofs[OEM_FLUSH_MONS];
+    MonDev m[OEM_FLUSH_MONS];
+};
+template <typename F>
+__global__ void __launch_bounds__(OEM_FLUSH_BLK)
+k_dft_flush(FlushDev d, int cnt, const int *__restrict__ stp)
+{
+    __shared__ double2 s_ph[64][OEM_FLUSH_FG];
+    int t = 0;
+    while (t + 1 < d.n && (int)blockIdx.x >= d.ofs[t + 1]) ++t;
+    flush_block<F>(d.m[t], (int)blockIdx.x - d.ofs[t], step_now(stp) - cnt, cnt, s_ph);
 }

@@ -70,7 +70,7 @@ struct PoolDev {
     int disp_ofs[OEM_POOL_MAX + 1];
     int pt_ofs[OEM_POOL_SLOTS][OEM_POOL_MAX + 1];
     int snap_ofs[OEM_POOL_MAX_MON + 1];
-    int flush_ofs[OEM_POOL_MAX_MON + 1];
+    int flush_ofs[OEM_POOL_MAX_MON + 1];      // blocks
     SceneDev sc[OEM_POOL_MAX];
     PtSeg pt[OEM_POOL_SLOTS][OEM_POOL_MAX];
     MonSeg mon[OEM_POOL_MAX_MON];
@@ -202,23 +202,21 @@ k_pool_snap(const PoolDev *__restrict__ P)
 }
 
 // After the block: replay each scene's snapshots since its last flush.
-__global__ void __launch_bounds__(OEM_POOL_BLK)
+__global__ void __launch_bounds__(OEM_FLUSH_BLK)
 k_pool_flush(const PoolDev *__restrict__ P)
 {
+    __shared__ double2 s_ph[64][OEM_FLUSH_FG];
     const int nm = P->n_mon;
     if (nm == 0) return;
     const int tot = P->flush_ofs[nm];
-    OEM_POOL_CHUNKS(tot) {
-        const int g = find_seg(P->flush_ofs, nm, base);
+    for (int b = blockIdx.x; b < tot; b += gridDim.x) {
+        const int g = find_seg(P->flush_ofs, nm, b);
         const MonSeg &M = P->mon[g];
         const SceneDev &S = P->sc[M.scene];
         const int now = S.stp[0], from = S.stp[1];
-        if (now <= from) continue;
-        const int r = base - P->flush_ofs[g] + (int)threadIdx.x;
-        if (r >= M.d.npts * M.d.nf) continue;
-        const int f = r / M.d.npts, q = r - f * M.d.npts;
-        if (M.d.ncomp == 4) flush_point<float, 4>(M.d, from, now - 1, f, q);
-        else flush_point<float, 6>(M.d, from, now - 1, f, q);
+        if (now <= from) continue;                    // uniform over the block
+        flush_block<float>(M.d, b - P->flush_ofs[g], from, now - from, s_ph);
+        __syncthreads();                              // every thread is done with the phases
     }
 }
 
@@ -402,7 +400,7 @@ int build_desc(oem_pool *pool, PoolDev *h) {
             h->snap_ofs[nm] = snap;
             h->flush_ofs[nm] = flush;
             snap += pad_blk(m.d.npts);
-            flush += pad_blk(m.d.npts * m.d.nf);
+            flush += flush_blocks(m.d);
             ++nm;
         }
         ++ns;

@@ -968,10 +968,17 @@ inline int blocks_for(int n, int bs) { return (n + bs - 1) / bs; }
 
 template <typename F>
 int launch_flush_t(oem_ctx *c, int cnt) {
-    for (auto &m : c->mons) {
-        const int ngrp = (m.d.nf + OEM_FLUSH_FG - 1) / OEM_FLUSH_FG;
-        const dim3 grid(blocks_for(m.d.npts, 256), m.d.ncomp * ngrp);
-        hipLaunchKernelGGL((k_dft_flush<F>), grid, dim3(256), 0, c->stream, m.d, cnt, c->d_step);
+    for (size_t t = 0; t < c->mons.size(); t += OEM_FLUSH_MONS) {
+        FlushDev d{};
+        int64_t nb = 0;
+        d.n = (int)std::min<size_t>(OEM_FLUSH_MONS, c->mons.size() - t);
+        for (int q = 0; q < d.n; ++q) {
+            d.m[q] = c->mons[t + q].d;
+            d.ofs[q] = (int)nb;
+            nb += flush_blocks(d.m[q]);
+        }
+        hipLaunchKernelGGL((k_dft_flush<F>), dim3((unsigned)nb), dim3(OEM_FLUSH_BLK), 0, c->stream,
+                           d, cnt, c->d_step);
     }
     HIP_OK(hipGetLastError());
     return OEM_OK;
