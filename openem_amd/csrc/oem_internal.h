@@ -60,7 +60,7 @@ struct Points {
     PointsDev d;
     int magnetic;       // 1: applied to H after update_h; 0: to E after update_e
     int kind;           // PT_*: launch order H: dipole, TF/SF, mode; E: TF/SF, mode, dipole
-    std::vector<int> cells;   // the group cells (host copy)
+    std::vector<int> cells, comps;   // the group cells and components (host copies)
 };
 
 // Kernel family of a point list (profiling ids of include/openem_hip.h).
@@ -146,6 +146,7 @@ struct oem_ctx {
     GridDev fg{};               // launch geometry of the fused H+E step
     bool fuse_plain = false;    // its stores keep their lines in the caches (march_bytes)
     FuseSnap fsnap{};           // the DFT monitors the fused step snaps
+    FusePts fpts{};             // the E-side points it applies (n = 0: none)
     bool fsnap_multi = false;   // some work-group meets more than one of them
     bool axis_set[3] = {false, false, false};
     MatDev mat{};

@@ -185,7 +185,13 @@ __device__ __forceinline__ int slab_of(int i, int n, int lo, int hi) {
     return i < lo ? i : (i >= n - hi ? i - (n - hi) + lo : -1);
 }
 
-__device__ __forceinline__ int step_now(const int *stp) { return *stp; }
+// The step a kernel takes: a device counter plus an offset fixed at the launch.  A captured block
+// of steps counts them by the offset and moves the counter once, at its end.
+struct StepRef {
+    const int *p;
+    int off;
+};
+__device__ __forceinline__ int step_now(StepRef r) { return *r.p + r.off; }
 
 // Next index along an axis: interior neighbours are i + 1 (the host checks), only the last
 // cell's neighbour comes from the table (`last` = A.nxt[n - 1], loaded once and marked
@@ -237,7 +243,7 @@ __device__ __forceinline__ F stretch_v(F &psi, F d, float a, float b, float invk
 template <typename F>
 __device__ __forceinline__ void update_h_tile(F *__restrict__ H, const F *__restrict__ E,
                                               const PsiDev &ps, const GridDev &g, float ch,
-                                              const PlaneSrcDev &pw, const int *__restrict__ stp,
+                                              const PlaneSrcDev &pw, StepRef stp,
                                               const TileCoord &tc)
 {
     typedef FT<F> T;
@@ -343,7 +349,7 @@ __device__ __forceinline__ void update_h_tile(F *__restrict__ H, const F *__rest
 template <typename F>
 __global__ void __launch_bounds__(OEM_TK * OEM_TJ)
 k_update_h(F *__restrict__ H, const F *__restrict__ E, PsiDev ps, GridDev g, float ch,
-           PlaneSrcDev pw, const int *__restrict__ stp)
+           PlaneSrcDev pw, StepRef stp)
 {
     const TileCoord tc = tile_coord(g, xcd_remap(blockIdx.x, g.nblocks));
     if (!tc.ok) return;
@@ -375,7 +381,7 @@ template <typename F>
 __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__restrict__ H,
                                               const PsiDev &ps, const GridDev &g,
                                               const MatDev &mat, float cw, const PlaneSrcDev &pw,
-                                              const int *__restrict__ stp, const TileCoord &tc,
+                                              StepRef stp, const TileCoord &tc,
                                               const float4 *s_lut, bool lds_lut)
 {
     typedef FT<F> T;
@@ -524,7 +530,7 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
 template <typename F>
 __global__ void __launch_bounds__(OEM_TK * OEM_TJ)
 k_update_e(F *__restrict__ E, const F *__restrict__ H, PsiDev ps, GridDev g, MatDev mat,
-           float cw, PlaneSrcDev pw, const int *__restrict__ stp)
+           float cw, PlaneSrcDev pw, StepRef stp)
 {
     __shared__ float4 s_lut[2 * OEM_LDS_CLASSES];
     const bool lds_lut = lut_in_lds(mat);
@@ -538,7 +544,7 @@ k_update_e(F *__restrict__ E, const F *__restrict__ H, PsiDev ps, GridDev g, Mat
 }
 
 // Plane-wave H-side correction at cell k (the injection term of update_h).
-__device__ __forceinline__ void pw_h_inj(const PlaneSrcDev &pw, int k, const int *stp,
+__device__ __forceinline__ void pw_h_inj(const PlaneSrcDev &pw, int k, StepRef stp,
                                          float &inj_hx, float &inj_hy) {
     inj_hx = 0.f;
     inj_hy = 0.f;
@@ -550,6 +556,85 @@ __device__ __forceinline__ void pw_h_inj(const PlaneSrcDev &pw, int k, const int
             if (pw.pol[s] == 0) inj_hy += v; else inj_hx += v;
         }
 }
+
+// ------------------------------------------------------------------------------------------
+// Grouped point corrections: one thread per distinct (component, cell), its points applied in
+// input order (no atomics, deterministic).  Used for
+//   * point dipoles (reference inject_dipole / inject_dipole_h,
+//     `openem/kernels/source_dft.cu:147-206`, which use atomicAdd):
+//     F -= scale * coef * amp[src][n]
+//   * TF/SF box face corrections (reference tfsf_corr_e / tfsf_corr_h,
+//     `openem/kernels/tfsf.cu:49-83`):  F += scale * coef * (table[n][col] * phase)
+// scale is ch on the H side and the cell's cb on the E side.
+// ------------------------------------------------------------------------------------------
+struct PointsDev {
+    int n_groups, nsteps1, ncol;
+    int e_side;                             // 1: scale by the cell's cb; 0: by ch
+    int tfsf;                               // 0: dipole amplitudes, 1: TF/SF table lookups
+    int cplx_amp;                           // dipole amplitude entries are complex doubles
+    const int *g_comp, *g_cell, *g_ofs;     // per group; ofs (n_groups+1) into the points
+    const float *coef;                      // per point
+    const int *col;                         // per point: source (dipole) or table column
+    const float *phase;                     // per point (re, im) for TF/SF, or nullptr
+    const double *tab;                      // dipole: n_src*nsteps1 (x2 if complex);
+                                            // TF/SF: nsteps1*ncol complex (re, im)
+};
+
+// A value of group t's cell with the group's points added (scale: ch or the cell's cb).
+template <typename F>
+__device__ __forceinline__ F point_terms(F v, const PointsDev &d, float scale, int n, int t)
+{
+    typedef FT<F> T;
+    if (n >= d.nsteps1) return v;
+    for (int q = d.g_ofs[t]; q < d.g_ofs[t + 1]; ++q) {
+        float ar, ai;
+        if (d.tfsf) {
+            const double *e = d.tab + 2 * ((size_t)n * d.ncol + d.col[q]);
+            const double pr = d.phase[2 * q], pi = d.phase[2 * q + 1];
+            ar = (float)(e[0] * pr - e[1] * pi);
+            ai = (float)(e[0] * pi + e[1] * pr);
+        } else if (d.cplx_amp) {
+            const double *e = d.tab + 2 * ((size_t)d.col[q] * d.nsteps1 + n);
+            ar = -(float)e[0];
+            ai = -(float)e[1];
+        } else {
+            ar = -(float)d.tab[(size_t)d.col[q] * d.nsteps1 + n];
+            ai = 0.f;
+        }
+        v = T::addc(v, scale * d.coef[q], ar, ai);
+    }
+    return v;
+}
+
+// Group t of a point list at step n.
+template <typename F>
+__device__ __forceinline__ void point_group(F *__restrict__ Fld, const PointsDev &d,
+                                            const MatDev &mat, float ch, size_t ncell, int n,
+                                            int t)
+{
+    const int c = d.g_comp[t], id = d.g_cell[t];
+    F *Fp = Fld + (size_t)c * ncell;
+    float scale;
+    if (!d.e_side) {
+        scale = ch;
+    } else if (mat.mode == 0) {
+        scale = mat.lut[8 * (size_t)mat.cls[id] + 2 * c + 1];
+    } else {
+        scale = mat.cb[(size_t)c * ncell + id];
+    }
+    Fp[id] = point_terms<F>(Fp[id], d, scale, n, t);
+}
+
+// The few E-side point groups (a dipole's stencil) that the fused step applies as it stores E, in
+// list order: group g[t] of list[lst[t]] corrects component c[t] of cell (i[t], j[t], k[t]).
+#define OEM_FUSE_PTS 8
+#define OEM_FUSE_LISTS 2
+struct FusePts {
+    int n;
+    int c[OEM_FUSE_PTS], i[OEM_FUSE_PTS], j[OEM_FUSE_PTS], k[OEM_FUSE_PTS];
+    int g[OEM_FUSE_PTS], lst[OEM_FUSE_PTS];
+    PointsDev list[OEM_FUSE_LISTS];
+};
 
 // ------------------------------------------------------------------------------------------
 // Fused H + E step.  A work-group owns a tile of OEM_CR rows (j) x 64 cells (k) (or 2 OEM_CR x 32
@@ -619,7 +704,7 @@ struct HColumn {
 
 template <typename F>
 __device__ __forceinline__ void hcolumn_init(HColumn<F> &c, const GridDev &g,
-                                             const PlaneSrcDev &pw, const int *stp, int j, int k,
+                                             const PlaneSrcDev &pw, StepRef stp, int j, int k,
                                              int jn, int kn, int ly, int lz) {
     typedef FT<F> T;
     const AxisDev &Y = g.ax[1], &Z = g.ax[2];
@@ -896,7 +981,7 @@ template <typename F, int MK, bool MULTI, int AUX>
 __global__ void __launch_bounds__(64 * (OEM_CR + 1))
 k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ En,
                 F *__restrict__ Hn, PsiDev ps, PsiDev pn, GridDev g, MatDev mat, float ch,
-                float cw, PlaneSrcDev pw, const int *__restrict__ stp, FuseSnap fs)
+                float cw, PlaneSrcDev pw, StepRef stp, FuseSnap fs, FusePts fpt)
 {
     typedef FT<F> T;
     // Ho = Eo + 3 components (the host allocates them so)
@@ -1083,6 +1168,12 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
                 if (pw.pol[s] == 0) { inj_ex += v; inj_x = true; } else { inj_ey += v; inj_y = true; }
             }
     }
+    // the point groups in this tile and chunk (most have none)
+    uint32_t pmask = 0;
+    for (int t = 0; t < fpt.n; ++t)
+        if (fpt.i[t] >= i0 && fpt.i[t] < i1 && fpt.j[t] >= j0 && fpt.j[t] < j0 + nr &&
+            fpt.k[t] >= k0 && fpt.k[t] < k0 + kw)
+            pmask |= 1u << t;
     const rsrc_t rC = mk_rsrc(mat.cls, (uint32_t)(ncell * 2));
     const int hbx = mat.hb[1] - mat.hb[0], hby = mat.hb[3] - mat.hb[2], hbz = mat.hb[5] - mat.hb[4];
     const uint32_t hcomp = (uint32_t)(hbx * hby * hbz);
@@ -1206,6 +1297,17 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         F nez = (caz * ez0 + cbz * (s_ez_x - s_ez_y - cw * hpz)) * pecx * pecy;
         if (inj_x) nex = T::addre(nex, cbx * inj_ex);
         if (inj_y) ney = T::addre(ney, cby * inj_ey);
+        if (pmask) {
+            for (uint32_t m = pmask; m; m &= m - 1u) {
+                const int t = __builtin_ctz(m);
+                if (fpt.i[t] != i || fpt.j[t] != j || fpt.k[t] != k || !own) continue;
+                const PointsDev &pd = fpt.list[fpt.lst[t]];
+                const int n = step_now(stp), gt = fpt.g[t];
+                if (fpt.c[t] == 0) nex = point_terms<F>(nex, pd, cbx, n, gt);
+                else if (fpt.c[t] == 1) ney = point_terms<F>(ney, pd, cby, n, gt);
+                else nez = point_terms<F>(nez, pd, cbz, n, gt);
+            }
+        }
         if (own) {
             T::template st<AUX>(io.fn, nex, ca.op, so);
             T::template st<AUX>(io.fn, ney, ca.op, so + io.cb);
@@ -1235,7 +1337,7 @@ template <typename F>
 __global__ void __launch_bounds__(256)
 k_rec_gather(const F *__restrict__ E, const int *__restrict__ comp,
              const int *__restrict__ cell, int n, size_t ncell, F *__restrict__ rec,
-             const int *__restrict__ stp, int64_t base)
+             StepRef stp, int64_t base)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= n) return;
@@ -1243,72 +1345,10 @@ k_rec_gather(const F *__restrict__ E, const int *__restrict__ comp,
     rec[(size_t)row * n + q] = E[(size_t)comp[q] * ncell + cell[q]];
 }
 
-// ------------------------------------------------------------------------------------------
-// Grouped point corrections: one thread per distinct (component, cell), its points applied in
-// input order (no atomics, deterministic).  Used for
-//   * point dipoles (reference inject_dipole / inject_dipole_h,
-//     `openem/kernels/source_dft.cu:147-206`, which use atomicAdd):
-//     F -= scale * coef * amp[src][n]
-//   * TF/SF box face corrections (reference tfsf_corr_e / tfsf_corr_h,
-//     `openem/kernels/tfsf.cu:49-83`):  F += scale * coef * (table[n][col] * phase)
-// scale is ch on the H side and the cell's cb on the E side.
-// ------------------------------------------------------------------------------------------
-struct PointsDev {
-    int n_groups, nsteps1, ncol;
-    int e_side;                             // 1: scale by the cell's cb; 0: by ch
-    int tfsf;                               // 0: dipole amplitudes, 1: TF/SF table lookups
-    int cplx_amp;                           // dipole amplitude entries are complex doubles
-    const int *g_comp, *g_cell, *g_ofs;     // per group; ofs (n_groups+1) into the points
-    const float *coef;                      // per point
-    const int *col;                         // per point: source (dipole) or table column
-    const float *phase;                     // per point (re, im) for TF/SF, or nullptr
-    const double *tab;                      // dipole: n_src*nsteps1 (x2 if complex);
-                                            // TF/SF: nsteps1*ncol complex (re, im)
-};
-
-// Group t of a point list at step n.
-template <typename F>
-__device__ __forceinline__ void point_group(F *__restrict__ Fld, const PointsDev &d,
-                                            const MatDev &mat, float ch, size_t ncell, int n,
-                                            int t)
-{
-    typedef FT<F> T;
-    if (n >= d.nsteps1) return;
-    const int c = d.g_comp[t], id = d.g_cell[t];
-    F *Fp = Fld + (size_t)c * ncell;
-    float scale;
-    if (!d.e_side) {
-        scale = ch;
-    } else if (mat.mode == 0) {
-        scale = mat.lut[8 * (size_t)mat.cls[id] + 2 * c + 1];
-    } else {
-        scale = mat.cb[(size_t)c * ncell + id];
-    }
-    F v = Fp[id];
-    for (int q = d.g_ofs[t]; q < d.g_ofs[t + 1]; ++q) {
-        float ar, ai;
-        if (d.tfsf) {
-            const double *e = d.tab + 2 * ((size_t)n * d.ncol + d.col[q]);
-            const double pr = d.phase[2 * q], pi = d.phase[2 * q + 1];
-            ar = (float)(e[0] * pr - e[1] * pi);
-            ai = (float)(e[0] * pi + e[1] * pr);
-        } else if (d.cplx_amp) {
-            const double *e = d.tab + 2 * ((size_t)d.col[q] * d.nsteps1 + n);
-            ar = -(float)e[0];
-            ai = -(float)e[1];
-        } else {
-            ar = -(float)d.tab[(size_t)d.col[q] * d.nsteps1 + n];
-            ai = 0.f;
-        }
-        v = T::addc(v, scale * d.coef[q], ar, ai);
-    }
-    Fp[id] = v;
-}
-
 template <typename F>
 __global__ void __launch_bounds__(256)
 k_points(F *__restrict__ Fld, PointsDev d, MatDev mat, float ch, size_t ncell,
-         const int *__restrict__ stp)
+         StepRef stp)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= d.n_groups) return;
@@ -1486,18 +1526,17 @@ struct TimeMonDev {
     void *buf;
 };
 
+// Cell q of the monitor at the end of step n, one shot.
 template <typename F>
-__global__ void __launch_bounds__(256)
-k_time_sample(TimeMonDev d, const F *__restrict__ E, const F *__restrict__ H, size_t ncell,
-              int ny, int pz, const int *__restrict__ stp, int shot)
+__device__ __forceinline__ void time_sample_cell(const TimeMonDev &d, const F *__restrict__ E,
+                                                 const F *__restrict__ H, size_t ncell, int ny,
+                                                 int pz, int n, int shot, int q)
 {
-    const int m = step_now(stp) + 1 - shot;
+    const int m = n + 1 - shot;
     const int off = m - d.beg;
     if (off < 0 || m >= d.end || off % d.iv) return;
     const int slot = off / d.iv;
     if (slot >= d.slots) return;
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= d.cells) return;
     const int a = q / (d.b[1] * d.b[2]), r = q - a * d.b[1] * d.b[2];
     const int b = r / d.b[2], c = r - b * d.b[2];
     const size_t id = ((size_t)(d.o[0] + a) * ny + (d.o[1] + b)) * pz + (d.o[2] + c);
@@ -1509,6 +1548,18 @@ k_time_sample(TimeMonDev d, const F *__restrict__ E, const F *__restrict__ H, si
         F &o = out[((size_t)t * d.slots + slot) * d.cells + q];
         o = shot ? o + v : v;
     }
+}
+
+template <typename F>
+__global__ void __launch_bounds__(256)
+k_time_sample(TimeMonDev d, const F *__restrict__ E, const F *__restrict__ H, size_t ncell,
+              int ny, int pz, StepRef stp)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= d.cells) return;
+    const int n = step_now(stp);
+    time_sample_cell<F>(d, E, H, ncell, ny, pz, n, 0, q);
+    time_sample_cell<F>(d, E, H, ncell, ny, pz, n, 1, q);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1569,7 +1620,7 @@ __device__ __forceinline__ double ft_block_sum(double v, double *sh) {
 template <typename F>
 __global__ void __launch_bounds__(OEM_FT_BLK)
 k_flux_time_partial(FluxTimeDev d, const F *__restrict__ E, const F *__restrict__ H,
-                    size_t ncell, int ny, int pz, const int *__restrict__ stp)
+                    size_t ncell, int ny, int pz, StepRef stp)
 {
     static_assert(sizeof(F) == 4, "flux-time monitors sample real fields");
     const int n = step_now(stp);
@@ -1626,7 +1677,7 @@ k_flux_time_partial(FluxTimeDev d, const F *__restrict__ E, const F *__restrict_
 
 template <typename F>
 __global__ void __launch_bounds__(OEM_FT_BLK)
-k_flux_time_sum(FluxTimeDev d, const int *__restrict__ stp)
+k_flux_time_sum(FluxTimeDev d, StepRef stp)
 {
     const int n = step_now(stp);
     const int s1 = ft_slot(d, n), s0 = ft_slot(d, n + 1);
@@ -1698,31 +1749,34 @@ __device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict_
 template <typename F>
 __global__ void __launch_bounds__(256)
 k_dft_snap(MonDev m, const F *__restrict__ E, const F *__restrict__ H, size_t ncell, int ny,
-           int pz, const int *__restrict__ stp)
+           int pz, StepRef stp)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= m.npts) return;
     snap_point<F>(m, E, H, ncell, ny, pz, step_now(stp) % m.T, q);
 }
 
-// The end of a step as one single-block launch, where three small launches would otherwise
+// The end of a step as one single-block launch, where several small launches would otherwise
 // close it: the E-side point lists in step order (each list after the one before it), then the
-// monitor points those lists corrected, snapped again, then the step counter.  Used when every
-// list fits the block and nothing else reads the step counter after the E-side points.
+// monitor points those lists corrected, snapped again, then the small time monitors, then the step
+// counter (adv: the steps it moves; 0 inside a captured block).  Used when every list fits the
+// block and nothing else reads the fields after the E-side points.
 #define OEM_TAIL_LISTS 4
 #define OEM_TAIL_THREADS 1024
+#define OEM_TAIL_TMONS 2
 struct TailDev {
-    int n_pts, n_snap;
+    int n_pts, n_snap, n_tm;
     PointsDev pts[OEM_TAIL_LISTS];
     MonDev mon[OEM_TAIL_LISTS];
     const int *qs[OEM_TAIL_LISTS];
     int nq[OEM_TAIL_LISTS];
+    TimeMonDev tm[OEM_TAIL_TMONS];
 };
 
 template <typename F>
 __global__ void __launch_bounds__(OEM_TAIL_THREADS)
 k_step_tail(F *__restrict__ E, const F *__restrict__ H, TailDev t, MatDev mat, float ch,
-            size_t ncell, int ny, int pz, int *__restrict__ stp)
+            size_t ncell, int ny, int pz, StepRef stp, int *__restrict__ counter, int adv)
 {
     const int n = step_now(stp);
     const int tid = threadIdx.x;
@@ -1732,15 +1786,20 @@ k_step_tail(F *__restrict__ E, const F *__restrict__ H, TailDev t, MatDev mat, f
     }
     for (int m = 0; m < t.n_snap; ++m)
         if (tid < t.nq[m]) snap_point<F>(t.mon[m], E, H, ncell, ny, pz, n % t.mon[m].T, t.qs[m][tid]);
+    for (int m = 0; m < t.n_tm; ++m)
+        if (tid < t.tm[m].cells) {
+            time_sample_cell<F>(t.tm[m], E, H, ncell, ny, pz, n, 0, tid);
+            time_sample_cell<F>(t.tm[m], E, H, ncell, ny, pz, n, 1, tid);
+        }
     __syncthreads();
-    if (tid == 0) *stp = n + 1;
+    if (tid == 0 && adv) *counter += adv;
 }
 
 // The points `qs[0..nq)` of a monitor whose other points the fused step snapped.
 template <typename F>
 __global__ void __launch_bounds__(256)
 k_dft_snap_list(MonDev m, const F *__restrict__ E, const F *__restrict__ H, size_t ncell, int ny,
-                int pz, const int *__restrict__ stp, const int *__restrict__ qs, int nq)
+                int pz, StepRef stp, const int *__restrict__ qs, int nq)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nq) return;
@@ -1843,7 +1902,7 @@ struct FlushDev {
 };
 template <typename F>
 __global__ void __launch_bounds__(OEM_FLUSH_BLK)
-k_dft_flush(FlushDev d, int cnt, const int *__restrict__ stp)
+k_dft_flush(FlushDev d, int cnt, StepRef stp)
 {
     __shared__ double2 s_ph[64][OEM_FLUSH_FG];
     int t = 0;

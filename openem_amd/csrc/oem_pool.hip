@@ -108,7 +108,7 @@ k_pool_update_h(const PoolDev *__restrict__ P)
         int n;
         if (!scene_live(S, &n)) continue;
         const TileCoord tc = tile_coord(S.g, lw - P->item_ofs[s]);
-        if (tc.ok) update_h_tile<float>(S.H, S.E, S.ps, S.g, S.ch, S.pw, S.stp, tc);
+        if (tc.ok) update_h_tile<float>(S.H, S.E, S.ps, S.g, S.ch, S.pw, StepRef{S.stp, 0}, tc);
     }
 }
 
@@ -132,7 +132,7 @@ k_pool_update_e(const PoolDev *__restrict__ P)
             staged = s;
         }
         const TileCoord tc = tile_coord(S.g, lw - P->item_ofs[s]);
-        if (tc.ok) update_e_tile<float>(S.E, S.H, S.ps, S.g, S.mat, S.cw, S.pw, S.stp, tc, s_lut, lds);
+        if (tc.ok) update_e_tile<float>(S.E, S.H, S.ps, S.g, S.mat, S.cw, S.pw, StepRef{S.stp, 0}, tc, s_lut, lds);
     }
 }
 
