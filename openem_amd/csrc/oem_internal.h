@@ -146,7 +146,7 @@ struct oem_ctx {
     GridDev fg{};               // launch geometry of the fused H+E step
     bool fuse_plain = false;    // its stores keep their lines in the caches (march_bytes)
     FuseSnap fsnap{};           // the DFT monitors the fused step snaps
-    FusePts fpts{};             // the E-side points it applies (n = 0: none)
+    FusePts fpts{};             // the E-side points the E update applies (n = 0: none)
     bool fsnap_multi = false;   // some work-group meets more than one of them
     bool axis_set[3] = {false, false, false};
     MatDev mat{};
@@ -192,11 +192,12 @@ struct oem_ctx {
         if (graph) (void)hipGraphExecDestroy(graph);
         if (red) oemi::reduce_state_free(red);
         if (adj) oemi::adjoint_state_free(adj);
+        // arena ranges before the capture lock: the pool's lock is never taken under it
+        if (pool)
+            for (void *p : allocs) oemi::pool_arena_free(pool, p);
         std::lock_guard<std::mutex> hold(oemi::device_sync_mutex());
-        for (void *p : allocs) {
-            if (pool) oemi::pool_arena_free(pool, p);
-            else (void)hipFree(p);
-        }
+        if (!pool)
+            for (void *p : allocs) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
     }
 

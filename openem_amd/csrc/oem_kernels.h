@@ -236,6 +236,102 @@ __device__ __forceinline__ F stretch_v(F &psi, F d, float a, float b, float invk
 }
 
 // ------------------------------------------------------------------------------------------
+// Grouped point corrections: one thread per distinct (component, cell), its points applied in
+// input order (no atomics, deterministic).  Used for
+//   * point dipoles (reference inject_dipole / inject_dipole_h,
+//     `openem/kernels/source_dft.cu:147-206`, which use atomicAdd):
+//     F -= scale * coef * amp[src][n]
+//   * TF/SF box face corrections (reference tfsf_corr_e / tfsf_corr_h,
+//     `openem/kernels/tfsf.cu:49-83`):  F += scale * coef * (table[n][col] * phase)
+// scale is ch on the H side and the cell's cb on the E side.
+// ------------------------------------------------------------------------------------------
+struct PointsDev {
+    int n_groups, nsteps1, ncol;
+    int e_side;                             // 1: scale by the cell's cb; 0: by ch
+    int tfsf;                               // 0: dipole amplitudes, 1: TF/SF table lookups
+    int cplx_amp;                           // dipole amplitude entries are complex doubles
+    const int *g_comp, *g_cell, *g_ofs;     // per group; ofs (n_groups+1) into the points
+    const float *coef;                      // per point
+    const int *col;                         // per point: source (dipole) or table column
+    const float *phase;                     // per point (re, im) for TF/SF, or nullptr
+    const double *tab;                      // dipole: n_src*nsteps1 (x2 if complex);
+                                            // TF/SF: nsteps1*ncol complex (re, im)
+};
+
+// A value of group t's cell with the group's points added (scale: ch or the cell's cb).
+template <typename F>
+__device__ __forceinline__ F point_terms(F v, const PointsDev &d, float scale, int n, int t)
+{
+    typedef FT<F> T;
+    if (n >= d.nsteps1) return v;
+    for (int q = d.g_ofs[t]; q < d.g_ofs[t + 1]; ++q) {
+        float ar, ai;
+        if (d.tfsf) {
+            const double *e = d.tab + 2 * ((size_t)n * d.ncol + d.col[q]);
+            const double pr = d.phase[2 * q], pi = d.phase[2 * q + 1];
+            ar = (float)(e[0] * pr - e[1] * pi);
+            ai = (float)(e[0] * pi + e[1] * pr);
+        } else if (d.cplx_amp) {
+            const double *e = d.tab + 2 * ((size_t)d.col[q] * d.nsteps1 + n);
+            ar = -(float)e[0];
+            ai = -(float)e[1];
+        } else {
+            ar = -(float)d.tab[(size_t)d.col[q] * d.nsteps1 + n];
+            ai = 0.f;
+        }
+        v = T::addc(v, scale * d.coef[q], ar, ai);
+    }
+    return v;
+}
+
+// Group t of a point list at step n.
+template <typename F>
+__device__ __forceinline__ void point_group(F *__restrict__ Fld, const PointsDev &d,
+                                            const MatDev &mat, float ch, size_t ncell, int n,
+                                            int t)
+{
+    const int c = d.g_comp[t], id = d.g_cell[t];
+    F *Fp = Fld + (size_t)c * ncell;
+    float scale;
+    if (!d.e_side) {
+        scale = ch;
+    } else if (mat.mode == 0) {
+        scale = mat.lut[8 * (size_t)mat.cls[id] + 2 * c + 1];
+    } else {
+        scale = mat.cb[(size_t)c * ncell + id];
+    }
+    Fp[id] = point_terms<F>(Fp[id], d, scale, n, t);
+}
+
+// The few E-side point groups (a dipole's stencil) that the E update applies as it stores E, in
+// list order: group g[t] of list[lst[t]] corrects component c[t] of cell (i[t], j[t], k[t]).
+#define OEM_FUSE_PTS 8
+#define OEM_FUSE_LISTS 2
+struct FusePts {
+    int n;
+    int c[OEM_FUSE_PTS], i[OEM_FUSE_PTS], j[OEM_FUSE_PTS], k[OEM_FUSE_PTS];
+    int g[OEM_FUSE_PTS], lst[OEM_FUSE_PTS];
+    PointsDev list[OEM_FUSE_LISTS];
+};
+
+// Add the groups of `mask` that lie at plane i of the thread's column to its new E.
+template <typename F>
+__device__ __forceinline__ void fold_points(const FusePts &fpt, uint32_t mask, int i, int j, int k,
+                                            int n, float cbx, float cby, float cbz, F &ex, F &ey,
+                                            F &ez)
+{
+    for (; mask; mask &= mask - 1u) {
+        const int t = __builtin_ctz(mask);
+        if (fpt.i[t] != i || fpt.j[t] != j || fpt.k[t] != k) continue;
+        const PointsDev &pd = fpt.list[fpt.lst[t]];
+        const int gt = fpt.g[t];
+        if (fpt.c[t] == 0) ex = point_terms<F>(ex, pd, cbx, n, gt);
+        else if (fpt.c[t] == 1) ey = point_terms<F>(ey, pd, cby, n, gt);
+        else ez = point_terms<F>(ez, pd, cbz, n, gt);
+    }
+}
+
+// ------------------------------------------------------------------------------------------
 // H half step (reference update_h, `openem/kernels/yee.cu:76-137`; complex variant
 // update_h_c, `openem/kernels/bloch.cu:38-126`) fused with the H side of the plane-wave TF/SF
 // correction (`openem/kernels/source_dft.cu:40-55`).
@@ -377,12 +473,15 @@ __device__ __forceinline__ void stage_lut(float4 *s_lut, const MatDev &mat) {
     for (int q = tid; q < 2 * mat.n_classes; q += OEM_TK * OEM_TJ) s_lut[q] = src[q];
 }
 
-template <typename F>
+// PTS: some E-side point groups are applied here (without, the complex sweep holds 78 registers,
+// three blocks a CU, with 81 and two).
+template <typename F, bool PTS>
 __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__restrict__ H,
                                               const PsiDev &ps, const GridDev &g,
                                               const MatDev &mat, float cw, const PlaneSrcDev &pw,
-                                              StepRef stp, const TileCoord &tc,
-                                              const float4 *s_lut, bool lds_lut)
+                                              const FusePts &fpt, StepRef stp,
+                                              const TileCoord &tc, const float4 *s_lut,
+                                              bool lds_lut)
 {
     typedef FT<F> T;
     const int j = tc.j, k = tc.k;
@@ -435,6 +534,11 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
     const uint32_t oc = (uint32_t)(j * pz + k) * 2u;               // uint16 class index
 
     const uint32_t planeB = (uint32_t)g.plane * T::B, plane2 = (uint32_t)g.plane * 2u;
+    // the point groups in this wave's columns and planes (most waves have none)
+    uint32_t pmask = 0;
+    for (int t = 0; PTS && t < fpt.n; ++t)
+        if (fpt.i[t] >= tc.i0 && fpt.i[t] < tc.i1 && __ballot(fpt.j[t] == j && fpt.k[t] == k))
+            pmask |= 1u << t;
     const uint32_t sp0 = (uint32_t)__builtin_amdgcn_readfirstlane(X.prv[tc.i0]) * planeB;
     F hy_m = T::ld(rHy, op, sp0), hz_m = T::ld(rHz, op, sp0);
     uint32_t cls_next = mat.mode == 0 ? bld_u16(rC, oc, (uint32_t)tc.i0 * plane2) : 0u;
@@ -519,6 +623,8 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
         ez = (caz * ez + cbz * (s_ez_x - s_ez_y - cw * phz)) * pecx * pecy;
         if (inj_x) ex = T::addre(ex, cbx * inj_ex);
         if (inj_y) ey = T::addre(ey, cby * inj_ey);
+        if (PTS && pmask)
+            fold_points<F>(fpt, pmask, i, j, k, step_now(stp), cbx, cby, cbz, ex, ey, ez);
         T::st(rEx, ex, op, so);
         T::st(rEy, ey, op, so);
         T::st(rEz, ez, op, so);
@@ -527,10 +633,10 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
     }
 }
 
-template <typename F>
+template <typename F, bool PTS>
 __global__ void __launch_bounds__(OEM_TK * OEM_TJ)
 k_update_e(F *__restrict__ E, const F *__restrict__ H, PsiDev ps, GridDev g, MatDev mat,
-           float cw, PlaneSrcDev pw, StepRef stp)
+           float cw, PlaneSrcDev pw, FusePts fpt, StepRef stp)
 {
     __shared__ float4 s_lut[2 * OEM_LDS_CLASSES];
     const bool lds_lut = lut_in_lds(mat);
@@ -540,7 +646,7 @@ k_update_e(F *__restrict__ E, const F *__restrict__ H, PsiDev ps, GridDev g, Mat
     }
     const TileCoord tc = tile_coord(g, xcd_remap(blockIdx.x, g.nblocks));
     if (!tc.ok) return;
-    update_e_tile<F>(E, H, ps, g, mat, cw, pw, stp, tc, s_lut, lds_lut);
+    update_e_tile<F, PTS>(E, H, ps, g, mat, cw, pw, fpt, stp, tc, s_lut, lds_lut);
 }
 
 // Plane-wave H-side correction at cell k (the injection term of update_h).
@@ -556,85 +662,6 @@ __device__ __forceinline__ void pw_h_inj(const PlaneSrcDev &pw, int k, StepRef s
             if (pw.pol[s] == 0) inj_hy += v; else inj_hx += v;
         }
 }
-
-// ------------------------------------------------------------------------------------------
-// Grouped point corrections: one thread per distinct (component, cell), its points applied in
-// input order (no atomics, deterministic).  Used for
-//   * point dipoles (reference inject_dipole / inject_dipole_h,
-//     `openem/kernels/source_dft.cu:147-206`, which use atomicAdd):
-//     F -= scale * coef * amp[src][n]
-//   * TF/SF box face corrections (reference tfsf_corr_e / tfsf_corr_h,
-//     `openem/kernels/tfsf.cu:49-83`):  F += scale * coef * (table[n][col] * phase)
-// scale is ch on the H side and the cell's cb on the E side.
-// ------------------------------------------------------------------------------------------
-struct PointsDev {
-    int n_groups, nsteps1, ncol;
-    int e_side;                             // 1: scale by the cell's cb; 0: by ch
-    int tfsf;                               // 0: dipole amplitudes, 1: TF/SF table lookups
-    int cplx_amp;                           // dipole amplitude entries are complex doubles
-    const int *g_comp, *g_cell, *g_ofs;     // per group; ofs (n_groups+1) into the points
-    const float *coef;                      // per point
-    const int *col;                         // per point: source (dipole) or table column
-    const float *phase;                     // per point (re, im) for TF/SF, or nullptr
-    const double *tab;                      // dipole: n_src*nsteps1 (x2 if complex);
-                                            // TF/SF: nsteps1*ncol complex (re, im)
-};
-
-// A value of group t's cell with the group's points added (scale: ch or the cell's cb).
-template <typename F>
-__device__ __forceinline__ F point_terms(F v, const PointsDev &d, float scale, int n, int t)
-{
-    typedef FT<F> T;
-    if (n >= d.nsteps1) return v;
-    for (int q = d.g_ofs[t]; q < d.g_ofs[t + 1]; ++q) {
-        float ar, ai;
-        if (d.tfsf) {
-            const double *e = d.tab + 2 * ((size_t)n * d.ncol + d.col[q]);
-            const double pr = d.phase[2 * q], pi = d.phase[2 * q + 1];
-            ar = (float)(e[0] * pr - e[1] * pi);
-            ai = (float)(e[0] * pi + e[1] * pr);
-        } else if (d.cplx_amp) {
-            const double *e = d.tab + 2 * ((size_t)d.col[q] * d.nsteps1 + n);
-            ar = -(float)e[0];
-            ai = -(float)e[1];
-        } else {
-            ar = -(float)d.tab[(size_t)d.col[q] * d.nsteps1 + n];
-            ai = 0.f;
-        }
-        v = T::addc(v, scale * d.coef[q], ar, ai);
-    }
-    return v;
-}
-
-// Group t of a point list at step n.
-template <typename F>
-__device__ __forceinline__ void point_group(F *__restrict__ Fld, const PointsDev &d,
-                                            const MatDev &mat, float ch, size_t ncell, int n,
-                                            int t)
-{
-    const int c = d.g_comp[t], id = d.g_cell[t];
-    F *Fp = Fld + (size_t)c * ncell;
-    float scale;
-    if (!d.e_side) {
-        scale = ch;
-    } else if (mat.mode == 0) {
-        scale = mat.lut[8 * (size_t)mat.cls[id] + 2 * c + 1];
-    } else {
-        scale = mat.cb[(size_t)c * ncell + id];
-    }
-    Fp[id] = point_terms<F>(Fp[id], d, scale, n, t);
-}
-
-// The few E-side point groups (a dipole's stencil) that the fused step applies as it stores E, in
-// list order: group g[t] of list[lst[t]] corrects component c[t] of cell (i[t], j[t], k[t]).
-#define OEM_FUSE_PTS 8
-#define OEM_FUSE_LISTS 2
-struct FusePts {
-    int n;
-    int c[OEM_FUSE_PTS], i[OEM_FUSE_PTS], j[OEM_FUSE_PTS], k[OEM_FUSE_PTS];
-    int g[OEM_FUSE_PTS], lst[OEM_FUSE_PTS];
-    PointsDev list[OEM_FUSE_LISTS];
-};
 
 // ------------------------------------------------------------------------------------------
 // Fused H + E step.  A work-group owns a tile of OEM_CR rows (j) x 64 cells (k) (or 2 OEM_CR x 32
@@ -1297,17 +1324,8 @@ k_update_he(const F *__restrict__ Eo, const F *__restrict__ Ho, F *__restrict__ 
         F nez = (caz * ez0 + cbz * (s_ez_x - s_ez_y - cw * hpz)) * pecx * pecy;
         if (inj_x) nex = T::addre(nex, cbx * inj_ex);
         if (inj_y) ney = T::addre(ney, cby * inj_ey);
-        if (pmask) {
-            for (uint32_t m = pmask; m; m &= m - 1u) {
-                const int t = __builtin_ctz(m);
-                if (fpt.i[t] != i || fpt.j[t] != j || fpt.k[t] != k || !own) continue;
-                const PointsDev &pd = fpt.list[fpt.lst[t]];
-                const int n = step_now(stp), gt = fpt.g[t];
-                if (fpt.c[t] == 0) nex = point_terms<F>(nex, pd, cbx, n, gt);
-                else if (fpt.c[t] == 1) ney = point_terms<F>(ney, pd, cby, n, gt);
-                else nez = point_terms<F>(nez, pd, cbz, n, gt);
-            }
-        }
+        if (pmask && own)
+            fold_points<F>(fpt, pmask, i, j, k, step_now(stp), cbx, cby, cbz, nex, ney, nez);
         if (own) {
             T::template st<AUX>(io.fn, nex, ca.op, so);
             T::template st<AUX>(io.fn, ney, ca.op, so + io.cb);
@@ -1746,12 +1764,22 @@ __device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict_
     }
 }
 
+// The snapshots of several monitors (up to OEM_SNAP_MONS) in one launch: ofs[t] is monitor t's
+// first block.  A launch per monitor cost 4.65 us each at 160^3, as long as its points took.
+#define OEM_SNAP_MONS 8
+struct SnapDev {
+    int n, ofs[OEM_SNAP_MONS];
+    MonDev m[OEM_SNAP_MONS];
+};
 template <typename F>
 __global__ void __launch_bounds__(256)
-k_dft_snap(MonDev m, const F *__restrict__ E, const F *__restrict__ H, size_t ncell, int ny,
+k_dft_snap(SnapDev d, const F *__restrict__ E, const F *__restrict__ H, size_t ncell, int ny,
            int pz, StepRef stp)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    int t = 0;
+    while (t + 1 < d.n && (int)blockIdx.x >= d.ofs[t + 1]) ++t;
+    const MonDev &m = d.m[t];
+    const int q = ((int)blockIdx.x - d.ofs[t]) * (int)blockDim.x + (int)threadIdx.x;
     if (q >= m.npts) return;
     snap_point<F>(m, E, H, ncell, ny, pz, step_now(stp) % m.T, q);
 }

@@ -4,14 +4,16 @@
 // first-fit sub-allocation, so admitting and retiring scenes never calls hipMalloc/hipFree
 // (hipFree synchronises the device) and the arena size is the admission budget.
 //
-// Launches.  A pool block is dft_batch steps captured once into a hipGraph.  Its kernels read a
+// Launches.  A pool block is dft_batch steps captured into a hipGraph.  Its kernels read a
 // descriptor table (PoolDev) from device memory: the scenes, the concatenated tile list of
 // their sweeps, and per kind the concatenated point groups, ADE entries and monitor points.
-// The sweep kernels walk the whole tile list with a fixed, over-sized grid (the graph is
-// captured once) and every kernel finds its scene by binary search over prefix offsets.  Each scene keeps its
-// own device step counter: kernels skip scenes that reached their n_steps, so a scene finishing
-// mid-block costs nothing further.  Changing the membership rewrites the descriptor table with
-// a stream-ordered copy between blocks; the graph itself never changes.
+// The sweep kernels walk the whole tile list with a fixed, over-sized grid and every kernel finds
+// its scene by binary search over prefix offsets.  A graph is captured for each combination of
+// launches that the running scenes need (desc_key) and kept.  Each scene keeps its own device
+// step counter, which stands still over a block (a step of the block is the counter plus the
+// step's number) and moves at its end: kernels skip scenes that reached their n_steps, so a scene
+// finishing mid-block costs nothing further.  Changing the membership rewrites the descriptor
+// table with a stream-ordered copy between blocks.
 //
 // Scenes are admitted at block boundaries at step 0, so their step counters stay multiples of
 // dft_batch at every boundary and the end-of-block flush replays exactly the steps since the
@@ -45,9 +47,10 @@ struct SceneDev {
     GridDev g;
     MatDev mat;
     PlaneSrcDev pw;
+    FusePts fpts;
     DispDev disp;
     float ch, cw;
-    int *stp;           // [0] steps taken, [1] steps flushed
+    int *stp;           // steps taken up to the block
     int n_total;
     int ny, pz;
     size_t ncell;       // cells of a component, row padding included
@@ -90,15 +93,16 @@ __device__ __forceinline__ int find_seg(const int *ofs, int n, int x) {
     return lo;
 }
 
-__device__ __forceinline__ bool scene_live(const SceneDev &S, int *n) {
-    *n = S.stp[0];
+// Step `s` of a block: the scene's counter stands at the block's first step until its end.
+__device__ __forceinline__ bool scene_live(const SceneDev &S, int s, int *n) {
+    *n = S.stp[0] + s;
     return *n < S.n_total;
 }
 
 // The grid is a multiple of the XCD count and blocks are dispatched round-robin over the XCDs,
 // so block b runs on XCD b % 8 and the remap hands each XCD a contiguous run of the tile list.
 __global__ void __launch_bounds__(OEM_TK * OEM_TJ)
-k_pool_update_h(const PoolDev *__restrict__ P)
+k_pool_update_h(const PoolDev *__restrict__ P, int step)
 {
     const int nit = P->n_items, ns = P->n_scenes;
     for (int w = blockIdx.x; w < nit; w += gridDim.x) {
@@ -106,14 +110,14 @@ k_pool_update_h(const PoolDev *__restrict__ P)
         const int s = find_seg(P->item_ofs, ns, lw);
         const SceneDev &S = P->sc[s];
         int n;
-        if (!scene_live(S, &n)) continue;
+        if (!scene_live(S, step, &n)) continue;
         const TileCoord tc = tile_coord(S.g, lw - P->item_ofs[s]);
-        if (tc.ok) update_h_tile<float>(S.H, S.E, S.ps, S.g, S.ch, S.pw, StepRef{S.stp, 0}, tc);
+        if (tc.ok) update_h_tile<float>(S.H, S.E, S.ps, S.g, S.ch, S.pw, StepRef{S.stp, step}, tc);
     }
 }
 
 __global__ void __launch_bounds__(OEM_TK * OEM_TJ)
-k_pool_update_e(const PoolDev *__restrict__ P)
+k_pool_update_e(const PoolDev *__restrict__ P, int step)
 {
     __shared__ float4 s_lut[2 * OEM_LDS_CLASSES];
     const int nit = P->n_items, ns = P->n_scenes;
@@ -123,7 +127,7 @@ k_pool_update_e(const PoolDev *__restrict__ P)
         const int s = find_seg(P->item_ofs, ns, lw);
         const SceneDev &S = P->sc[s];
         int n;
-        if (!scene_live(S, &n)) continue;             // uniform over the block
+        if (!scene_live(S, step, &n)) continue;             // uniform over the block
         const bool lds = lut_in_lds(S.mat);
         if (lds && s != staged) {
             __syncthreads();                          // every thread is done with the old LUT
@@ -132,7 +136,8 @@ k_pool_update_e(const PoolDev *__restrict__ P)
             staged = s;
         }
         const TileCoord tc = tile_coord(S.g, lw - P->item_ofs[s]);
-        if (tc.ok) update_e_tile<float>(S.E, S.H, S.ps, S.g, S.mat, S.cw, S.pw, StepRef{S.stp, 0}, tc, s_lut, lds);
+        if (tc.ok) update_e_tile<float, true>(S.E, S.H, S.ps, S.g, S.mat, S.cw, S.pw, S.fpts,
+                                         StepRef{S.stp, step}, tc, s_lut, lds);
     }
 }
 
@@ -143,7 +148,7 @@ k_pool_update_e(const PoolDev *__restrict__ P)
          base < (tot); base += gridDim.x * OEM_POOL_BLK)
 
 __global__ void __launch_bounds__(OEM_POOL_BLK)
-k_pool_points(const PoolDev *__restrict__ P, int slot)
+k_pool_points(const PoolDev *__restrict__ P, int step, int slot)
 {
     const int ns = P->n_pt[slot];
     if (ns == 0) return;
@@ -154,7 +159,7 @@ k_pool_points(const PoolDev *__restrict__ P, int slot)
         const PtSeg &seg = P->pt[slot][g];
         const SceneDev &S = P->sc[seg.scene];
         int n;
-        if (!scene_live(S, &n)) continue;
+        if (!scene_live(S, step, &n)) continue;
         const int t = base - ofs[g] + (int)threadIdx.x;
         if (t < seg.d.n_groups)
             point_group<float>(seg.d.e_side ? S.E : S.H, seg.d, S.mat, S.ch, S.ncell, n, t);
@@ -163,7 +168,7 @@ k_pool_points(const PoolDev *__restrict__ P, int slot)
 
 // phase 0: the ADE pre of scenes at step 0; phase 1: post (last step) or fused post + pre.
 __global__ void __launch_bounds__(OEM_POOL_BLK)
-k_pool_disp(const PoolDev *__restrict__ P, int phase)
+k_pool_disp(const PoolDev *__restrict__ P, int step, int phase)
 {
     const int ns = P->n_scenes;
     const int tot = P->disp_ofs[ns];
@@ -171,7 +176,7 @@ k_pool_disp(const PoolDev *__restrict__ P, int phase)
         const int s = find_seg(P->disp_ofs, ns, base);
         const SceneDev &S = P->sc[s];
         int n;
-        if (!scene_live(S, &n)) continue;
+        if (!scene_live(S, step, &n)) continue;
         int mode;
         if (phase == 0) {
             if (n != 0) continue;
@@ -185,7 +190,7 @@ k_pool_disp(const PoolDev *__restrict__ P, int phase)
 }
 
 __global__ void __launch_bounds__(OEM_POOL_BLK)
-k_pool_snap(const PoolDev *__restrict__ P)
+k_pool_snap(const PoolDev *__restrict__ P, int step)
 {
     const int nm = P->n_mon;
     if (nm == 0) return;
@@ -195,45 +200,37 @@ k_pool_snap(const PoolDev *__restrict__ P)
         const MonSeg &M = P->mon[g];
         const SceneDev &S = P->sc[M.scene];
         int n;
-        if (!scene_live(S, &n)) continue;
+        if (!scene_live(S, step, &n)) continue;
         const int q = base - P->snap_ofs[g] + (int)threadIdx.x;
         if (q < M.d.npts) snap_point<float>(M.d, S.E, S.H, S.ncell, S.ny, S.pz, n % M.d.T, q);
     }
 }
 
-// After the block: replay each scene's snapshots since its last flush.
+// After the block: replay the snapshots of each scene's steps of the block.
 __global__ void __launch_bounds__(OEM_FLUSH_BLK)
-k_pool_flush(const PoolDev *__restrict__ P)
+k_pool_flush(const PoolDev *__restrict__ P, int T)
 {
     __shared__ double2 s_ph[64][OEM_FLUSH_FG];
     const int nm = P->n_mon;
-    if (nm == 0) return;
     const int tot = P->flush_ofs[nm];
     for (int b = blockIdx.x; b < tot; b += gridDim.x) {
         const int g = find_seg(P->flush_ofs, nm, b);
         const MonSeg &M = P->mon[g];
         const SceneDev &S = P->sc[M.scene];
-        const int now = S.stp[0], from = S.stp[1];
-        if (now <= from) continue;                    // uniform over the block
-        flush_block<float>(M.d, b - P->flush_ofs[g], from, now - from, s_ph);
+        const int from = S.stp[0], cnt = min(T, S.n_total - from);
+        if (cnt <= 0) continue;                       // uniform over the block
+        flush_block<float>(M.d, b - P->flush_ofs[g], from, cnt, s_ph);
         __syncthreads();                              // every thread is done with the phases
     }
 }
 
-__global__ void k_pool_advance(const PoolDev *__restrict__ P)
+// The end of a block: every scene's counter moves past its steps.
+__global__ void k_pool_advance(const PoolDev *__restrict__ P, int T)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= P->n_scenes) return;
     int *stp = P->sc[s].stp;
-    if (stp[0] < P->sc[s].n_total) stp[0] += 1;
-}
-
-__global__ void k_pool_mark_flushed(const PoolDev *__restrict__ P)
-{
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= P->n_scenes) return;
-    int *stp = P->sc[s].stp;
-    stp[1] = stp[0];
+    stp[0] = min(stp[0] + T, P->sc[s].n_total);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -244,7 +241,7 @@ struct oem_pool {
     int device = 0;
     int T = 16;
     hipStream_t stream = nullptr;
-    std::mutex mu;
+    std::mutex mu;              // taken before the device-wide capture lock, never after it
 
     // arena: free ranges by offset, live allocations by offset
     char *base = nullptr;
@@ -263,7 +260,9 @@ struct oem_pool {
     bool stage_used[OEM_POOL_STAGES] = {};
     int stage_next = 0;
 
-    hipGraphExec_t graph = nullptr;
+    // the block graphs captured so far, by what they launch (desc_key)
+    std::map<uint32_t, hipGraphExec_t> graphs;
+    uint32_t desc_key = 0;                 // what the current descriptor table needs
     int grid_h = 0, grid_e = 0, grid_aux = 0, grid_pts = 0;
 
     int64_t launched = 0;                  // blocks enqueued
@@ -373,6 +372,7 @@ int build_desc(oem_pool *pool, PoolDev *h) {
         S.g = c->g;
         S.mat = c->mat;
         S.pw = c->pw;
+        S.fpts = c->fpts;
         if (c->has_disp) S.disp = c->disp;
         S.ch = c->dims.ch;
         S.cw = c->dims.cw;
@@ -387,6 +387,7 @@ int build_desc(oem_pool *pool, PoolDev *h) {
         dsp += c->has_disp ? pad_blk(c->disp.n_entry) : 0;
         for (auto &pt : c->points) {
             const int slot = points_slot(pt);
+            if (!pt.magnetic && c->fpts.n) continue;          // applied by the E update
             const int q = npt[slot]++;
             h->pt[slot][q].scene = ns;
             h->pt[slot][q].d = pt.d;
@@ -419,45 +420,82 @@ int build_desc(oem_pool *pool, PoolDev *h) {
     return OEM_OK;
 }
 
-int capture_graph(oem_pool *pool) {
+// What a block has to launch beside the sweeps: a bit per point slot, the ADE pass, the ADE pre of a
+// scene's first step, the monitors.  A launch with nothing to do cost 4 to 5 us a step (ten mixed
+// scenes of 64 to 144 cells a side: 13 launches a step, 5 of them needed).
+enum { BLK_DISP = 1 << OEM_POOL_SLOTS, BLK_PRE = BLK_DISP << 1, BLK_MON = BLK_PRE << 1, BLK_ALL = 2 * BLK_MON - 1 };
+#define OEM_POOL_GRAPHS 32          // captured kinds kept; past them a block launches everything
+
+uint32_t desc_key(const PoolDev *h) {
+    uint32_t k = 0;
+    for (int s = 0; s < OEM_POOL_SLOTS; ++s)
+        if (h->n_pt[s]) k |= 1u << s;
+    if (h->disp_ofs[h->n_scenes]) k |= BLK_DISP;
+    if (h->n_mon) k |= BLK_MON;
+    return k;
+}
+
+int capture_graph(oem_pool *pool, uint32_t key, hipGraphExec_t *out) {
     std::lock_guard<std::mutex> hold(oemi::device_sync_mutex());
     hipGraph_t gr = nullptr;
     HIP_OK(hipStreamBeginCapture(pool->stream, hipStreamCaptureModeThreadLocal));
     const PoolDev *P = pool->d_desc;
     const dim3 tb(OEM_TK, OEM_TJ), ab(OEM_POOL_BLK);
+    auto points = [&](int s, int slot) {
+        if (key >> slot & 1u)
+            hipLaunchKernelGGL(k_pool_points, dim3(pool->grid_pts), ab, 0, pool->stream, P, s, slot);
+    };
     for (int s = 0; s < pool->T; ++s) {
-        hipLaunchKernelGGL(k_pool_update_h, dim3(pool->grid_h), tb, 0, pool->stream, P);
-        for (int slot = 0; slot < 3; ++slot)
-            hipLaunchKernelGGL(k_pool_points, dim3(pool->grid_pts), ab, 0, pool->stream, P, slot);
-        hipLaunchKernelGGL(k_pool_disp, dim3(pool->grid_aux), ab, 0, pool->stream, P, 0);
-        hipLaunchKernelGGL(k_pool_update_e, dim3(pool->grid_e), tb, 0, pool->stream, P);
-        for (int slot = 3; slot < 6; ++slot)
-            hipLaunchKernelGGL(k_pool_points, dim3(pool->grid_pts), ab, 0, pool->stream, P, slot);
-        hipLaunchKernelGGL(k_pool_disp, dim3(pool->grid_aux), ab, 0, pool->stream, P, 1);
-        hipLaunchKernelGGL(k_pool_snap, dim3(pool->grid_aux), ab, 0, pool->stream, P);
-        hipLaunchKernelGGL(k_pool_advance, dim3(1), dim3(OEM_POOL_MAX), 0, pool->stream, P);
+        hipLaunchKernelGGL(k_pool_update_h, dim3(pool->grid_h), tb, 0, pool->stream, P, s);
+        for (int slot = 0; slot < 3; ++slot) points(s, slot);
+        // scenes join at block boundaries, so only a block's first step can be a scene's first
+        if (s == 0 && (key & BLK_PRE))
+            hipLaunchKernelGGL(k_pool_disp, dim3(pool->grid_aux), ab, 0, pool->stream, P, s, 0);
+        hipLaunchKernelGGL(k_pool_update_e, dim3(pool->grid_e), tb, 0, pool->stream, P, s);
+        for (int slot = 3; slot < 6; ++slot) points(s, slot);
+        if (key & BLK_DISP)
+            hipLaunchKernelGGL(k_pool_disp, dim3(pool->grid_aux), ab, 0, pool->stream, P, s, 1);
+        if (key & BLK_MON)
+            hipLaunchKernelGGL(k_pool_snap, dim3(pool->grid_aux), ab, 0, pool->stream, P, s);
     }
-    hipLaunchKernelGGL(k_pool_flush, dim3(pool->grid_aux), ab, 0, pool->stream, P);
-    hipLaunchKernelGGL(k_pool_mark_flushed, dim3(1), dim3(OEM_POOL_MAX), 0, pool->stream, P);
+    if (key & BLK_MON)
+        hipLaunchKernelGGL(k_pool_flush, dim3(pool->grid_aux), ab, 0, pool->stream, P, pool->T);
+    hipLaunchKernelGGL(k_pool_advance, dim3(1), dim3(OEM_POOL_MAX), 0, pool->stream, P, pool->T);
     const hipError_t el = hipGetLastError();
     const hipError_t ec = hipStreamEndCapture(pool->stream, &gr);
     if (el != hipSuccess || ec != hipSuccess) {
         if (gr) (void)hipGraphDestroy(gr);
         return fail(OEM_EHIP, "pool graph capture: %s", hipGetErrorString(el != hipSuccess ? el : ec));
     }
-    const hipError_t ei = hipGraphInstantiate(&pool->graph, gr, nullptr, nullptr, 0);
+    const hipError_t ei = hipGraphInstantiate(out, gr, nullptr, nullptr, 0);
     (void)hipGraphDestroy(gr);
     if (ei != hipSuccess) {
-        pool->graph = nullptr;
+        *out = nullptr;
         return fail(OEM_EHIP, "pool graph instantiate: %s", hipGetErrorString(ei));
     }
+    return OEM_OK;
+}
+
+// The captured block of a kind, captured on its first use (caller holds the pool's lock).
+int block_graph(oem_pool *pool, uint32_t key, hipGraphExec_t *out) {
+    auto it = pool->graphs.find(key);
+    if (it == pool->graphs.end()) {
+        if (pool->graphs.size() >= OEM_POOL_GRAPHS) {
+            *out = pool->graphs.at(BLK_ALL);
+            return OEM_OK;
+        }
+        hipGraphExec_t g = nullptr;
+        TRY(capture_graph(pool, key, &g));
+        it = pool->graphs.emplace(key, g).first;
+    }
+    *out = it->second;
     return OEM_OK;
 }
 
 void destroy_pool(oem_pool *p) {
     if (p->stream) (void)hipStreamSynchronize(p->stream);
     for (auto &f : p->inflight) (void)hipEventDestroy(f.second);
-    if (p->graph) (void)hipGraphExecDestroy(p->graph);
+    for (auto &g : p->graphs) (void)hipGraphExecDestroy(g.second);
     std::lock_guard<std::mutex> hold(oemi::device_sync_mutex());
     for (int i = 0; i < OEM_POOL_STAGES; ++i) {
         if (p->h_stage[i]) (void)hipHostFree(p->h_stage[i]);
@@ -522,7 +560,8 @@ extern "C" int oem_pool_create(int32_t device, uint64_t arena_bytes, int32_t dft
         if (gm && std::atoi(gm) > 0) p->grid_h = p->grid_e = std::atoi(gm) / OEM_NXCD * OEM_NXCD;
         const char *ga = std::getenv("OEM_POOL_AUX_GRID");
         if (ga && std::atoi(ga) > 0) p->grid_aux = std::atoi(ga) / OEM_NXCD * OEM_NXCD;
-        rc = capture_graph(p);
+        hipGraphExec_t g = nullptr;
+        rc = block_graph(p, BLK_ALL, &g);
     }
     if (rc) {
         destroy_pool(p);
@@ -621,6 +660,7 @@ extern "C" int oem_pool_launch(oem_pool *pool, int32_t n_blocks) {
                 }
                 rc = build_desc(pool, pool->h_stage[si]);
                 if (rc) break;
+                pool->desc_key = desc_key(pool->h_stage[si]);
                 if (hipMemcpyAsync(pool->d_desc, pool->h_stage[si], sizeof(PoolDev),
                                    hipMemcpyHostToDevice, pool->stream) != hipSuccess ||
                     hipEventRecord(pool->stage_ev[si], pool->stream) != hipSuccess) {
@@ -630,7 +670,13 @@ extern "C" int oem_pool_launch(oem_pool *pool, int32_t n_blocks) {
                 pool->stage_used[si] = true;
                 pool->dirty = false;
             }
-            if (hipGraphLaunch(pool->graph, pool->stream) != hipSuccess) {
+            uint32_t key = pool->desc_key;
+            for (oem_ctx *c : pool->members)
+                if (c->has_disp && c->step == 0) key |= BLK_PRE;
+            hipGraphExec_t graph = nullptr;
+            rc = block_graph(pool, key, &graph);
+            if (rc) break;
+            if (hipGraphLaunch(graph, pool->stream) != hipSuccess) {
                 rc = fail(OEM_EHIP, "pool graph launch");
                 break;
             }

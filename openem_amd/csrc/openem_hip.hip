@@ -716,7 +716,7 @@ extern "C" int oem_read_flux_time_monitor(oem_ctx *ctx, int32_t mon_id, double *
     return OEM_OK;
 }
 
-// The E-side point lists as part of the fused step when they are a few points (OEM_TAIL=0: never):
+// The E-side point lists as part of the E update when they are a few points (OEM_TAIL=0: never):
 // a launch of its own that corrects one cell held the step up by 2 to 8 us.  With the counter moved
 // once per captured block, a whole run of a 64^3 box soup went from 44.5 to 42.4 ms, of the 30 x 30
 // x 174 slab (no points) from 28.7 to 26.0, 512 steps of a graded 150 x 133 x 141 from 37.6 to 33.4.
@@ -940,6 +940,7 @@ extern "C" int oem_prepare(oem_ctx *ctx) {
     const long long nb = (long long)g.tiles * ((g.nx + g.chunk - 1) / g.chunk);
     if (nb > 0x7fffffffLL) return fail(OEM_EINVAL, "launch too large");
     g.nblocks = (int)nb;
+    plan_fused_points(ctx);
     // OEM_FUSE=1: the fused H+E step at any size, 0: never, outside a serving pool
     // (oem_set_step_form overrides the rule and OEM_FUSE)
     const char *fe = std::getenv("OEM_FUSE");
@@ -980,7 +981,6 @@ extern "C" int oem_prepare(oem_ctx *ctx) {
         ctx->fg.nblocks = (int)fb;
         ctx->fused = true;
         ctx->fuse_plain = march_bytes(ctx) <= OEM_MARCH_CACHED;
-        plan_fused_points(ctx);
         const char *fsn = std::getenv("OEM_FUSE_SNAP");
         if (!(fsn && fsn[0] == '0')) TRY(plan_fused_snaps(ctx));
     }
@@ -1144,8 +1144,12 @@ int launch_step_t(oem_ctx *c, int flush_after, Prof *pr, bool last, int off, int
         TRY(mark(OEM_K_DISP_PRE, false));
     }
     TRY(mark(OEM_K_UPDATE_E, true));
-    hipLaunchKernelGGL((k_update_e<F>), yg, yb, 0, c->stream, E, (const F *)H, c->psi, c->g,
-                       c->mat, c->dims.cw, c->pw, stp);
+    if (c->fpts.n)
+        hipLaunchKernelGGL((k_update_e<F, true>), yg, yb, 0, c->stream, E, (const F *)H, c->psi, c->g,
+                           c->mat, c->dims.cw, c->pw, c->fpts, stp);
+    else
+        hipLaunchKernelGGL((k_update_e<F, false>), yg, yb, 0, c->stream, E, (const F *)H, c->psi, c->g,
+                           c->mat, c->dims.cw, c->pw, c->fpts, stp);
     TRY(mark(OEM_K_UPDATE_E, false));
     }
     // ADE post on the new E (after every E-side correction); the post of a run's last step is
@@ -1209,20 +1213,35 @@ int launch_step_t(oem_ctx *c, int flush_after, Prof *pr, bool last, int off, int
                 TRY(mark(OEM_K_DFT_SNAP, false));
             }
         }
+        SnapDev sd{};
+        int64_t nb = 0;
+        auto snap = [&]() -> int {
+            if (!sd.n) return OEM_OK;
+            TRY(mark(OEM_K_DFT_SNAP, true));
+            hipLaunchKernelGGL((k_dft_snap<F>), dim3((unsigned)nb), dim3(256), 0, c->stream, sd,
+                               (const F *)E, (const F *)H, nc, c->dims.ny, c->pz, stp);
+            TRY(mark(OEM_K_DFT_SNAP, false));
+            sd.n = 0;
+            nb = 0;
+            return OEM_OK;
+        };
         for (auto &m : c->mons) {
             if (c->mons_off) break;
-            if (c->fused && m.fused && !m.n_patch) continue;
-            TRY(mark(OEM_K_DFT_SNAP, true));
-            if (c->fused && m.fused)
+            if (c->fused && m.fused) {
+                if (!m.n_patch) continue;
+                TRY(mark(OEM_K_DFT_SNAP, true));
                 hipLaunchKernelGGL((k_dft_snap_list<F>), dim3(blocks_for(m.n_patch, 256)), dim3(256), 0,
                                    c->stream, m.d, (const F *)E, (const F *)H, nc, c->dims.ny,
                                    c->pz, stp, (const int *)m.patch, m.n_patch);
-            else
-                hipLaunchKernelGGL((k_dft_snap<F>), dim3(blocks_for(m.d.npts, 256)), dim3(256), 0,
-                                   c->stream, m.d, (const F *)E, (const F *)H, nc, c->dims.ny,
-                                   c->pz, stp);
-            TRY(mark(OEM_K_DFT_SNAP, false));
+                TRY(mark(OEM_K_DFT_SNAP, false));
+                continue;
+            }
+            sd.ofs[sd.n] = (int)nb;
+            sd.m[sd.n++] = m.d;
+            nb += blocks_for(m.d.npts, 256);
+            if (sd.n == OEM_SNAP_MONS) TRY(snap());
         }
+        TRY(snap());
         if (adv) {
             TRY(mark(OEM_K_STEP, true));
             hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, c->stream, c->d_step, adv);
