@@ -740,6 +740,7 @@ struct oem_adjoint_state {
     float *rec = nullptr;            // (max_seg + 1) * n_design values of the field type
     int64_t rec_s0 = -1;
     int rec_n = 0;
+    BlkTab rec_tab{};                // the design cells by work-group of the E sweep
     // objective point lists: E side, H side; the (field, component, cell) keys they touch, and
     // whether every key is touched by one list only (then one launch applies them all)
     std::vector<Points> obj;
@@ -773,6 +774,18 @@ static void gather_design(oem_ctx *ctx, oem_adjoint_state *a, size_t row) {
     else
         hipLaunchKernelGGL((k_adj_gather<float>), g, b, 0, ctx->stream, ctx->cur_E(), a->d_comp,
                            a->d_cell, a->n_design, ctx->nst, a->rec + o);
+}
+
+// Every step from s0 on leaves E at the design cells in its row of the record.
+static void record_hook(oem_ctx *ctx, oem_adjoint_state *a, int64_t s0) {
+    oem_ctx::RecHook &h = ctx->rec_hook;
+    h.comp = a->d_comp;
+    h.cell = a->d_cell;
+    h.n = a->n_design;
+    h.rec = a->rec;
+    h.base = s0;
+    h.tab = a->rec_tab;
+    h.on = true;
 }
 
 static int adj_check(oem_ctx *ctx) {
@@ -892,6 +905,7 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
     std::vector<int> dcell(n_design);
     for (int q = 0; q < n_design; ++q) dcell[q] = (int)ctx->dev_cell(cell[q]);
     TRY(ctx->upload(&a->d_cell, (const int *)dcell.data(), dcell.size()));
+    (void)oemi::plan_sweep_record(ctx, cell, n_design, &a->rec_tab);
     TRY(ctx->upload(&a->dca, dca, (size_t)n_design));
     TRY(ctx->upload(&a->dcb, dcb, (size_t)n_design));
     TRY(ctx->upload(&a->ca, ca, (size_t)n_design));
@@ -952,13 +966,13 @@ extern "C" int oem_adjoint_record(oem_ctx *ctx, int64_t n_steps) {
     ctx->mons_off = true;
     a->rec_s0 = ctx->step;
     gather_design(ctx, a, 0);
+    record_hook(ctx, a, ctx->step);
     int rc = OEM_OK;
     // the last step's ADE post is not fused with a next pre: the pole state ends as P^n, as a
-    // run leaves it
-    for (int64_t s = 0; s < n_steps && !rc; ++s) {
-        rc = oemi::launch_one_step(ctx, s == n_steps - 1);
-        if (!rc) gather_design(ctx, a, (size_t)(s + 1));
-    }
+    // run leaves it.  The step counter moves once, at the end.
+    for (int64_t s = 0; s < n_steps && !rc; ++s)
+        rc = oemi::launch_one_step(ctx, s == n_steps - 1, (int)s, s == n_steps - 1 ? (int)n_steps : 0);
+    ctx->rec_hook.on = false;
     ctx->mons_off = false;
     TRY(rc);
     HIP_OK(hipGetLastError());
@@ -981,12 +995,7 @@ extern "C" int oem_adjoint_forward(oem_ctx *ctx, int64_t n_steps) {
     }
     const int64_t s0 = ctx->step;
     gather_design(ctx, a, 0);
-    ctx->rec_hook.comp = a->d_comp;
-    ctx->rec_hook.cell = a->d_cell;
-    ctx->rec_hook.n = a->n_design;
-    ctx->rec_hook.rec = a->rec;
-    ctx->rec_hook.base = s0;
-    ctx->rec_hook.on = true;
+    record_hook(ctx, a, s0);
     const int rc = oem_run(ctx, n_steps);
     ctx->rec_hook.on = false;
     if (ctx->graph) {

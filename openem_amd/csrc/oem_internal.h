@@ -39,6 +39,7 @@ struct Monitor {
     bool fused = false;   // the fused step writes its snapshots; `patch` lists the points an
     int *patch = nullptr; // E-side point list corrects afterwards, snapped again
     int n_patch = 0;
+    bool blk = false;     // the E sweep's work-groups write its snapshots
 };
 
 struct TimeMonitor {
@@ -148,6 +149,9 @@ struct oem_ctx {
     FuseSnap fsnap{};           // the DFT monitors the fused step snaps
     FusePts fpts{};             // the E-side points the E update applies (n = 0: none)
     bool fsnap_multi = false;   // some work-group meets more than one of them
+    BlkPts blk_h{}, blk_e{};    // the point lists the H and the E sweep apply (t.n = 0: none)
+    BlkSnap blk_snap{};         // the monitors the E sweep snaps
+    bool e_swept = false;       // the E sweep's work-groups leave the step's final E
     bool axis_set[3] = {false, false, false};
     MatDev mat{};
     bool mat_set = false;
@@ -176,6 +180,7 @@ struct oem_ctx {
         int n = 0;
         float *rec = nullptr;       // of the field type (two floats per value on complex fields)
         int64_t base = 0;
+        BlkTab tab{};               // its entries by work-group of the E sweep (n = 0: a launch)
     } rec_hook;
     struct oem_adjoint_state *adj = nullptr;
     hipGraphExec_t graph = nullptr;
@@ -263,7 +268,11 @@ int build_points(oem_ctx *ctx, int magnetic, int kind, int tfsf, int cplx_amp, i
                  const int32_t *comp, const int32_t *cell, const float *coef, const int32_t *col,
                  const float *phase, int32_t ncol, const double *tab, size_t tab_doubles,
                  Points *out);
-int launch_one_step(oem_ctx *ctx, bool last);       // one eager step, no flush, no profiling
+// One eager step, no flush, no profiling: the step at the device counter plus off, which then
+// moves by adv.
+int launch_one_step(oem_ctx *ctx, bool last, int off, int adv);
+// The entries of a cell list by work-group of the E sweep; false: they keep a launch of their own.
+bool plan_sweep_record(oem_ctx *ctx, const int32_t *cell, int n, BlkTab *out);
 int pool_retire(oem_ctx *ctx);                  // oem_ctx_destroy of a pool context
 int pool_wait_done(oem_ctx *ctx);               // before reading a pool context's results
 }

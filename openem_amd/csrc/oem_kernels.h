@@ -332,6 +332,122 @@ __device__ __forceinline__ void fold_points(const FusePts &fpt, uint32_t mask, i
 }
 
 // ------------------------------------------------------------------------------------------
+// Running DFT, batched: every step a snapshot of the monitored values goes into a ring of T
+// rows; every T steps one flush replays them in step order against the float64 phase table and
+// adds into the float64 accumulators (reference accumulate_dft / accumulate_dft_box and the
+// batched dft_snap_* / dft_flush_*, `openem/kernels/source_dft.cu:216-271`, `:371-430`,
+// `:453-779`; there the partial sums are float32, here they are float64).  Complex fields
+// accumulate (u_r + i u_i) e^{i w t}, the reference's complex DFT (`bloch.cu:389-481`).
+// ------------------------------------------------------------------------------------------
+struct MonDev {
+    int kind;                // 0 plane, 1 box
+    int axis, km, n1, n2;    // plane
+    int o[3], b[3];          // box
+    int ncomp, npts, nf, T;
+    void *snap;              // T * ncomp * npts elements of F
+    double *re, *im;         // ncomp * nf * npts
+    const double *phase;     // n_steps * nf * 4
+};
+
+// Point q of a monitor into ring row `slot`.
+template <typename F>
+__device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict__ E,
+                                           const F *__restrict__ H, size_t ncell, int ny, int pz,
+                                           int slot, int q)
+{
+    F *row = static_cast<F *>(m.snap) + (size_t)slot * m.ncomp * m.npts;
+    if (m.kind == 0) {
+        const int a = q / m.n2, b = q - a * m.n2;
+        int c[3];
+        const int t1 = m.axis == 0 ? 1 : 0, t2 = m.axis == 2 ? 1 : 2;
+        c[m.axis] = m.km; c[t1] = a; c[t2] = b;
+        const size_t id = ((size_t)c[0] * ny + c[1]) * pz + c[2];
+        c[m.axis] = m.km - 1;
+        const size_t idm = ((size_t)c[0] * ny + c[1]) * pz + c[2];
+        row[q] = E[(size_t)t1 * ncell + id];
+        row[m.npts + q] = E[(size_t)t2 * ncell + id];
+        row[2 * m.npts + q] = 0.5f * (H[(size_t)t1 * ncell + id] + H[(size_t)t1 * ncell + idm]);
+        row[3 * m.npts + q] = 0.5f * (H[(size_t)t2 * ncell + id] + H[(size_t)t2 * ncell + idm]);
+    } else {
+        const int bjk = m.b[1] * m.b[2];
+        const int a = q / bjk, r = q - a * bjk, b = r / m.b[2], cc = r - b * m.b[2];
+        const size_t id = ((size_t)(m.o[0] + a) * ny + (m.o[1] + b)) * pz + (m.o[2] + cc);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            row[(size_t)c * m.npts + q] = E[(size_t)c * ncell + id];
+            row[(size_t)(3 + c) * m.npts + q] = H[(size_t)c * ncell + id];
+        }
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// What a work-group of the two sweeps does for its own cells after its march: the point
+// corrections of the field it wrote and, on the E side, the monitors' snapshots and an adjoint's
+// design cells.  Tables made once per context list them by the work-group that owns the cell
+// (row lb of a table of n lists: items idx[ofs[lb n + l] .. ofs[lb n + l + 1]) of list l), so no
+// other work-group touches or needs them in the same launch and a barrier orders them after the
+// march's stores.  As launches of their own they cost 3.4 to 5 us each for a few thousand points.
+// ------------------------------------------------------------------------------------------
+#define OEM_BLK_LISTS 4
+#define OEM_BLK_MONS 8
+struct BlkTab {
+    int n;                      // lists (0: nothing to do)
+    const int *ofs, *idx;
+};
+struct BlkPts {
+    BlkTab t;
+    PointsDev p[OEM_BLK_LISTS];
+};
+struct BlkSnap {
+    BlkTab t;
+    MonDev m[OEM_BLK_MONS];
+};
+struct BlkRec {
+    BlkTab t;                   // one list: entries of the design tables
+    const int *comp, *cell;
+    int n;                      // entries of a row of rec
+    void *rec;
+    int64_t base;               // row (step + 1 - base)
+};
+
+// For each list of row lb that has items: a barrier, then do_item(list, item) over the block.
+template <typename Fn>
+__device__ __forceinline__ void blk_items(const BlkTab &t, int lb, Fn do_item) {
+    if (!t.n) return;
+    const int *o = t.ofs + (size_t)lb * t.n;
+    if (o[0] == o[t.n]) return;
+    const int tid = threadIdx.y * blockDim.x + threadIdx.x, nt = blockDim.x * blockDim.y;
+    for (int l = 0; l < t.n; ++l) {
+        const int a = o[l], b = o[l + 1];
+        if (a == b) continue;
+        __syncthreads();
+        for (int q = a + tid; q < b; q += nt) do_item(l, t.idx[q]);
+    }
+}
+template <typename F>
+__device__ __forceinline__ void blk_points(F *Fld, const BlkPts &bp, const MatDev &mat, float ch,
+                                           size_t ncell, StepRef stp, int lb) {
+    blk_items(bp.t, lb, [&](int l, int t) {
+        point_group<F>(Fld, bp.p[l], mat, ch, ncell, step_now(stp), t);
+    });
+}
+template <typename F>
+__device__ __forceinline__ void blk_snaps(const F *E, const F *H, const BlkSnap &bs, size_t ncell,
+                                          int ny, int pz, StepRef stp, int lb) {
+    blk_items(bs.t, lb, [&](int l, int q) {
+        snap_point<F>(bs.m[l], E, H, ncell, ny, pz, step_now(stp) % bs.m[l].T, q);
+    });
+}
+template <typename F>
+__device__ __forceinline__ void blk_record(const F *E, const BlkRec &br, size_t ncell, StepRef stp,
+                                           int lb) {
+    blk_items(br.t, lb, [&](int, int q) {
+        F *row = static_cast<F *>(br.rec) + (size_t)((int64_t)step_now(stp) + 1 - br.base) * br.n;
+        row[q] = E[(size_t)br.comp[q] * ncell + br.cell[q]];
+    });
+}
+
+// ------------------------------------------------------------------------------------------
 // H half step (reference update_h, `openem/kernels/yee.cu:76-137`; complex variant
 // update_h_c, `openem/kernels/bloch.cu:38-126`) fused with the H side of the plane-wave TF/SF
 // correction (`openem/kernels/source_dft.cu:40-55`).
@@ -445,11 +561,12 @@ __device__ __forceinline__ void update_h_tile(F *__restrict__ H, const F *__rest
 template <typename F>
 __global__ void __launch_bounds__(OEM_TK * OEM_TJ)
 k_update_h(F *__restrict__ H, const F *__restrict__ E, PsiDev ps, GridDev g, float ch,
-           PlaneSrcDev pw, StepRef stp)
+           PlaneSrcDev pw, StepRef stp, BlkPts bp, size_t ncell)
 {
-    const TileCoord tc = tile_coord(g, xcd_remap(blockIdx.x, g.nblocks));
-    if (!tc.ok) return;
-    update_h_tile<F>(H, E, ps, g, ch, pw, stp, tc);
+    const int lb = xcd_remap(blockIdx.x, g.nblocks);
+    const TileCoord tc = tile_coord(g, lb);
+    if (tc.ok) update_h_tile<F>(H, E, ps, g, ch, pw, stp, tc);
+    blk_points<F>(H, bp, MatDev{}, ch, ncell, stp, lb);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -633,10 +750,10 @@ __device__ __forceinline__ void update_e_tile(F *__restrict__ E, const F *__rest
     }
 }
 
-template <typename F, bool PTS>
+template <typename F>
 __global__ void __launch_bounds__(OEM_TK * OEM_TJ)
 k_update_e(F *__restrict__ E, const F *__restrict__ H, PsiDev ps, GridDev g, MatDev mat,
-           float cw, PlaneSrcDev pw, FusePts fpt, StepRef stp)
+           float cw, PlaneSrcDev pw, StepRef stp, BlkPts bp, BlkSnap bs, BlkRec br, size_t ncell)
 {
     __shared__ float4 s_lut[2 * OEM_LDS_CLASSES];
     const bool lds_lut = lut_in_lds(mat);
@@ -644,9 +761,13 @@ k_update_e(F *__restrict__ E, const F *__restrict__ H, PsiDev ps, GridDev g, Mat
         stage_lut(s_lut, mat);
         __syncthreads();
     }
-    const TileCoord tc = tile_coord(g, xcd_remap(blockIdx.x, g.nblocks));
-    if (!tc.ok) return;
-    update_e_tile<F, PTS>(E, H, ps, g, mat, cw, pw, fpt, stp, tc, s_lut, lds_lut);
+    const int lb = xcd_remap(blockIdx.x, g.nblocks);
+    const TileCoord tc = tile_coord(g, lb);
+    if (tc.ok)
+        update_e_tile<F, false>(E, H, ps, g, mat, cw, pw, FusePts{}, stp, tc, s_lut, lds_lut);
+    blk_points<F>(E, bp, mat, 0.f, ncell, stp, lb);
+    blk_snaps<F>(E, H, bs, ncell, g.ny, g.pz, stp, lb);
+    blk_record<F>(E, br, ncell, stp, lb);
 }
 
 // Plane-wave H-side correction at cell k (the injection term of update_h).
@@ -1712,55 +1833,6 @@ k_flux_time_sum(FluxTimeDev d, StepRef stp)
     if (threadIdx.x == 0) {
         if (s1 >= 0) d.buf[s1] += t1;
         if (s0 >= 0) d.buf[s0] = t0;
-    }
-}
-
-// ------------------------------------------------------------------------------------------
-// Running DFT, batched: every step a snapshot of the monitored values goes into a ring of T
-// rows; every T steps one flush replays them in step order against the float64 phase table and
-// adds into the float64 accumulators (reference accumulate_dft / accumulate_dft_box and the
-// batched dft_snap_* / dft_flush_*, `openem/kernels/source_dft.cu:216-271`, `:371-430`,
-// `:453-779`; there the partial sums are float32, here they are float64).  Complex fields
-// accumulate (u_r + i u_i) e^{i w t}, the reference's complex DFT (`bloch.cu:389-481`).
-// ------------------------------------------------------------------------------------------
-struct MonDev {
-    int kind;                // 0 plane, 1 box
-    int axis, km, n1, n2;    // plane
-    int o[3], b[3];          // box
-    int ncomp, npts, nf, T;
-    void *snap;              // T * ncomp * npts elements of F
-    double *re, *im;         // ncomp * nf * npts
-    const double *phase;     // n_steps * nf * 4
-};
-
-// Point q of a monitor into ring row `slot`.
-template <typename F>
-__device__ __forceinline__ void snap_point(const MonDev &m, const F *__restrict__ E,
-                                           const F *__restrict__ H, size_t ncell, int ny, int pz,
-                                           int slot, int q)
-{
-    F *row = static_cast<F *>(m.snap) + (size_t)slot * m.ncomp * m.npts;
-    if (m.kind == 0) {
-        const int a = q / m.n2, b = q - a * m.n2;
-        int c[3];
-        const int t1 = m.axis == 0 ? 1 : 0, t2 = m.axis == 2 ? 1 : 2;
-        c[m.axis] = m.km; c[t1] = a; c[t2] = b;
-        const size_t id = ((size_t)c[0] * ny + c[1]) * pz + c[2];
-        c[m.axis] = m.km - 1;
-        const size_t idm = ((size_t)c[0] * ny + c[1]) * pz + c[2];
-        row[q] = E[(size_t)t1 * ncell + id];
-        row[m.npts + q] = E[(size_t)t2 * ncell + id];
-        row[2 * m.npts + q] = 0.5f * (H[(size_t)t1 * ncell + id] + H[(size_t)t1 * ncell + idm]);
-        row[3 * m.npts + q] = 0.5f * (H[(size_t)t2 * ncell + id] + H[(size_t)t2 * ncell + idm]);
-    } else {
-        const int bjk = m.b[1] * m.b[2];
-        const int a = q / bjk, r = q - a * bjk, b = r / m.b[2], cc = r - b * m.b[2];
-        const size_t id = ((size_t)(m.o[0] + a) * ny + (m.o[1] + b)) * pz + (m.o[2] + cc);
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            row[(size_t)c * m.npts + q] = E[(size_t)c * ncell + id];
-            row[(size_t)(3 + c) * m.npts + q] = H[(size_t)c * ncell + id];
-        }
     }
 }
 

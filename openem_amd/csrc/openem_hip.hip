@@ -835,6 +835,125 @@ static int plan_fused_snaps(oem_ctx *ctx) {
     return OEM_OK;
 }
 
+// The work-groups the chip holds at once, and the share of a larger launch's that may have a tail
+// (build_blk).
+#define OEM_BLK_RESIDENT 1024
+#define OEM_BLK_SHARE 8
+
+// Tables of the items of several lists by the work-group that owns them: blk(l, t) of the n[l]
+// items of list l.  False, and the lists keep their own launches, when out of memory or when too
+// many work-groups would end with a tail of dependent loads: a grid whose work-groups all run at
+// once hides them behind each other (120 x 120 x 44, mode source, planes and design: E sweep 11.2
+// us with 11.8 us of launches after it, 12.5 with the lists), a larger one pays them per round
+// (160^3 with a z plane, in every work-group: 42.7 us against 35.6 and a launch of 5; 400 x 400 x
+// 48 with a 160 x 160 design, in a sixth of them: 99.9 against 79.3 and 5.2).
+template <typename Fn>
+static bool build_blk(oem_ctx *ctx, int nblocks, const std::vector<int> &n, Fn blk, BlkTab *out) {
+    const size_t nl = n.size();
+    std::vector<int> ofs((size_t)nblocks * nl + 1, 0);
+    size_t total = 0;
+    for (size_t l = 0; l < nl; ++l) {
+        for (int t = 0; t < n[l]; ++t) ++ofs[(size_t)blk((int)l, t) * nl + l + 1];
+        total += (size_t)n[l];
+    }
+    if (total > 0x7fffffff) return false;
+    int touched = 0;
+    for (int b = 0; b < nblocks; ++b) {
+        bool any = false;
+        for (size_t l = 0; l < nl; ++l) any |= ofs[(size_t)b * nl + l + 1] != 0;
+        touched += any;
+    }
+    if (nblocks > OEM_BLK_RESIDENT && touched > nblocks / OEM_BLK_SHARE) return false;
+    for (size_t q = 1; q < ofs.size(); ++q) ofs[q] += ofs[q - 1];
+    std::vector<int> at(ofs.begin(), ofs.end() - 1), idx(total);
+    for (size_t l = 0; l < nl; ++l)
+        for (int t = 0; t < n[l]; ++t) idx[at[(size_t)blk((int)l, t) * nl + l]++] = t;
+    int *d_ofs = nullptr, *d_idx = nullptr;
+    if (ctx->upload(&d_ofs, ofs.data(), ofs.size()) || ctx->upload(&d_idx, idx.data(), idx.size())) {
+        (void)hipGetLastError();
+        return false;
+    }
+    *out = BlkTab{(int)nl, d_ofs, d_idx};
+    return true;
+}
+
+// The work-group of the sweeps that owns the cell (i, j, k) (tile_coord).
+static int sweep_block(const GridDev &g, int i, int j, int k) {
+    const int nkt = (g.nz + OEM_TK - 1) / OEM_TK;
+    const int tile = g.flat ? (int)(((int64_t)j * g.nz + k) / (OEM_TK * OEM_TJ))
+                            : j / OEM_TJ * nkt + k / OEM_TK;
+    return i / g.chunk * g.tiles + tile;
+}
+
+// The entries of a cell list by work-group of the E sweep, for the recording of an adjoint's design
+// cells; false where they keep a launch of their own.
+bool oemi::plan_sweep_record(oem_ctx *ctx, const int32_t *cell, int n, BlkTab *out) {
+    if (!ctx->e_swept) return false;
+    const int ny = ctx->dims.ny, nz = ctx->dims.nz;
+    return build_blk(ctx, ctx->g.nblocks, {n}, [&](int, int t) {
+        const int r = cell[t] % (ny * nz);
+        return sweep_block(ctx->g, cell[t] / (ny * nz), r / nz, r % nz);
+    }, out);
+}
+
+// The point lists and the snapshots that the work-groups of the two sweeps take with them (their
+// cells' own, after the march), outside serving pools: the point lists of a side when they are at
+// most OEM_BLK_LISTS, the monitors when they are at most OEM_BLK_MONS and no E-side list is left to
+// a launch after the sweep, both within build_blk's bound.  OEM_TAIL=0 keeps the separate launches.
+static void plan_sweeps(oem_ctx *ctx) {
+    const char *te = std::getenv("OEM_TAIL");
+    if (te && te[0] == '0') return;
+    const GridDev &g = ctx->g;
+    const int ny = g.ny, nz = g.nz;
+    for (int side = 0; side < 2; ++side) {
+        std::vector<const Points *> ls;
+        std::vector<int> n;
+        for (int slot = 3 * side; slot < 3 * side + 3; ++slot)
+            for (const auto &pt : ctx->points)
+                if (oemi::points_slot(pt) == slot) {
+                    ls.push_back(&pt);
+                    n.push_back(pt.d.n_groups);
+                }
+        if (ls.empty()) {
+            ctx->e_swept = side != 0;
+            continue;
+        }
+        if (ls.size() > OEM_BLK_LISTS) continue;
+        BlkPts &b = side ? ctx->blk_e : ctx->blk_h;
+        if (!build_blk(ctx, g.nblocks, n, [&](int l, int t) {
+                const int id = ls[l]->cells[t], r = id % (ny * nz);
+                return sweep_block(g, id / (ny * nz), r / nz, r % nz);
+            }, &b.t))
+            continue;
+        for (size_t l = 0; l < ls.size(); ++l) b.p[l] = ls[l]->d;
+        ctx->e_swept = side != 0;
+    }
+    const size_t nm = ctx->mons.size();
+    if (!ctx->e_swept || nm < 1 || nm > OEM_BLK_MONS) return;
+    std::vector<int> n;
+    for (size_t m = 0; m < nm; ++m) n.push_back(ctx->mons[m].d.npts);
+    BlkSnap b{};
+    if (!build_blk(ctx, g.nblocks, n, [&](int l, int q) {
+            const MonDev &m = ctx->mons[l].d;
+            int c[3];
+            if (m.kind == 0) {
+                c[m.axis] = m.km;
+                c[m.axis == 0 ? 1 : 0] = q / m.n2;
+                c[m.axis == 2 ? 1 : 2] = q % m.n2;
+            } else {
+                const int bjk = m.b[1] * m.b[2], r = q % bjk;
+                c[0] = m.o[0] + q / bjk; c[1] = m.o[1] + r / m.b[2]; c[2] = m.o[2] + r % m.b[2];
+            }
+            return sweep_block(g, c[0], c[1], c[2]);
+        }, &b.t))
+        return;
+    for (size_t m = 0; m < nm; ++m) {
+        b.m[m] = ctx->mons[m].d;
+        ctx->mons[m].blk = true;
+    }
+    ctx->blk_snap = b;
+}
+
 // The fused step's tiles of the (ny, nz) plane: 64-wide strips and, when at most 32 cells of a
 // row are left, one 32-wide strip of twice the rows, which idles fewer lanes (step times with and
 // without it: 200^3 186 / 201 us, 144^3 57.5 / 59.8, 80^3 23.6 / 25.6, 250 x 230 x 210 233 / 241).
@@ -983,6 +1102,9 @@ extern "C" int oem_prepare(oem_ctx *ctx) {
         ctx->fuse_plain = march_bytes(ctx) <= OEM_MARCH_CACHED;
         const char *fsn = std::getenv("OEM_FUSE_SNAP");
         if (!(fsn && fsn[0] == '0')) TRY(plan_fused_snaps(ctx));
+    } else if (!ctx->pool) {
+        ctx->fpts = FusePts{};      // the sweeps' work-groups take whole lists
+        plan_sweeps(ctx);
     }
     ctx->prepared = true;
     return OEM_OK;
@@ -1027,7 +1149,7 @@ int launch_flush(oem_ctx *c, int cnt) {
 // OEM_TAIL=0 keeps the separate launches.
 static bool tail_plan(const oem_ctx *c, TailDev *t) {
     const char *te = std::getenv("OEM_TAIL");
-    if ((te && te[0] == '0') || c->rec_hook.on) return false;
+    if ((te && te[0] == '0') || (c->rec_hook.on && !c->rec_hook.tab.n)) return false;
     t->n_pts = t->n_snap = t->n_tm = 0;
     if (!c->mons_off) {
         if (!c->ftmons.empty() || c->tmons.size() > OEM_TAIL_TMONS) return false;
@@ -1038,12 +1160,13 @@ static bool tail_plan(const oem_ctx *c, TailDev *t) {
     }
     for (int slot = 3; slot < 6; ++slot)
         for (const auto &pt : c->points) {
-            if (points_slot(pt) != slot || c->fpts.n) continue;
+            if (points_slot(pt) != slot || c->fpts.n || c->blk_e.t.n) continue;
             if (t->n_pts == OEM_TAIL_LISTS || pt.d.n_groups > OEM_TAIL_THREADS) return false;
             t->pts[t->n_pts++] = pt.d;
         }
     if (!c->mons_off)
         for (const auto &m : c->mons) {
+            if (m.blk) continue;
             if (!(c->fused && m.fused)) return false;
             if (!m.n_patch) continue;
             if (t->n_snap == OEM_TAIL_LISTS || m.n_patch > OEM_TAIL_THREADS) return false;
@@ -1127,11 +1250,11 @@ int launch_step_t(oem_ctx *c, int flush_after, Prof *pr, bool last, int off, int
     } else {
     TRY(mark(OEM_K_UPDATE_H, true));
     hipLaunchKernelGGL((k_update_h<F>), yg, yb, 0, c->stream, H, (const F *)E, c->psi, c->g,
-                       c->dims.ch, c->pw, stp);
+                       c->dims.ch, c->pw, stp, c->blk_h, nc);
     TRY(mark(OEM_K_UPDATE_H, false));
     for (int slot = 0; slot < 3; ++slot)
         for (auto &pt : c->points) {
-            if (points_slot(pt) != slot) continue;
+            if (points_slot(pt) != slot || c->blk_h.t.n) continue;
             TRY(mark(points_kid(pt), true));
             hipLaunchKernelGGL((k_points<F>), dim3(blocks_for(pt.d.n_groups, 256)), dim3(256), 0,
                                c->stream, H, pt.d, c->mat, c->dims.ch, nc, stp);
@@ -1144,12 +1267,11 @@ int launch_step_t(oem_ctx *c, int flush_after, Prof *pr, bool last, int off, int
         TRY(mark(OEM_K_DISP_PRE, false));
     }
     TRY(mark(OEM_K_UPDATE_E, true));
-    if (c->fpts.n)
-        hipLaunchKernelGGL((k_update_e<F, true>), yg, yb, 0, c->stream, E, (const F *)H, c->psi, c->g,
-                           c->mat, c->dims.cw, c->pw, c->fpts, stp);
-    else
-        hipLaunchKernelGGL((k_update_e<F, false>), yg, yb, 0, c->stream, E, (const F *)H, c->psi, c->g,
-                           c->mat, c->dims.cw, c->pw, c->fpts, stp);
+    const BlkSnap bs = c->mons_off ? BlkSnap{} : c->blk_snap;
+    const oem_ctx::RecHook &rh = c->rec_hook;
+    const BlkRec br = rh.on ? BlkRec{rh.tab, rh.comp, rh.cell, rh.n, rh.rec, rh.base} : BlkRec{};
+    hipLaunchKernelGGL((k_update_e<F>), yg, yb, 0, c->stream, E, (const F *)H, c->psi, c->g, c->mat,
+                       c->dims.cw, c->pw, stp, c->blk_e, bs, br, nc);
     TRY(mark(OEM_K_UPDATE_E, false));
     }
     // ADE post on the new E (after every E-side correction); the post of a run's last step is
@@ -1181,14 +1303,14 @@ int launch_step_t(oem_ctx *c, int flush_after, Prof *pr, bool last, int off, int
         // `openem/solver.py:945-968`)
         for (int slot = 3; slot < 6; ++slot)
             for (auto &pt : c->points) {
-                if (points_slot(pt) != slot || c->fpts.n) continue;
+                if (points_slot(pt) != slot || c->fpts.n || c->blk_e.t.n) continue;
                 TRY(mark(points_kid(pt), true));
                 hipLaunchKernelGGL((k_points<F>), dim3(blocks_for(pt.d.n_groups, 256)), dim3(256), 0,
                                    c->stream, E, pt.d, c->mat, c->dims.ch, nc, stp);
                 TRY(mark(points_kid(pt), false));
             }
         TRY(disp_post());
-        if (c->rec_hook.on)
+        if (c->rec_hook.on && !c->rec_hook.tab.n)
             hipLaunchKernelGGL((k_rec_gather<F>), dim3(blocks_for(c->rec_hook.n, 256)), dim3(256), 0,
                                c->stream, (const F *)E, c->rec_hook.comp, c->rec_hook.cell,
                                c->rec_hook.n, nc, reinterpret_cast<F *>(c->rec_hook.rec), stp,
@@ -1227,6 +1349,7 @@ int launch_step_t(oem_ctx *c, int flush_after, Prof *pr, bool last, int off, int
         };
         for (auto &m : c->mons) {
             if (c->mons_off) break;
+            if (m.blk) continue;
             if (c->fused && m.fused) {
                 if (!m.n_patch) continue;
                 TRY(mark(OEM_K_DFT_SNAP, true));
@@ -1264,8 +1387,8 @@ int launch_step(oem_ctx *c, int flush_after, Prof *pr, bool last, int off = 0, i
 
 }  // namespace
 
-int oemi::launch_one_step(oem_ctx *ctx, bool last) {
-    TRY(launch_step(ctx, 0, nullptr, last));
+int oemi::launch_one_step(oem_ctx *ctx, bool last, int off, int adv) {
+    TRY(launch_step(ctx, 0, nullptr, last, off, adv));
     ctx->step++;
     return OEM_OK;
 }
