@@ -43,9 +43,20 @@
 #ifndef OEM_ADJ_TJ
 #define OEM_ADJ_TJ 4
 #endif
-// 8 planes measured best on the 400 x 400 x 48 bend (s per design: 4 3.04-3.06, 6 3.01, 8
-// 3.02-3.09, 12 3.08, 16 3.11-3.18, 24 3.10, 32 3.17)
+// 8 planes on large grids (400 x 400 x 48 bend, s per design: 4 3.04-3.06, 6 3.01, 8 3.02-3.09, 12
+// 3.08, 16 3.11-3.18, 24 3.10, 32 3.17), fewer where that leaves under OEM_ADJ_BLOCKS work-groups
+// (ms per pass with 2 / 4 / 8 planes: 120 x 120 x 44, 1000 steps, 73.4 / 77.5 / 88.8; 96 x 96 x 40,
+// 64 steps, 3.0 / 3.3 / 3.9; 120 x 120 x 100 5.8 / 5.4 / 5.9; 160 x 160 x 64 6.7 / 6.5 / 6.3)
 #define OEM_ADJ_CHUNK 8
+#define OEM_ADJ_BLOCKS 1000
+// the fused transposes: threads of a work-group, work-groups the chip holds at once, the longest
+// row and the most rows of a tile, and the bytes of both sets up to which the stores stay in the
+// caches
+#define OEM_ADJ_WG 512
+#define OEM_ADJ_RESIDENT 512
+#define OEM_ADJ_FUSE_NZ 128
+#define OEM_ADJ_ROWS 64
+#define OEM_ADJ_CACHED (200ull << 20)
 
 namespace {
 
@@ -59,6 +70,10 @@ struct AdjDev {
     float ch;
     size_t ncell;                // cells of a component, row padding included
     int chunk;                   // x planes per block of the transposes
+    // the fused transposes: where they write the new lE and lH, the rows of a work-group's tile
+    // (the first a halo), the tiles along y and the work-groups
+    float *lE_n, *lH_n;
+    int rows, tiles, nblocks;
 };
 
 // E transpose, part 1: lH_b += D_bwd^T q_{c,a} for the two terms with source b.
@@ -595,21 +610,360 @@ __device__ __forceinline__ double grad_term(float l, float dca, float dcb, float
     const float s = (e1 - ca * e0) / cb;
     return (double)l * ((double)dca * e0 + (double)dcb * s);
 }
+// The design tables of one backward step: e0, e1 the recorded rows of E before and after it.
+struct GradDev {
+    const int *comp, *cell;
+    const float *dca, *dcb, *ca, *cb;
+    const void *e0, *e1;
+    double *g;
+    int n;
+};
 template <typename F>
-__global__ void __launch_bounds__(256)
-k_adj_grad(const F *lE, const int *comp, const int *cell, const float *dca, const float *dcb,
-           const float *ca, const float *cb, const F *e0, const F *e1, int n,
-           size_t ncell, double *g)
+__device__ __forceinline__ void grad_entry(const F *lE, const GradDev &d, int q, size_t ncell) {
+    const F *e0 = static_cast<const F *>(d.e0), *e1 = static_cast<const F *>(d.e1);
+    const F l = lE[(size_t)d.comp[q] * ncell + d.cell[q]];
+    if constexpr (sizeof(F) == 4) {
+        d.g[q] += grad_term(l, d.dca[q], d.dcb[q], d.ca[q], d.cb[q], e0[q], e1[q]);
+    } else {
+        d.g[q] += grad_term(l.r, d.dca[q], d.dcb[q], d.ca[q], d.cb[q], e0[q].r, e1[q].r) +
+                  grad_term(l.i, d.dca[q], d.dcb[q], d.ca[q], d.cb[q], e0[q].i, e1[q].i);
+    }
+}
+template <typename F>
+__global__ void __launch_bounds__(256) k_adj_grad(const F *lE, GradDev d, size_t ncell)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    const F l = lE[(size_t)comp[q] * ncell + cell[q]];
-    if constexpr (sizeof(F) == 4) {
-        g[q] += grad_term(l, dca[q], dcb[q], ca[q], cb[q], e0[q], e1[q]);
-    } else {
-        g[q] += grad_term(l.r, dca[q], dcb[q], ca[q], cb[q], e0[q].r, e1[q].r) +
-                grad_term(l.i, dca[q], dcb[q], ca[q], cb[q], e0[q].i, e1[q].i);
+    if (q < d.n) grad_entry<F>(lE, d, q, ncell);
+}
+
+// What a work-group of the fused transposes does for its own cells after its march: the objective
+// points and the eps gradient of the next backward step (forward step n), by tables like the
+// sweeps'.
+struct AdjTail {
+    BlkTab obj, grad;
+    ObjDev o;
+    GradDev g;
+    int n;
+};
+
+// Both transposes in one march up x, on real fields.  The E transpose takes lambda_E from the
+// forward neighbours and the H transpose the resulting lambda_H from the backward ones, the forward
+// step's own pattern: a work-group holds whole rows of the (y, z) plane (rows of nz threads, the
+// first a halo row whose lambda_H it recomputes), exchanges the y and z terms of each half through
+// LDS and carries the x terms in registers, so the new lambda_H is used without going through
+// memory (48 bytes a cell instead of 72, and one launch: 120 x 120 x 44 21.5 us a step with the tail
+// below against 24 for the two kernels and 9.6 for their launches, 400 x 400 x 48 165 against 178).
+// The last row's forward neighbour is recomputed from its cell; a chunk starts with the
+// plane before it, for the x terms of its lambda_H alone.  Old and new values are two sets (the
+// halos read old ones that other work-groups replace): fields [lE, lH], psi [lpe, lph].
+//
+// Small grids are bound by instruction issue, so the masks (0 or +-1 here: exact) are folded into
+// the 1/dl of their term and a term that a cell does not have gets the weight 0 instead of a branch.
+// MK: where the coefficients come from (mat_kind).
+template <int MK, int AUX>
+__global__ void __launch_bounds__(OEM_ADJ_WG, 4) k_adj_he(AdjDev d, AdjTail tl)
+{
+    typedef FT<float> T;
+    __shared__ float4 s_lut[MK == 0 ? 2 * OEM_LDS_CLASSES : 1];
+    __shared__ float s_e[4][OEM_ADJ_WG], s_h[4][OEM_ADJ_WG];
+    const MatDev &mat = d.mat;
+    if (MK == 0) {
+        stage_lut_adj(s_lut, mat);
+        __syncthreads();
     }
+    const GridDev &g = d.g;
+    const AxisDev &X = g.ax[0], &Y = g.ax[1], &Z = g.ax[2];
+    const int nx = g.nx, ny = g.ny, nz = g.nz, pz = g.pz;
+    const int lb = xcd_remap(blockIdx.x, d.nblocks);
+    const int tile = lb % d.tiles, chunk = lb / d.tiles;
+    const int i0 = chunk * d.chunk, i1 = min(i0 + d.chunk, nx);
+    const int tid = threadIdx.x;
+    // row r of the tile is row j0 + r - 1 of the grid, row 0 the backward neighbour of j0; threads
+    // past the tile or the grid take a valid column and store nothing
+    const int rr = tid / nz, k = tid - rr * nz, r = min(rr, d.rows - 1);
+    const int j0 = tile * (d.rows - 1), jr = j0 + r - 1;
+    const bool act = rr < d.rows && r > 0 && jr < ny;
+    const int j = r > 0 ? min(jr, ny - 1) : j0 > 0 ? j0 - 1 : cidx_at(Y.prv, 0);
+    const uint32_t nc = (uint32_t)d.ncell, plane = (uint32_t)(ny * pz), pl4 = 4u * plane;
+    const int wy = Y.lo + Y.hi, wz = Z.lo + Z.hi;
+    const uint32_t syp = 4u * (uint32_t)(wy * pz), szp = 4u * (uint32_t)(ny * wz);
+    const float mch = -d.ch;
+    const uint32_t cB = 4u * nc, pB = 4u * d.psl.total;
+    const rsrc_t rF = mk_rsrc(d.lE, 6u * cB), rFn = mk_rsrc(d.lE_n, 6u * cB);
+    const rsrc_t rP = mk_rsrc(d.lpe, 2u * pB), rPn = mk_rsrc(d.lpe_n, 2u * pB);
+    const rsrc_t rC = mk_rsrc(mat.cls, nc * 2u);
+    const rsrc_t rL = mk_rsrc(mat.lut, (uint32_t)mat.n_classes * 32u);
+    const uint32_t ox0 = 4u * d.psl.off[0], ox1 = 4u * d.psl.off[1], oy0 = 4u * d.psl.off[2],
+                   oy1 = 4u * d.psl.off[3], oz0 = 4u * d.psl.off[4], oz1 = 4u * d.psl.off[5];
+    // neighbours: interior ones are one away, the ends' come from the tables
+    const int yw = cidx_at(Y.nxt, ny - 1), yv = cidx_at(Y.prv, 0);
+    const int zw = cidx_at(Z.nxt, nz - 1), zv = cidx_at(Z.prv, 0);
+    const int jn = j + 1 < ny ? j + 1 : yw, jp = j > 0 ? j - 1 : yv;
+    const int kn = k + 1 < nz ? k + 1 : zw, kp = k > 0 ? k - 1 : zv;
+    // a term's weights: 1/dl at the cell, mask / dl of the cell's own difference at a clamped end,
+    // mask / dl of the neighbour's
+    struct Wt { float c, end, nb; };
+    const bool ye_nb = j + 1 < ny || (yw != j && cidx_at(Y.prv, yw) == j);
+    const bool ze_nb = k + 1 < nz || (zw != k && cidx_at(Z.prv, zw) == k);
+    const bool yh_nb = j > 0 || (yv != 0 && cidx_at(Y.nxt, yv) == 0);
+    const bool zh_nb = k > 0 || (zv != 0 && cidx_at(Z.nxt, zv) == 0);
+    auto weight = [](const AxisDev &A, int p, int q, bool end, bool nb, int fidl, int fm) {
+        const float c = axv(A, p, fidl);
+        return Wt{c, end ? axv(A, p, fm) * c : 0.f, nb ? axv(A, q, fm) * axv(A, q, fidl) : 0.f};
+    };
+    const Wt ye = weight(Y, j, jn, jp == j, ye_nb, AX_IDLD, AX_MPV);
+    const Wt ze = weight(Z, k, kn, kp == k, ze_nb, AX_IDLD, AX_MPV);
+    const Wt yh = weight(Y, j, jp, jn == j, yh_nb, AX_IDLP, AX_MNX);
+    const Wt zh = weight(Z, k, kp, kn == k, zh_nb, AX_IDLP, AX_MNX);
+    const float ypec = axv(Y, j, AX_PEC), zpec = axv(Z, k, AX_PEC), yz = ypec * zpec;
+    const int ys = slab_of(j, ny, Y.lo, Y.hi), zs = slab_of(k, nz, Z.lo, Z.hi);
+    // CPML (a, b, 1/kappa + a) of the cell, E side and H side
+    auto stretch = [](const AxisDev &A, int p, int fa, int fb, int fk) {
+        const float a = axv(A, p, fa);
+        return make_float3(a, axv(A, p, fb), axv(A, p, fk) + a);
+    };
+    const float3 cye = stretch(Y, j, AX_AE, AX_BE, AX_KE), cze = stretch(Z, k, AX_AE, AX_BE, AX_KE);
+    const float3 cyh = stretch(Y, j, AX_AH, AX_BH, AX_KH), czh = stretch(Z, k, AX_AH, AX_BH, AX_KH);
+    // LDS slots of the neighbours: the z ones are in the row; the y one behind is the row before,
+    // the y one ahead the next row, but for the tile's last row (grid row jl, its neighbour jln)
+    const bool y_lds = rr + 1 < d.rows && jn == j0 + r;
+    const int jl = __builtin_amdgcn_readfirstlane(min(j0 + d.rows - 2, ny - 1));
+    const int jln = jl + 1 < ny ? jl + 1 : yw;
+    const bool y_rec = rr < d.rows && r > 0 && jr == jl && ye_nb && !y_lds;
+    const ctab_t yl = ctab_row(Y, jln);
+    const int yls = slab_of(jln, ny, Y.lo, Y.hi);
+    const int ty = min(tid + nz, OEM_ADJ_WG - 1), tz = min(tid - k + kn, OEM_ADJ_WG - 1);
+    const int tyb = max(tid - nz, 0), tzb = min(tid - k + kp, OEM_ADJ_WG - 1);
+    const uint32_t vo = 4u * (uint32_t)(j * pz + k), vyn = 4u * (uint32_t)(jln * pz + k);
+    const uint32_t vpy = 4u * (uint32_t)(max(ys, 0) * pz + k);
+    const uint32_t vpyn = 4u * (uint32_t)(max(yls, 0) * pz + k);
+    const uint32_t vpz = 4u * (uint32_t)(j * wz + max(zs, 0));
+    // the class of a cell, and its (ca, cb) pairs from it or from the dense arrays
+    auto cls_at = [&](uint32_t v, int i) -> uint32_t {
+        return MK != 2 ? bld_u16(rC, v >> 1, (uint32_t)i * (plane * 2u)) : 0u;
+    };
+    struct Coef { float ax, bx, ay, by, az, bz; };
+    auto coef = [&](uint32_t c, uint32_t v, int i) {
+        if constexpr (MK == 0) {
+            const float4 u = s_lut[2 * c];
+            const float2 w = *reinterpret_cast<const float2 *>(&s_lut[2 * c + 1]);
+            return Coef{u.x, u.y, u.z, u.w, w.x, w.y};
+        } else if constexpr (MK == 1) {
+            const uint32_t q = c * 32u;
+            return Coef{T::ld(rL, q, 0u),  T::ld(rL, q, 4u),  T::ld(rL, q, 8u),
+                        T::ld(rL, q, 12u), T::ld(rL, q, 16u), T::ld(rL, q, 20u)};
+        } else {
+            const uint32_t id = (uint32_t)i * plane + (v >> 2);
+            return Coef{mat.ca[id], mat.cb[id], mat.ca[nc + id], mat.cb[nc + id],
+                        mat.ca[2 * (size_t)nc + id], mat.cb[2 * (size_t)nc + id]};
+        }
+    };
+    struct EPlane { float l0, l1, l2, p0, p1; Coef c; };
+    auto load_e = [&](int i, uint32_t cls, EPlane &e) {
+        const uint32_t sp = (uint32_t)i * pl4;
+        const int s = slab_of(i, nx, X.lo, X.hi);
+        e.c = coef(cls, vo, i);
+        e.l0 = T::ld(rF, vo, sp);
+        e.l1 = T::ld(rF, vo, sp + cB);
+        e.l2 = T::ld(rF, vo, sp + 2u * cB);
+        if (s >= 0) {
+            e.p0 = T::ld(rP, vo, ox0 + (uint32_t)s * pl4);
+            e.p1 = T::ld(rP, vo, ox1 + (uint32_t)s * pl4);
+        }
+    };
+    // the x terms (t3, t4) of a plane's E side
+    auto x_terms = [&](int i, const EPlane &e, float &q3, float &q4) {
+        const ctab_t t = ctab_row(X, i);
+        const float xpec = t[AX_PEC];
+        const float nu1 = e.c.by * (zpec * xpec) * e.l1;
+        const float nu2 = e.c.bz * (xpec * ypec) * e.l2;
+        q3 = -nu1;
+        q4 = nu2;
+        if (slab_of(i, nx, X.lo, X.hi) >= 0) {
+            const float a = t[AX_AE], ika = t[AX_KE] + a;
+            q3 = a * e.p0 - ika * nu1;
+            q4 = ika * nu2 + a * e.p1;
+        }
+    };
+    auto term_e = [](float q, const Wt &w, float qn) { return q * w.c - q * w.end - qn * w.nb; };
+    auto term_h = [](float q, const Wt &w, float qn) { return q * w.end - q * w.c + qn * w.nb; };
+    const int wrap_hi = cidx_at(X.nxt, nx - 1), wrap_lo = cidx_at(X.prv, 0);
+    const bool top_nb = i1 < nx || (wrap_hi != nx - 1 && cidx_at(X.prv, wrap_hi) == nx - 1);
+    const bool bot_nb = i0 > 0 || (wrap_lo != 0 && cidx_at(X.nxt, wrap_lo) == 0);
+    // plane s of the chunk's march, -1 the one before it and n the one after
+    const int n = i1 - i0, s0 = bot_nb ? -1 : 0, s1 = top_nb ? n : n - 1;
+    auto plane_of = [&](int s) {
+        return s < 0 ? (i0 > 0 ? i0 - 1 : wrap_lo) : i0 + s < nx ? i0 + s : wrap_hi;
+    };
+    // classes, loaded a plane before what they index: of the cell, and of the last row's neighbour
+    uint32_t c1 = cls_at(vo, plane_of(s0)), m0 = y_rec ? cls_at(vyn, plane_of(s0)) : 0u;
+    EPlane cur, nxt;
+    load_e(plane_of(s0), c1, cur);
+    if (s0 < s1) c1 = cls_at(vo, plane_of(s0 + 1));
+    float q3, q4, q3p = 0.f, q4p = 0.f;
+    x_terms(plane_of(s0), cur, q3, q4);
+    for (int s = s0; s < n; ++s) {
+        const bool halo = s < 0;
+        const int i = plane_of(s), in = plane_of(s + 1);
+        const bool xe_nb = s < s1;
+        const uint32_t sp = (uint32_t)i * pl4;
+        const uint32_t sy = (uint32_t)i * syp, sz = (uint32_t)i * szp;
+        const ctab_t xt = ctab_row(X, i);
+        const int xs = slab_of(i, nx, X.lo, X.hi);
+        const uint32_t sx = (uint32_t)max(xs, 0) * pl4;
+        const float xpec = xt[AX_PEC], zx = zpec * xpec, xy = xpec * ypec;
+        // every load of the plane: the next one's E side (its x terms are used here), the rest
+        if (xe_nb) load_e(in, c1, nxt);
+        float h0 = T::ld(rF, vo, sp + 3u * cB), h1 = T::ld(rF, vo, sp + 4u * cB),
+              h2 = T::ld(rF, vo, sp + 5u * cB);
+        float py0, py1, pz0, pz1, hx0, hx1, hy0, hy1, hz0, hz1;
+        if (ys >= 0) {
+            py0 = T::ld(rP, vpy, oy0 + sy); py1 = T::ld(rP, vpy, oy1 + sy);
+            hy0 = T::ld(rP, vpy, pB + oy0 + sy); hy1 = T::ld(rP, vpy, pB + oy1 + sy);
+        }
+        if (zs >= 0) {
+            pz0 = T::ld(rP, vpz, oz0 + sz); pz1 = T::ld(rP, vpz, oz1 + sz);
+            hz0 = T::ld(rP, vpz, pB + oz0 + sz); hz1 = T::ld(rP, vpz, pB + oz1 + sz);
+        }
+        if (xs >= 0) {
+            hx0 = T::ld(rP, vo, pB + ox0 + sx); hx1 = T::ld(rP, vo, pB + ox1 + sx);
+        }
+        float rbx, rbz, rl0, rl2, rp0, rp1;
+        if (y_rec) {
+            const Coef c = coef(m0, vyn, i);
+            rbx = c.bx;
+            rbz = c.bz;
+            rl0 = T::ld(rF, vyn, sp);
+            rl2 = T::ld(rF, vyn, sp + 2u * cB);
+            if (yls >= 0) {
+                rp0 = T::ld(rP, vpyn, oy0 + sy);
+                rp1 = T::ld(rP, vpyn, oy1 + sy);
+            }
+            if (s + 1 < n) m0 = cls_at(vyn, in);
+        }
+        if (s + 2 <= s1) c1 = cls_at(vo, plane_of(s + 2));
+        // E transpose: nu_c = cb_c pec_c lE_c and the cell's terms, sgn nu outside the slabs and
+        // (1/kappa + a) sgn nu + a psi in them
+        const float nu0 = cur.c.bx * yz * cur.l0;
+        const float nu1 = cur.c.by * zx * cur.l1;
+        const float nu2 = cur.c.bz * xy * cur.l2;
+        float e0 = nu0, e5 = -nu2, e1 = -nu0, e2 = nu1;
+        if (ys >= 0) {
+            e0 = cye.z * nu0 + cye.x * py0;
+            e5 = cye.x * py1 - cye.z * nu2;
+        }
+        if (zs >= 0) {
+            e1 = cze.x * pz0 - cze.z * nu0;
+            e2 = cze.z * nu1 + cze.x * pz1;
+        }
+        s_e[0][tid] = e0;
+        s_e[1][tid] = e5;
+        s_e[2][tid] = e1;
+        s_e[3][tid] = e2;
+        float q0n = 0.f, q5n = 0.f;
+        if (y_rec) {
+            const float lp = yl[AX_PEC];
+            const float n0 = rbx * (lp * zpec) * rl0, n2 = rbz * (xpec * lp) * rl2;
+            q0n = n0;
+            q5n = -n2;
+            if (yls >= 0) {
+                const float a = yl[AX_AE], ika = yl[AX_KE] + a;
+                q0n = ika * n0 + a * rp0;
+                q5n = a * rp1 - ika * n2;
+            }
+        }
+        float q3n = 0.f, q4n = 0.f;
+        if (xe_nb) x_terms(in, nxt, q3n, q4n);
+        __syncthreads();
+        if (y_lds) {
+            q0n = s_e[0][ty];
+            q5n = s_e[1][ty];
+        }
+        const float q1n = s_e[2][tz], q2n = s_e[3][tz];
+        {
+            const ctab_t xn = ctab_row(X, in);
+            const bool x_lo = cidx_at(X.prv, i) == i;
+            const Wt xe{xt[AX_IDLD], x_lo ? xt[AX_MPV] * xt[AX_IDLD] : 0.f,
+                        xe_nb ? xn[AX_MPV] * xn[AX_IDLD] : 0.f};
+            h0 += term_e(e2, ze, q2n) + term_e(e5, ye, q5n);
+            h1 += term_e(e1, ze, q1n) + term_e(q4, xe, q4n);
+            h2 += term_e(e0, ye, q0n) + term_e(q3, xe, q3n);
+        }
+        // H transpose from the new lambda_H: f = -ch sgn lH_c
+        const float f1 = mch * h1, f2 = mch * h2;
+        float g3 = -f1, g4 = f2;
+        if (xs >= 0) {
+            const float a = xt[AX_AH], ika = xt[AX_KH] + a;
+            g3 = a * hx0 - ika * f1;
+            g4 = ika * f2 + a * hx1;
+        }
+        if (!halo) {
+            const float f0 = mch * h0;
+            float g0 = f0, g5 = -f2, g1 = -f0, g2 = f1;
+            if (ys >= 0) {
+                g0 = cyh.z * f0 + cyh.x * hy0;
+                g5 = cyh.x * hy1 - cyh.z * f2;
+            }
+            if (zs >= 0) {
+                g1 = czh.x * hz0 - czh.z * f0;
+                g2 = czh.z * f1 + czh.x * hz1;
+            }
+            s_h[0][tid] = g0;
+            s_h[1][tid] = g5;
+            s_h[2][tid] = g1;
+            s_h[3][tid] = g2;
+            __syncthreads();
+            const float g0n = s_h[0][tyb], g5n = s_h[1][tyb], g1n = s_h[2][tzb], g2n = s_h[3][tzb];
+            const bool x_hi = cidx_at(X.nxt, i) == i;
+            const ctab_t xp = ctab_row(X, i > 0 ? i - 1 : wrap_lo);
+            const Wt xh{xt[AX_IDLP], x_hi ? xt[AX_MNX] * xt[AX_IDLP] : 0.f,
+                        s > 0 || bot_nb ? xp[AX_MNX] * xp[AX_IDLP] : 0.f};
+            const float a0 = term_h(g2, zh, g2n) + term_h(g5, yh, g5n);
+            const float a1 = term_h(g1, zh, g1n) + term_h(g4, xh, q4p);
+            const float a2 = term_h(g0, yh, g0n) + term_h(g3, xh, q3p);
+            if (act) {
+                T::template st<AUX>(rFn, h0, vo, sp + 3u * cB);
+                T::template st<AUX>(rFn, h1, vo, sp + 4u * cB);
+                T::template st<AUX>(rFn, h2, vo, sp + 5u * cB);
+                // lambda_E <- ca pec lambda_E + the sum
+                T::template st<AUX>(rFn, cur.c.ax * yz * cur.l0 + a0, vo, sp);
+                T::template st<AUX>(rFn, cur.c.ay * zx * cur.l1 + a1, vo, sp + cB);
+                T::template st<AUX>(rFn, cur.c.az * xy * cur.l2 + a2, vo, sp + 2u * cB);
+                // the psi adjoints: lpe <- b (sgn nu + lpe), lph <- b (f + lph)
+                if (xs >= 0) {
+                    const float be = xt[AX_BE], bh = xt[AX_BH];
+                    T::template st<AUX>(rPn, be * (cur.p0 - nu1), vo, ox0 + sx);
+                    T::template st<AUX>(rPn, be * (nu2 + cur.p1), vo, ox1 + sx);
+                    T::template st<AUX>(rPn, bh * (hx0 - f1), vo, pB + ox0 + sx);
+                    T::template st<AUX>(rPn, bh * (f2 + hx1), vo, pB + ox1 + sx);
+                }
+                if (ys >= 0) {
+                    T::template st<AUX>(rPn, cye.y * (nu0 + py0), vpy, oy0 + sy);
+                    T::template st<AUX>(rPn, cye.y * (py1 - nu2), vpy, oy1 + sy);
+                    T::template st<AUX>(rPn, cyh.y * (f0 + hy0), vpy, pB + oy0 + sy);
+                    T::template st<AUX>(rPn, cyh.y * (hy1 - f2), vpy, pB + oy1 + sy);
+                }
+                if (zs >= 0) {
+                    T::template st<AUX>(rPn, cze.y * (pz0 - nu0), vpz, oz0 + sz);
+                    T::template st<AUX>(rPn, cze.y * (nu1 + pz1), vpz, oz1 + sz);
+                    T::template st<AUX>(rPn, czh.y * (hz0 - f0), vpz, pB + oz0 + sz);
+                    T::template st<AUX>(rPn, czh.y * (f1 + hz1), vpz, pB + oz1 + sz);
+                }
+            }
+        } else {
+            __syncthreads();        // the next plane writes s_e
+        }
+        q3p = g3;
+        q4p = g4;
+        q3 = q3n;
+        q4 = q4n;
+        cur = nxt;
+    }
+    // the step before: its objective points and eps gradient, on this work-group's own cells
+    blk_items(tl.obj, lb, [&](int l, int t) {
+        point_group<float>(tl.o.mag[l] ? d.lH_n : d.lE_n, tl.o.p[l], mat, 1.0f, d.ncell, tl.n, t);
+    });
+    blk_items(tl.grad, lb, [&](int, int q) { grad_entry<float>(d.lE_n, tl.g, q, d.ncell); });
 }
 
 // rec[q] = E[comp[q]][cell[q]]
@@ -732,6 +1086,11 @@ struct oem_adjoint_state {
     // adjoint fields, of the field type (two floats per value on complex fields)
     float *lE = nullptr, *lH = nullptr, *lpe = nullptr, *lph = nullptr;
     float *lpe2 = nullptr, *lph2 = nullptr;   // the other halves of the ping-pong
+    float *lE2 = nullptr, *lH2 = nullptr;     // and of the fields', where the transposes are fused
+    // work-group tables of the fused transposes' tail, for this chunk and number of lists
+    BlkTab obj_tab{}, grad_tab{};
+    int tab_chunk = 0;
+    size_t tab_lists = 0;
     // design
     int n_design = 0, max_seg = 0;
     int *d_comp = nullptr, *d_cell = nullptr;
@@ -744,6 +1103,7 @@ struct oem_adjoint_state {
     // objective point lists: E side, H side; the (field, component, cell) keys they touch, and
     // whether every key is touched by one list only (then one launch applies them all)
     std::vector<Points> obj;
+    std::vector<int32_t> cells;      // the design cells (host copy)
     std::unordered_set<uint64_t> obj_keys;
     bool obj_disjoint = true;
     // ADE poles: lambda_P per pole (lambda_Q of the Im E driven state on complex fields), the
@@ -761,6 +1121,22 @@ static int adj_chunk() {
     const char *e = std::getenv("OEM_ADJ_CHUNK");
     const int v = e ? std::atoi(e) : 0;
     return v > 0 ? v : OEM_ADJ_CHUNK;
+}
+
+// Whether the two transposes run as one march: on real fields with masks of 0 and +-1 (k_adj_he
+// folds them), rows of at most OEM_ADJ_FUSE_NZ cells (the halo row is one of 512 / nz) and sets that
+// one buffer resource covers.  64 backward steps with the forward ones, ms with one kernel / two: 96
+// x 96 x 40 2.9 / 3.0, 120 x 120 x 100 4.4 / 5.4, 160 x 160 x 64 5.2 / 6.3, 200 x 200 x 128 12.5 /
+// 12.8, 400 x 400 x 48 21.5 / 22.3; 1000 steps of 120 x 120 x 44 62 / 73.
+static int fuse_rows(const oem_ctx *c) {
+    return std::min({OEM_ADJ_WG / c->dims.nz, OEM_ADJ_ROWS, c->dims.ny + 1});
+}
+static int fuse_tiles(const oem_ctx *c, int rows) { return (c->dims.ny + rows - 2) / (rows - 1); }
+static bool adj_fuses(const oem_ctx *ctx) {
+    const char *e = std::getenv("OEM_ADJ_FUSE");
+    if (e && e[0] == '0') return false;
+    return !ctx->cplx && ctx->unit_masks && ctx->dims.nz <= OEM_ADJ_FUSE_NZ &&
+           24ull * ctx->nst < (1ull << 32) && 8ull * ctx->psi.total < (1ull << 32);
 }
 
 // rec_row[q] = E[comp[q]][cell[q]] of the current state, in the field type
@@ -895,17 +1271,31 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
         if (cb[q] == 0.f) return fail(OEM_EINVAL, "design entry %d has cb = 0 (PEC)", q);
     }
     const size_t nc = ctx->nst, es = ctx->esz;
-    TRY(ctx->alloc(&a->lE, 3 * nc * es, true));
-    TRY(ctx->alloc(&a->lH, 3 * nc * es, true));
-    TRY(ctx->alloc(&a->lpe, (size_t)ctx->psi.total * es, true));
-    TRY(ctx->alloc(&a->lph, (size_t)ctx->psi.total * es, true));
-    TRY(ctx->alloc(&a->lpe2, (size_t)ctx->psi.total * es, true));
-    TRY(ctx->alloc(&a->lph2, (size_t)ctx->psi.total * es, true));
+    // E and H, and the psi of both sides, next to each other (the fused transposes address them
+    // as one)
+    const size_t pt = (size_t)ctx->psi.total * es;
+    TRY(ctx->alloc(&a->lE, 6 * nc * es, true));
+    a->lH = a->lE + 3 * nc * es;
+    TRY(ctx->alloc(&a->lpe, 2 * pt, true));
+    a->lph = a->lpe + pt;
+    TRY(ctx->alloc(&a->lpe2, 2 * pt, true));
+    a->lph2 = a->lpe2 + pt;
     TRY(ctx->upload(&a->d_comp, (const int *)comp, (size_t)n_design));
     std::vector<int> dcell(n_design);
     for (int q = 0; q < n_design; ++q) dcell[q] = (int)ctx->dev_cell(cell[q]);
     TRY(ctx->upload(&a->d_cell, (const int *)dcell.data(), dcell.size()));
     (void)oemi::plan_sweep_record(ctx, cell, n_design, &a->rec_tab);
+    a->cells.assign(cell, cell + n_design);
+    if (adj_fuses(ctx)) {
+        // without the memory for a second set the two kernels step in one
+        float *p = nullptr;
+        if (ctx->alloc(&p, 6 * nc * es, true)) {
+            (void)hipGetLastError();
+        } else {
+            a->lE2 = p;
+            a->lH2 = p + 3 * nc * es;
+        }
+    }
     TRY(ctx->upload(&a->dca, dca, (size_t)n_design));
     TRY(ctx->upload(&a->dcb, dcb, (size_t)n_design));
     TRY(ctx->upload(&a->ca, ca, (size_t)n_design));
@@ -1009,16 +1399,32 @@ extern "C" int oem_adjoint_forward(oem_ctx *ctx, int64_t n_steps) {
 }
 
 // The backward steps over the recorded segment, from its last: the objective points, the ADE
-// transposes, the eps gradient, then the E and H transposes.  F: the field type.
+// transposes, the eps gradient, then the E and H transposes.  F: the field type.  fused: the
+// transposes as one march, whose tail takes the next step's objective points (tl.obj) and gradient
+// (tl.grad) where it has tables for them.
 template <typename F>
-static void back_steps(oem_ctx *ctx, oem_adjoint_state *a, AdjDev &d, const ObjDev &od, bool all,
-                       dim3 tm, dim3 tb) {
-    F *lE = reinterpret_cast<F *>(a->lE), *lH = reinterpret_cast<F *>(a->lH);
+static void back_steps(oem_ctx *ctx, oem_adjoint_state *a, AdjDev &d, AdjTail &tl, bool all,
+                       bool fused, bool plain) {
     const F *rec = reinterpret_cast<const F *>(a->rec);
     const dim3 gb(256), gg((a->n_design + 255) / 256);
+    const ObjDev &od = tl.o;
+    const dim3 tb(OEM_ADJ_TK, OEM_ADJ_TJ);
+    const int cols = ctx->dims.ny * ctx->dims.nz;
+    const dim3 tm((cols + OEM_ADJ_TK * OEM_ADJ_TJ - 1) / (OEM_ADJ_TK * OEM_ADJ_TJ), 1,
+                  (ctx->dims.nx + d.chunk - 1) / d.chunk);
+    auto grad_of = [&](int s) {
+        return GradDev{a->d_comp, a->d_cell, a->dca, a->dcb, a->ca, a->cb,
+                       rec + (size_t)s * a->n_design, rec + (size_t)(s + 1) * a->n_design, a->grad,
+                       a->n_design};
+    };
+    const BlkTab obj = tl.obj, grad = tl.grad;
     for (int s = a->rec_n - 1; s >= 0; --s) {
+        F *lE = reinterpret_cast<F *>(a->lE), *lH = reinterpret_cast<F *>(a->lH);
         const int n = (int)(a->rec_s0 + s);          // forward step n: E^n -> E^{n+1}
-        if (all) {
+        const bool first = s == a->rec_n - 1;
+        if (!first && obj.n) {
+            // taken by the step before's tail
+        } else if (all) {
             if (od.ofs[od.n] > 0)
                 hipLaunchKernelGGL((k_adj_obj_all<F>), dim3((od.ofs[od.n] + 255) / 256), dim3(256),
                                    0, ctx->stream, lE, lH, od, ctx->mat, ctx->nst, n);
@@ -1031,19 +1437,65 @@ static void back_steps(oem_ctx *ctx, oem_adjoint_state *a, AdjDev &d, const ObjD
             hipLaunchKernelGGL((k_adj_disp<F>), dim3((ctx->disp.n_entry + 255) / 256), dim3(256), 0,
                                ctx->stream, lE, ctx->disp, a->lP, a->lQ,
                                reinterpret_cast<F *>(a->pend), a->wnu, ctx->nst);
-        hipLaunchKernelGGL((k_adj_grad<F>), gg, gb, 0, ctx->stream, lE, a->d_comp, a->d_cell,
-                           a->dca, a->dcb, a->ca, a->cb, rec + (size_t)s * a->n_design,
-                           rec + (size_t)(s + 1) * a->n_design, a->n_design, ctx->nst, a->grad);
-        // E transpose: reads lE and lpe, adds to lH, writes the new lpe to the other buffer;
-        // then the H transpose: reads lH and lph, rewrites lE in place as ca pec lE + its
-        // sum, writes the new lph to the other buffer
+        if (first || !grad.n)
+            hipLaunchKernelGGL((k_adj_grad<F>), gg, gb, 0, ctx->stream, lE, grad_of(s), ctx->nst);
         d.lE = a->lE; d.lpe = a->lpe; d.lpe_n = a->lpe2;
-        hipLaunchKernelGGL((k_adj_e1<F>), tm, tb, 0, ctx->stream, d);
+        d.lH = a->lH; d.lph = a->lph; d.lph_n = a->lph2;
+        bool done = false;
+        if constexpr (sizeof(F) == 4) if (fused) {
+            d.lE_n = a->lE2;
+            d.lH_n = a->lH2;
+            tl.n = n - 1;
+            tl.obj = s ? obj : BlkTab{};
+            tl.grad = s ? grad : BlkTab{};
+            if (s) tl.g = grad_of(s - 1);
+#define OEM_ADJ_HE(MKV)                                                                     \
+            if (plain)                                                                        \
+                hipLaunchKernelGGL((k_adj_he<MKV, 0>), dim3(d.nblocks), dim3(OEM_ADJ_WG), 0,  \
+                                   ctx->stream, d, tl);                                       \
+            else                                                                              \
+                hipLaunchKernelGGL((k_adj_he<MKV, OEM_ST_NT>), dim3(d.nblocks),               \
+                                   dim3(OEM_ADJ_WG), 0, ctx->stream, d, tl)
+            const int mk = mat_kind(ctx->mat);
+            if (mk == 0) { OEM_ADJ_HE(0); } else if (mk == 1) { OEM_ADJ_HE(1); } else { OEM_ADJ_HE(2); }
+#undef OEM_ADJ_HE
+            std::swap(a->lE, a->lE2);
+            std::swap(a->lH, a->lH2);
+            done = true;
+        }
+        if (!done) {
+            // E transpose: reads lE and lpe, adds to lH, writes the new lpe to the other buffer;
+            // then the H transpose: reads lH and lph, rewrites lE in place as ca pec lE + its
+            // sum, writes the new lph to the other buffer
+            hipLaunchKernelGGL((k_adj_e1<F>), tm, tb, 0, ctx->stream, d);
+            hipLaunchKernelGGL((k_adj_h1<F>), tm, tb, 0, ctx->stream, d);
+        }
         std::swap(a->lpe, a->lpe2);
-        d.lph = a->lph; d.lph_n = a->lph2;
-        hipLaunchKernelGGL((k_adj_h1<F>), tm, tb, 0, ctx->stream, d);
         std::swap(a->lph, a->lph2);
     }
+}
+
+// The tables of the fused transposes' tail: the objective lists when one launch could apply them
+// all, the design when no ADE transpose comes between them and the gradient.
+static void plan_tail(oem_ctx *ctx, oem_adjoint_state *a, const AdjDev &d) {
+    if (a->tab_chunk == d.chunk && a->tab_lists == a->obj.size()) return;
+    const int ny = ctx->dims.ny, nz = ctx->dims.nz;
+    auto owner = [&](int id) {
+        const int i = id / (ny * nz), j = id % (ny * nz) / nz;
+        return i / d.chunk * d.tiles + j / (d.rows - 1);
+    };
+    a->obj_tab = a->grad_tab = BlkTab{};
+    std::vector<int> n;
+    for (const auto &P : a->obj) n.push_back(P.d.n_groups);
+    bool ok = true;
+    if (!a->obj.empty())
+        ok = build_blk(ctx, d.nblocks, n, [&](int l, int t) { return owner(a->obj[l].cells[t]); },
+                       &a->obj_tab, OEM_ADJ_RESIDENT);
+    if (ok && !ctx->has_disp)
+        (void)build_blk(ctx, d.nblocks, {a->n_design}, [&](int, int t) { return owner(a->cells[t]); },
+                        &a->grad_tab, OEM_ADJ_RESIDENT);
+    a->tab_chunk = d.chunk;
+    a->tab_lists = a->obj.size();
 }
 
 extern "C" int oem_adjoint_back(oem_ctx *ctx, int64_t n_steps) {
@@ -1060,12 +1512,28 @@ extern "C" int oem_adjoint_back(oem_ctx *ctx, int64_t n_steps) {
     d.ch = ctx->dims.ch;
     d.ncell = ctx->nst;
     d.chunk = adj_chunk();
-    const dim3 tb(OEM_ADJ_TK, OEM_ADJ_TJ);
-    const int cols = ctx->dims.ny * ctx->dims.nz;
-    const dim3 tm((cols + OEM_ADJ_TK * OEM_ADJ_TJ - 1) / (OEM_ADJ_TK * OEM_ADJ_TJ), 1,
-                  (ctx->dims.nx + d.chunk - 1) / d.chunk);
+    const bool fused = a->lE2 != nullptr, pick = !std::getenv("OEM_ADJ_CHUNK");
+    bool plain = false;
+    const int nx = ctx->dims.nx;
+    if (!fused && pick) {
+        const int64_t tiles = ((int64_t)ctx->dims.ny * ctx->dims.nz + OEM_ADJ_TK * OEM_ADJ_TJ - 1) /
+                              (OEM_ADJ_TK * OEM_ADJ_TJ);
+        d.chunk = (int)std::min<int64_t>(OEM_ADJ_CHUNK, std::max<int64_t>(2, nx * tiles / OEM_ADJ_BLOCKS));
+    }
+    if (fused) {
+        // one round of work-groups while their chunks are at most 8 planes, else 12 planes (ms
+        // with 8 / 12 / 16: 400 x 400 x 48 21.98 / 21.51 / 21.86)
+        d.rows = fuse_rows(ctx);
+        d.tiles = fuse_tiles(ctx, d.rows);
+        const int64_t one = ((int64_t)nx * d.tiles + OEM_ADJ_RESIDENT - 1) / OEM_ADJ_RESIDENT;
+        if (pick) d.chunk = one > 8 ? 12 : (int)std::max<int64_t>(2, one);
+        d.chunk = std::min(d.chunk, nx);
+        d.nblocks = d.tiles * ((nx + d.chunk - 1) / d.chunk);
+        plain = 48ull * ctx->nst + 16ull * ctx->psi.total <= OEM_ADJ_CACHED;
+    }
     // the objective lists in one launch per step when they touch disjoint cells
-    ObjDev od{};
+    AdjTail tl{};
+    ObjDev &od = tl.o;
     const bool all = a->obj_disjoint && a->obj.size() <= OEM_ADJ_OBJ_MAX &&
                      !(std::getenv("OEM_ADJ_OBJ_ALL") && std::getenv("OEM_ADJ_OBJ_ALL")[0] == '0');
     if (all) {
@@ -1076,10 +1544,15 @@ extern "C" int oem_adjoint_back(oem_ctx *ctx, int64_t n_steps) {
             od.ofs[l + 1] = od.ofs[l] + a->obj[l].d.n_groups;
         }
     }
+    if (fused && all) {
+        plan_tail(ctx, a, d);
+        tl.obj = a->obj_tab;
+        tl.grad = a->grad_tab;
+    }
     if (ctx->cplx)
-        back_steps<cf2>(ctx, a, d, od, all, tm, tb);
+        back_steps<cf2>(ctx, a, d, tl, all, false, false);
     else
-        back_steps<float>(ctx, a, d, od, all, tm, tb);
+        back_steps<float>(ctx, a, d, tl, all, fused, plain);
     HIP_OK(hipGetLastError());
     HIP_OK(hipStreamSynchronize(ctx->stream));
     a->rec_s0 = -1;

@@ -210,6 +210,8 @@ extern "C" int oem_set_axis(oem_ctx *ctx, int32_t axis, const float *idl_p, cons
                          AX_BE,   AX_KE,   AX_AH,  AX_BH,  AX_KH};
     for (int t = 0; t < 11; ++t)
         for (int i = 0; i < n; ++i) tab[(size_t)i * AX_W + fid[t]] = fa[t][i];
+    for (int i = 0; i < n; ++i)
+        for (const float m : {mnx[i], mpv[i]}) ctx->unit_masks &= m == 0.f || m == 1.f || m == -1.f;
     for (int i = 0; i < n; ++i) {
         const float a = mnx_im ? mnx_im[i] : 0.f, b = mpv_im ? mpv_im[i] : 0.f;
         if ((a != 0.f || b != 0.f) && !ctx->cplx)
@@ -833,48 +835,6 @@ static int plan_fused_snaps(oem_ctx *ctx) {
         }
     }
     return OEM_OK;
-}
-
-// The work-groups the chip holds at once, and the share of a larger launch's that may have a tail
-// (build_blk).
-#define OEM_BLK_RESIDENT 1024
-#define OEM_BLK_SHARE 8
-
-// Tables of the items of several lists by the work-group that owns them: blk(l, t) of the n[l]
-// items of list l.  False, and the lists keep their own launches, when out of memory or when too
-// many work-groups would end with a tail of dependent loads: a grid whose work-groups all run at
-// once hides them behind each other (120 x 120 x 44, mode source, planes and design: E sweep 11.2
-// us with 11.8 us of launches after it, 12.5 with the lists), a larger one pays them per round
-// (160^3 with a z plane, in every work-group: 42.7 us against 35.6 and a launch of 5; 400 x 400 x
-// 48 with a 160 x 160 design, in a sixth of them: 99.9 against 79.3 and 5.2).
-template <typename Fn>
-static bool build_blk(oem_ctx *ctx, int nblocks, const std::vector<int> &n, Fn blk, BlkTab *out) {
-    const size_t nl = n.size();
-    std::vector<int> ofs((size_t)nblocks * nl + 1, 0);
-    size_t total = 0;
-    for (size_t l = 0; l < nl; ++l) {
-        for (int t = 0; t < n[l]; ++t) ++ofs[(size_t)blk((int)l, t) * nl + l + 1];
-        total += (size_t)n[l];
-    }
-    if (total > 0x7fffffff) return false;
-    int touched = 0;
-    for (int b = 0; b < nblocks; ++b) {
-        bool any = false;
-        for (size_t l = 0; l < nl; ++l) any |= ofs[(size_t)b * nl + l + 1] != 0;
-        touched += any;
-    }
-    if (nblocks > OEM_BLK_RESIDENT && touched > nblocks / OEM_BLK_SHARE) return false;
-    for (size_t q = 1; q < ofs.size(); ++q) ofs[q] += ofs[q - 1];
-    std::vector<int> at(ofs.begin(), ofs.end() - 1), idx(total);
-    for (size_t l = 0; l < nl; ++l)
-        for (int t = 0; t < n[l]; ++t) idx[at[(size_t)blk((int)l, t) * nl + l]++] = t;
-    int *d_ofs = nullptr, *d_idx = nullptr;
-    if (ctx->upload(&d_ofs, ofs.data(), ofs.size()) || ctx->upload(&d_idx, idx.data(), idx.size())) {
-        (void)hipGetLastError();
-        return false;
-    }
-    *out = BlkTab{(int)nl, d_ofs, d_idx};
-    return true;
 }
 
 // The work-group of the sweeps that owns the cell (i, j, k) (tile_coord).
