@@ -11,7 +11,9 @@
 // cell-local scaling), and the transpose of the H update (gather from the backward neighbour).
 // Each transpose is one kernel that reads the old adjoint fields and writes the new cell-local
 // ones (lambda_E, the psi adjoints) to a second buffer, so no thread reads a value another
-// overwrites; the buffers swap after each kernel.
+// overwrites; the buffers swap after each kernel.  On real fields with short rows both run as one
+// march between two sets of adjoint fields (k_adj_he), whose tail takes the next step's objective
+// points and eps gradient.
 //
 // ADE poles (per entry: component c at a cell, complex pole states P_p driven by the real E)
 // add two cell-local transposes per step, one kernel over the entries before the eps gradient
@@ -1193,7 +1195,15 @@ extern "C" int oem_checkpoint_alloc(oem_ctx *ctx, int32_t n_slots) {
     TRY(adj_check(ctx));
     oem_adjoint_state *a = ctx->adj;
     if (n_slots < 1 || a->n_slots) return fail(OEM_EINVAL, "checkpoint slots %d (once per context)", n_slots);
-    TRY(ctx->alloc(&a->ckpt, (size_t)n_slots * state_floats(ctx), false));
+    int rc = ctx->alloc(&a->ckpt, (size_t)n_slots * state_floats(ctx), false);
+    if (rc && a->lE2) {
+        // give up the second set of the fused transposes for them
+        (void)hipGetLastError();
+        TRY(ctx->release(a->lE2));
+        a->lE2 = a->lH2 = nullptr;
+        rc = ctx->alloc(&a->ckpt, (size_t)n_slots * state_floats(ctx), false);
+    }
+    TRY(rc);
     a->n_slots = n_slots;
     a->ckpt_step.assign(n_slots, -1);
     return OEM_OK;
@@ -1286,16 +1296,6 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
     TRY(ctx->upload(&a->d_cell, (const int *)dcell.data(), dcell.size()));
     (void)oemi::plan_sweep_record(ctx, cell, n_design, &a->rec_tab);
     a->cells.assign(cell, cell + n_design);
-    if (adj_fuses(ctx)) {
-        // without the memory for a second set the two kernels step in one
-        float *p = nullptr;
-        if (ctx->alloc(&p, 6 * nc * es, true)) {
-            (void)hipGetLastError();
-        } else {
-            a->lE2 = p;
-            a->lH2 = p + 3 * nc * es;
-        }
-    }
     TRY(ctx->upload(&a->dca, dca, (size_t)n_design));
     TRY(ctx->upload(&a->dcb, dcb, (size_t)n_design));
     TRY(ctx->upload(&a->ca, ca, (size_t)n_design));
@@ -1311,6 +1311,16 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
         hipLaunchKernelGGL(k_adj_disp_setup, dim3((ne + 255) / 256), dim3(256), 0, ctx->stream,
                            ctx->disp, ctx->mat, ctx->g, ctx->dims.cw, ctx->nst, a->wnu);
         HIP_OK(hipGetLastError());
+    }
+    if (adj_fuses(ctx)) {
+        // last of all: without the memory for a second set the two kernels step in one
+        float *p = nullptr;
+        if (ctx->alloc(&p, 6 * nc * es, true)) {
+            (void)hipGetLastError();
+        } else {
+            a->lE2 = p;
+            a->lH2 = p + 3 * nc * es;
+        }
     }
     a->n_design = n_design;
     a->max_seg = max_seg;

@@ -223,6 +223,17 @@ struct oem_ctx {
         return OEM_OK;
     }
 
+    // give back an allocation of a standalone context
+    int release(void *p) {
+        auto it = std::find(allocs.begin(), allocs.end(), p);
+        if (it == allocs.end()) return OEM_OK;
+        HIP_OK(hipStreamSynchronize(stream));
+        allocs.erase(it);
+        std::lock_guard<std::mutex> hold(oemi::device_sync_mutex());
+        HIP_OK(hipFree(p));
+        return OEM_OK;
+    }
+
     // flat cell of the ABI -> flat cell of the pitched device arrays
     size_t dev_cell(size_t id) const {
         const size_t nz = (size_t)dims.nz;
