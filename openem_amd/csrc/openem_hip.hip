@@ -718,7 +718,8 @@ extern "C" int oem_read_flux_time_monitor(oem_ctx *ctx, int32_t mon_id, double *
     return OEM_OK;
 }
 
-// The E-side point lists as part of the E update when they are a few points (OEM_TAIL=0: never):
+// The E-side point lists as part of the E update when they are a few points, in the march and in the
+// pool's sweeps (a scene's own sweeps take whole lists, plan_sweeps; OEM_TAIL=0: never):
 // a launch of its own that corrects one cell held the step up by 2 to 8 us.  With the counter moved
 // once per captured block, a whole run of a 64^3 box soup went from 44.5 to 42.4 ms, of the 30 x 30
 // x 174 slab (no points) from 28.7 to 26.0, 512 steps of a graded 150 x 133 x 141 from 37.6 to 33.4.
