@@ -654,7 +654,7 @@ struct AdjTail {
 // first a halo row whose lambda_H it recomputes), exchanges the y and z terms of each half through
 // LDS and carries the x terms in registers, so the new lambda_H is used without going through
 // memory (48 bytes a cell instead of 72, and one launch: 120 x 120 x 44 21.5 us a step with the tail
-// below against 24 for the two kernels and 9.6 for their launches, 400 x 400 x 48 165 against 178).
+// below against 24 for the two kernels and 9.6 for their launches, 400 x 400 x 48 157 against 178).
 // The last row's forward neighbour is recomputed from its cell; a chunk starts with the
 // plane before it, for the x terms of its lambda_H alone.  Old and new values are two sets (the
 // halos read old ones that other work-groups replace): fields [lE, lH], psi [lpe, lph].
