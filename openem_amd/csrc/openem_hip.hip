@@ -940,6 +940,24 @@ static uint64_t march_bytes(const oem_ctx *c) {
 // 99 / 93; 512^3 1.74 / 1.70 ms).
 #define OEM_MARCH_CACHED (200ull << 20)
 
+// Whether a small scene's columns use the march's lanes.  The march's tiles are 64 or 32 lanes by 7
+// or 14 rows, the sweeps number the columns of a plane without a gap, so a thin or flat scene idles
+// most of a march: step times march / sweeps (us) by the share of lanes used: 0.03 (1000 x 1000 x 1)
+// 229 / 19, (300 x 300 x 1) 34 / 14; 0.14 (1000 x 1 x 1000) 60 / 19; 0.15 (700 x 700 x 4) 122 / 37;
+// 0.25 (500 x 500 x 8) 68 / 34; 0.37 (400 x 400 x 12) 49 / 32; 0.51 (200 x 200 x 33) 32.6 / 26.9;
+// 0.74 (200 x 200 x 48) 42.8 / 41.5; 0.87 (250 x 250 x 28) 29.4 / 32.4; 0.99 (250 x 250 x 32) 30.4 /
+// 34.9.  From a half on it beats the two launches it replaced with their point, snapshot and counter
+// launches (200 x 200 x 33: 35.2).  Up to half a million lanes a step is launches and latency and
+// the march's single launch wins whatever it idles: 64 x 64 x 1 9.2 / 12.9, 120 x 120 x 16 13.4 /
+// 14.5, 50 x 50 x 33 9.6 / 15.3; 150 x 150 x 8 (0.74 M lanes) 16.6 / 13.1.
+#define OEM_MARCH_LANES 500000
+static bool march_fills(const oem_ctx *c) {
+    GridDev g = c->g;
+    march_tiles(g, mat_kind(c->mat) == 2);
+    const uint64_t lanes = (uint64_t)g.tiles * OEM_CT * (uint64_t)g.nx;
+    return lanes <= OEM_MARCH_LANES || 2 * (uint64_t)c->ncell >= lanes;
+}
+
 // Whether the fused H+E step is the faster form.  It moves two thirds of the sweeps' bytes but
 // alternates between two field sets.  From OEM_FUSE_MIN_CELLS on the bytes decide: 320^3 516 us
 // against 677 with the two sweeps, 512^3 1.70 ms against 2.53.  While its state stays in the
@@ -953,7 +971,7 @@ static bool march_pays(const oem_ctx *c) {
     if (c->ncell >= OEM_FUSE_MIN_CELLS) return true;
     for (const auto &p : c->points)
         if (p.magnetic) return false;
-    return march_bytes(c) <= OEM_MARCH_CACHED;
+    return march_bytes(c) <= OEM_MARCH_CACHED && march_fills(c);
 }
 
 extern "C" int oem_prepare(oem_ctx *ctx) {
