@@ -3,8 +3,9 @@ kernels whose lanes they would leave idle, and the values of both forms on them.
 
 import numpy as np
 import pytest
+import torch
 
-from openem_amd import cpml, grid, model, scenes, tables, waveform
+from openem_amd import _lib, adjoint, cpml, grid, model, scenes, tables, waveform
 from openem_amd.solver import Stepper
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +66,51 @@ def test_both_forms_agree_on_flat_scenes(gpu_lib, shape):
             st.close()
     for a, b in zip(*out):
         assert np.isfinite(b).all() and np.array_equal(a, b)
+
+
+def _setup_bytes(shape):
+    """Device memory that oem_adjoint_setup takes (the fused transposes keep a second field set)."""
+    st = Stepper(tables.build(_scene(shape)), form="sweeps")
+    try:
+        cell = np.array([int(np.prod(shape)) // 2], np.int32)
+        comp = np.array([2], np.int32)
+        co = adjoint.design_coefficients(st.tabs, comp, cell)
+        before = torch.cuda.mem_get_info()[0]
+        _lib.check(st.lib, st.lib.oem_adjoint_setup(st.ctx, 1, _lib.ptr(comp), _lib.ptr(cell),
+                                                    *[_lib.ptr(x) for x in co], 4))
+        return before - torch.cuda.mem_get_info()[0]
+    finally:
+        st.close()
+
+
+# the share of the fused transposes' lanes in use: 0.12, 0.23, 0.37, 0.25 with more than two million
+# of them; 0.12 with fewer, 0.73
+@pytest.mark.parametrize("shape,fused", [
+    ((1000, 1000, 1), False), ((700, 700, 2), False), ((1000, 1000, 3), False),
+    ((8000, 1, 128), False), ((400, 400, 1), True), ((500, 500, 6), True)])
+def test_transposes_form_by_lane_use(gpu_lib, monkeypatch, shape, fused):
+    monkeypatch.delenv("OEM_ADJ_FUSE", raising=False)
+    default = _setup_bytes(shape)
+    monkeypatch.setenv("OEM_ADJ_FUSE", "0")
+    two = _setup_bytes(shape)
+    second = 24 * int(np.prod(shape))               # the set's bytes; allocations round up to 2 MiB
+    assert (default - two > second / 2) == fused, (default, two, second)
+
+
+# few rows, few cells a row: where the halo row, the wrap and the clamp of a tile meet
+@pytest.mark.parametrize("shape", [(45, 41, 1), (45, 1, 41), (60, 2, 50), (1, 45, 41), (43, 44, 3),
+                                   (50, 3, 2)])
+def test_fused_transposes_on_flat_grids(gpu_lib, monkeypatch, shape):
+    sc = _scene(shape, steps=60)
+    rng = np.random.default_rng(5)
+    cell = rng.choice(int(np.prod(shape)), 30, replace=False)
+    comp = rng.integers(3, size=30)
+    m = tables.build(sc).monitors[0]
+    K = rng.standard_normal((4, m.n1, m.n2)) + 1j * rng.standard_normal((4, m.n1, m.n2))
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("OEM_ADJ_FUSE", fuse)
+        out.append(adjoint.overlap_power_gradient(sc, sc.flux_monitors[0].name, K, comp, cell))
+    a, b = out
+    assert np.isfinite(b.grad).all() and np.abs(b.grad).max() > 0
+    assert a.J == b.J and np.array_equal(a.grad, b.grad)
