@@ -20,6 +20,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #define OEM_NXCD 8
 #define OEM_MAX_PW 2
@@ -1917,12 +1918,18 @@ __device__ __forceinline__ void dft_acc(double &sr, double &si, cf2 v, double c,
 
 // Replay of one (component, frequency group) of a monitor for the 256 points of a block: a
 // thread per point forms the group's sums over the cnt snapshots from step `first` in step order
-// and adds them to the accumulators.  The time of a small monitor was the chain of a load and a
-// scalar phase read per step (22-29 us for 16 steps whatever its size, once per monitor), so the
-// phases are staged in LDS and 16 snapshots are in flight before the first is used: three flux
-// planes of 64^3 went from 47 to 8.5 us a batch in one launch, of 256^3 from 65 to 34.
+// and adds them to the accumulators.  A small monitor is a chain of loads (one per step and a scalar
+// phase read each: 22-29 us for 16 steps whatever its size), so the phases are staged in LDS and
+// several snapshots are in flight before the first is used: 8 real or 4 complex ones, then 4, 2, 1 for
+// the rest of a short batch.  A large monitor is bound by its accumulators' traffic and needs waves
+// to cover it, so a thread stays within 64 registers (8 waves a SIMD).  us a batch with a chain per
+// step at 8 waves / 16 in flight and the rest one by one at 5 (real) or 3 (complex) waves / this:
+// 64^3, 3 planes x 9 frequencies, 16 steps 83 / 15 / 13; 2 x 512 x 512 cells x 8, 16 steps 217 / 206 /
+// 174, 10 steps 180 / 214 / 153, 1 step 123 / 154 / 125; complex 4 planes of 256 x 256 x 21, 16 steps 293
+// / 290 / 164, 10 steps 236 / 290 / 141, 1 step 146 / 202 / 116, 64 steps 822 / 590 / 437.
 #define OEM_FLUSH_FG 8          // frequencies of a group: each snapshot is read once per group
 #define OEM_FLUSH_BLK 256
+#define OEM_FLUSH_WAVES 8       // waves per SIMD that its registers leave room for
 // G: the group's frequencies, rounded up to 1, 2, 4 or 8 (the phases past nfl are zero)
 template <typename F, int G>
 __device__ __forceinline__ void flush_sums(const MonDev &m, int c, int f0, int nfl, int q,
@@ -1935,24 +1942,32 @@ __device__ __forceinline__ void flush_sums(const MonDev &m, int c, int f0, int n
     const size_t row = (size_t)m.ncomp * m.npts;
     const F *col = static_cast<const F *>(m.snap) + (size_t)c * m.npts + q;
     int slot = first % m.T, s = 0;
-    for (; s + 16 <= cnt; s += 16) {
-        F v[16];
+    // N snapshots in flight, then their terms in step order, two frequencies' phases at a time (the
+    // compiler would read all of them ahead)
+    auto take = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        F v[N];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
+        for (int e = 0; e < N; ++e) {
             v[e] = col[(size_t)slot * row];
             slot = slot + 1 == m.T ? 0 : slot + 1;
         }
 #pragma unroll
-        for (int e = 0; e < 16; ++e)
+        for (int e = 0; e < N; ++e) {
 #pragma unroll
-            for (int u = 0; u < G; ++u) dft_acc(sre[u], sim[u], v[e], ph[s + e][u].x, ph[s + e][u].y);
-    }
-    for (; s < cnt; ++s) {
-        const F v = col[(size_t)slot * row];
-        slot = slot + 1 == m.T ? 0 : slot + 1;
-#pragma unroll
-        for (int u = 0; u < G; ++u) dft_acc(sre[u], sim[u], v, ph[s][u].x, ph[s][u].y);
-    }
+            for (int u = 0; u < G; ++u) {
+                dft_acc(sre[u], sim[u], v[e], ph[s + e][u].x, ph[s + e][u].y);
+                if (u & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        s += N;
+    };
+    constexpr int D = 32 / sizeof(F);
+    while (s + D <= cnt) take(std::integral_constant<int, D>{});
+    if (D > 4 && s + 4 <= cnt) take(std::integral_constant<int, 4>{});
+    if (s + 2 <= cnt) take(std::integral_constant<int, 2>{});
+    if (s < cnt) take(std::integral_constant<int, 1>{});
 #pragma unroll
     for (int u = 0; u < G; ++u)
         if (u < nfl) {
@@ -2001,7 +2016,7 @@ struct FlushDev {
     MonDev m[OEM_FLUSH_MONS];
 };
 template <typename F>
-__global__ void __launch_bounds__(OEM_FLUSH_BLK)
+__global__ void __launch_bounds__(OEM_FLUSH_BLK, OEM_FLUSH_WAVES)
 k_dft_flush(FlushDev d, int cnt, StepRef stp)
 {
     __shared__ double2 s_ph[64][OEM_FLUSH_FG];

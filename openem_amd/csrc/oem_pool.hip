@@ -207,7 +207,7 @@ k_pool_snap(const PoolDev *__restrict__ P, int step)
 }
 
 // After the block: replay the snapshots of each scene's steps of the block.
-__global__ void __launch_bounds__(OEM_FLUSH_BLK)
+__global__ void __launch_bounds__(OEM_FLUSH_BLK, OEM_FLUSH_WAVES)
 k_pool_flush(const PoolDev *__restrict__ P, int T)
 {
     __shared__ double2 s_ph[64][OEM_FLUSH_FG];
