@@ -2008,11 +2008,14 @@ __host__ __device__ __forceinline__ int flush_blocks(const MonDev &m) {
 }
 
 // The monitors of a scene (up to OEM_FLUSH_MONS a launch) replayed together: ofs[t] is the first
-// block of monitor t.  Launched after the step counter advanced past the last snapshot: the cnt
-// snapshots ending at step *stp - 1 are replayed.
+// block of monitor t, base the launch's first.  Launched after the step counter advanced past the last
+// snapshot: the cnt snapshots ending at step *stp - 1 are replayed.  At most OEM_FLUSH_LAUNCH blocks a
+// launch: one grid dimension holds fewer than 2^32 threads, and a monitor's points times its
+// components and frequency groups can be more.
 #define OEM_FLUSH_MONS 8
+#define OEM_FLUSH_LAUNCH (1 << 20)
 struct FlushDev {
-    int n, ofs[OEM_FLUSH_MONS];
+    int n, base, ofs[OEM_FLUSH_MONS];
     MonDev m[OEM_FLUSH_MONS];
 };
 template <typename F>
@@ -2020,7 +2023,8 @@ __global__ void __launch_bounds__(OEM_FLUSH_BLK, OEM_FLUSH_WAVES)
 k_dft_flush(FlushDev d, int cnt, StepRef stp)
 {
     __shared__ double2 s_ph[64][OEM_FLUSH_FG];
+    const int b = d.base + (int)blockIdx.x;
     int t = 0;
-    while (t + 1 < d.n && (int)blockIdx.x >= d.ofs[t + 1]) ++t;
-    flush_block<F>(d.m[t], (int)blockIdx.x - d.ofs[t], step_now(stp) - cnt, cnt, s_ph);
+    while (t + 1 < d.n && b >= d.ofs[t + 1]) ++t;
+    flush_block<F>(d.m[t], b - d.ofs[t], step_now(stp) - cnt, cnt, s_ph);
 }

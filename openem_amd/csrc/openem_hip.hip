@@ -1110,8 +1110,11 @@ int launch_flush_t(oem_ctx *c, int cnt) {
             d.ofs[q] = (int)nb;
             nb += flush_blocks(d.m[q]);
         }
-        hipLaunchKernelGGL((k_dft_flush<F>), dim3((unsigned)nb), dim3(OEM_FLUSH_BLK), 0, c->stream,
-                           d, cnt, StepRef{c->d_step, 0});
+        for (int64_t b = 0; b < nb; b += OEM_FLUSH_LAUNCH) {
+            d.base = (int)b;
+            hipLaunchKernelGGL((k_dft_flush<F>), dim3((unsigned)std::min<int64_t>(nb - b, OEM_FLUSH_LAUNCH)),
+                               dim3(OEM_FLUSH_BLK), 0, c->stream, d, cnt, StepRef{c->d_step, 0});
+        }
     }
     HIP_OK(hipGetLastError());
     return OEM_OK;
