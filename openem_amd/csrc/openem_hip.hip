@@ -974,6 +974,24 @@ static bool march_pays(const oem_ctx *c) {
     return march_bytes(c) <= OEM_MARCH_CACHED && march_fills(c);
 }
 
+// The other field set and H-side psi of the fused step (the E-side psi stays in place); without the
+// memory for both the context is left as it was.
+static int second_set(oem_ctx *ctx) {
+    float *f = nullptr, *p = nullptr;
+    int rc = ctx->alloc(&f, 6 * ctx->nst * ctx->esz, true);
+    if (!rc) rc = ctx->alloc(&p, (size_t)ctx->psi.total * ctx->esz, true);
+    if (rc) {
+        (void)hipGetLastError();
+        if (f) (void)ctx->release(f);
+        return rc;
+    }
+    ctx->E2 = f;
+    ctx->H2 = f + 3 * ctx->nst * ctx->esz;
+    ctx->psi2 = ctx->psi;
+    ctx->psi2.h = p;
+    return OEM_OK;
+}
+
 extern "C" int oem_prepare(oem_ctx *ctx) {
     CHECK_CTX(ctx);
     if (ctx->prepared) return OEM_OK;
@@ -1053,13 +1071,13 @@ extern "C" int oem_prepare(oem_ctx *ctx) {
         return fail(OEM_ENOTSUP, "the fused step addresses a field set with 32-bit offsets");
     fuse &= fits;
     if (fuse) {
-        const size_t nc = ctx->nst;
-        TRY(ctx->alloc(&ctx->E2, 6 * nc * ctx->esz, true));
-        ctx->H2 = ctx->E2 + 3 * nc * ctx->esz;
-        float *pp = nullptr;
-        TRY(ctx->alloc(&pp, (size_t)ctx->psi.total * ctx->esz, true));
-        ctx->psi2 = ctx->psi;       // the E-side psi stays in place
-        ctx->psi2.h = pp;
+        const int rc = second_set(ctx);
+        // a small scene does not need the march: with room for one field set only it takes the sweeps
+        const bool asked = ctx->form_req == 2 || (fe && fe[0] == '1');
+        if (rc && (asked || ctx->ncell >= OEM_FUSE_MIN_CELLS)) return rc;
+        fuse = !rc;
+    }
+    if (fuse) {
         HIP_OK(hipStreamSynchronize(ctx->stream));
         ctx->fg = g;
         march_tiles(ctx->fg, mat_kind(ctx->mat) == 2);
