@@ -1210,7 +1210,6 @@ extern "C" int oem_checkpoint_alloc(oem_ctx *ctx, int32_t n_slots) {
     int rc = ctx->alloc(&a->ckpt, (size_t)n_slots * state_floats(ctx), false);
     if (rc && a->lE2) {
         // give up the second set of the fused transposes for them
-        (void)hipGetLastError();
         TRY(ctx->release(a->lE2));
         a->lE2 = a->lH2 = nullptr;
         rc = ctx->alloc(&a->ckpt, (size_t)n_slots * state_floats(ctx), false);
@@ -1327,9 +1326,7 @@ extern "C" int oem_adjoint_setup(oem_ctx *ctx, int32_t n_design, const int32_t *
     if (adj_fuses(ctx)) {
         // last of all: without the memory for a second set the two kernels step in one
         float *p = nullptr;
-        if (ctx->alloc(&p, 6 * nc * es, true)) {
-            (void)hipGetLastError();
-        } else {
+        if (!ctx->alloc(&p, 6 * nc * es, true)) {
             a->lE2 = p;
             a->lH2 = p + 3 * nc * es;
         }

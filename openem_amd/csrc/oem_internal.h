@@ -215,7 +215,12 @@ struct oem_ctx {
             TRY(oemi::pool_arena_alloc(pool, n * sizeof(T), &p));
         } else {
             std::lock_guard<std::mutex> hold(oemi::device_sync_mutex());
-            HIP_OK(hipMalloc(&p, n * sizeof(T)));
+            const hipError_t e = hipMalloc(&p, n * sizeof(T));
+            if (e != hipSuccess) {
+                (void)hipGetLastError();    // reported here, not by the thread's next launch check
+                return fail(e == hipErrorOutOfMemory ? OEM_ENOMEM : OEM_EHIP, "hipMalloc of %zu bytes: %s",
+                            n * sizeof(T), hipGetErrorString(e));
+            }
         }
         allocs.push_back(p);
         if (zero) HIP_OK(hipMemsetAsync(p, 0, n * sizeof(T), stream));
@@ -306,10 +311,8 @@ bool build_blk(oem_ctx *ctx, int nblocks, const std::vector<int> &n, Fn blk, Blk
     for (size_t l = 0; l < nl; ++l)
         for (int t = 0; t < n[l]; ++t) idx[at[(size_t)blk((int)l, t) * nl + l]++] = t;
     int *d_ofs = nullptr, *d_idx = nullptr;
-    if (ctx->upload(&d_ofs, ofs.data(), ofs.size()) || ctx->upload(&d_idx, idx.data(), idx.size())) {
-        (void)hipGetLastError();
+    if (ctx->upload(&d_ofs, ofs.data(), ofs.size()) || ctx->upload(&d_idx, idx.data(), idx.size()))
         return false;
-    }
     *out = BlkTab{(int)nl, d_ofs, d_idx};
     return true;
 }

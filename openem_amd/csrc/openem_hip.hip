@@ -981,7 +981,6 @@ static int second_set(oem_ctx *ctx) {
     int rc = ctx->alloc(&f, 6 * ctx->nst * ctx->esz, true);
     if (!rc) rc = ctx->alloc(&p, (size_t)ctx->psi.total * ctx->esz, true);
     if (rc) {
-        (void)hipGetLastError();
         if (f) (void)ctx->release(f);
         return rc;
     }

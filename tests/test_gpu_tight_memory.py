@@ -1,5 +1,5 @@
-"""GPU test of a small scene on a nearly full device: the fused step's second field set is optional
-below the size from which every scene takes it."""
+"""GPU tests of small scenes on a nearly full device: the fused step's second field set is optional
+below the size from which every scene takes it, and a failed allocation is reported once."""
 
 import gc
 
@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from openem_amd import scenes, tables
+from openem_amd import _lib, scenes, tables
 from openem_amd.solver import Stepper
 
 pytestmark = pytest.mark.gpu
@@ -18,6 +18,15 @@ def _free():
     gc.collect()
     torch.cuda.empty_cache()
     return torch.cuda.mem_get_info()[0]
+
+
+def _fill(leave):
+    """Blocks that leave about ``leave`` bytes of the device (the large one frees some of its own
+    bookkeeping, so the rest goes in smaller ones)."""
+    hold = [torch.empty(_free() - (4 << 30), dtype=torch.uint8, device="cuda")]
+    while (left := torch.cuda.mem_get_info()[0] - leave) >= 4 << 20:
+        hold.append(torch.empty(left, dtype=torch.uint8, device="cuda"))
+    return hold
 
 
 def _run(st):
@@ -43,11 +52,8 @@ def test_small_scene_without_room_for_two_field_sets(gpu_lib, monkeypatch):
     st = Stepper(tabs)
     assert st.launch["form"] == "fused"
     st.close()
-    # one field set and its tables fit, half a set is left; the large block frees some of its own
-    # bookkeeping, so the rest goes in smaller ones
-    leave, hold = one + field_set // 2, [torch.empty(_free() - (4 << 30), dtype=torch.uint8, device="cuda")]
-    while (left := torch.cuda.mem_get_info()[0] - leave) >= 4 << 20:
-        hold.append(torch.empty(left, dtype=torch.uint8, device="cuda"))
+    # one field set and its tables fit, half a set is left
+    hold = _fill(one + field_set // 2)
     try:
         st = Stepper(tabs)
         form = st.launch["form"]
@@ -57,3 +63,18 @@ def test_small_scene_without_room_for_two_field_sets(gpu_lib, monkeypatch):
     assert form == "sweeps"
     for a, b in zip(_run(st), want):
         assert np.abs(b).max() > 0 and np.array_equal(a, b)
+
+
+def test_a_failed_allocation_is_reported_once(gpu_lib):
+    sc = scenes.mini_scene(shape=(16, 17, 40), num_steps=N)
+    st = Stepper(tables.build(sc))
+    big = tables.build(scenes.mini_scene(shape=(140, 138, 136), num_steps=N, field_box=False))
+    hold = _fill(32 << 20)
+    try:
+        with pytest.raises(_lib.OpenEMError) as e:
+            Stepper(big)
+        assert e.value.code == _lib.OEM_ENOMEM
+    finally:
+        del hold
+        _free()
+    assert np.abs(_run(st)[2]).max() > 0            # the other context's launches did not fail
