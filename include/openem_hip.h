@@ -201,12 +201,14 @@ int oem_read_flux_time_monitor(oem_ctx *ctx, int32_t mon_id, double *out, size_t
  * `openem/knobs.py:64`); set by the launch autotuner (openem_amd/autotune.py). */
 int oem_set_chunk(oem_ctx *ctx, int32_t chunk);
 
-/* Step form: 0 = the library's choice (the fused H+E march from 10 M cells, and below that
- * while the state of two steps stays in the memory-side cache and no point list corrects H, else
- * the two sweeps; OEM_FUSE=0/1 forces one), 1 = the two sweeps, 2 = the fused march (OEM_ENOTSUP when a
- * field set exceeds its 32-bit offsets or the context is pooled).  Before oem_prepare.  No
- * counterpart in the reference (its H+E fusion is a global knob, `openem/knobs.py:61`); set by
- * the launch autotuner (openem_amd/autotune.py) together with oem_set_chunk. */
+/* Step form: 0 = the library's choice (the fused H+E march from 10 M cells, and below that while the
+ * state of two steps stays in the memory-side cache, most of its lanes have a cell and no point list
+ * corrects H, else the two sweeps; OEM_FUSE=0/1 forces one), 1 = the two sweeps, 2 = the fused march
+ * (OEM_ENOTSUP when a field set exceeds its 32-bit offsets or the context is pooled).  Before
+ * oem_prepare, and best right after oem_ctx_create: the device rows are laid out for the form (padded
+ * for the march alone).  No counterpart in the reference (its H+E fusion is a global knob,
+ * `openem/knobs.py:61`); set by the launch autotuner (openem_amd/autotune.py) together with
+ * oem_set_chunk. */
 int oem_set_step_form(oem_ctx *ctx, int32_t form);
 
 /* The launch plan oem_prepare chose: form 1 (two sweeps) or 2 (fused) and its x chunk. */

@@ -132,6 +132,8 @@ struct oem_ctx {
     size_t ncell = 0;           // cells of the grid (the ABI's flat index space)
     int pz = 0;                 // row pitch of the device arrays (row_pitch)
     size_t nst = 0;             // cells of one device component, nx*ny*pz
+    size_t n_laid = 0;          // allocations up to the fields' (lay_out)
+    bool written = false;       // oem_write_field was called
     float *stage = nullptr;     // dense rows of a padded field on their way to or from the host
     bool cplx = false;          // Bloch: complex fields, (re, im) interleaved
     size_t esz = 1;             // floats per field element
@@ -317,8 +319,8 @@ bool build_blk(oem_ctx *ctx, int nblocks, const std::vector<int> &n, Fn blk, Blk
     return true;
 }
 
-// Row pitch (cells) of a context's device arrays, chosen from the dimensions alone.
-int row_pitch(const oem_dims *d, bool pooled);
+// Row pitch (cells) of a context's device arrays, from the dimensions and the step form requested.
+int row_pitch(const oem_dims *d, bool pooled, int form);
 
 // Shared by oem_ctx_create and oem_pool_ctx_create: validate dims and allocate the fields,
 // psi slabs and counters of a context (through the pool's arena when ctx->pool is set).

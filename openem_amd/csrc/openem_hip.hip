@@ -55,26 +55,82 @@ static size_t psi_cells(const oem_dims *d, size_t pz) {
 // partial lines: 250 x 230 x 210 (840-byte rows) stepped in 320 us, with 896-byte rows in 246;
 // 256 x 256 x 250 in 399 and 297; 256 x 256 x 240 (960-byte rows, aligned to 64 bytes) in 296 and
 // 274.  Scenes below the fused step's size keep their rows back to back: the sweeps walk the
-// columns of such a plane without a gap (padded they took 291 against 279 us at 250 x 230 x 210).
-int row_pitch(const oem_dims *d, bool pooled) {
+// columns of such a plane without a gap (padded they took 291 against 279 us at 250 x 230 x 210), and
+// so do scenes that the march cannot step (its field set and psi exceed 32-bit offsets) or was not
+// asked to (form: the step form requested so far).
+int row_pitch(const oem_dims *d, bool pooled, int form) {
     const int esz = d->complex_fields ? 2 : 1;
     const int al = 128 / (4 * esz);
     const int pz = (d->nz + al - 1) / al * al;
     const char *re = std::getenv("OEM_ROW_PAD");   // "0": never, "1": any size outside a pool
     const bool forced = re && re[0] == '1';
     if (pooled || (re && re[0] == '0')) return d->nz;
-    if (!forced && ((int64_t)d->nx * d->ny * d->nz < OEM_FUSE_MIN_CELLS ||
+    const char *fe = std::getenv("OEM_FUSE");
+    const bool sweeps = form == 1 || (form == 0 && fe && fe[0] == '0');
+    const uint64_t cells = (uint64_t)d->nx * d->ny * pz, b = 4ull * esz;
+    const bool march = !sweeps && 6 * cells * b < (1ull << 32) && 2 * psi_cells(d, pz) * b < (1ull << 32);
+    if (!forced && (!march || (int64_t)d->nx * d->ny * d->nz < OEM_FUSE_MIN_CELLS ||
                     8 * (int64_t)(pz - d->nz) > d->nz))
         return d->nz;
     // no pad that would take the scene past a limit it keeps without it: 32-bit offsets over a
     // component, a psi side, a field set (fused step) and an adjoint field; 30-bit cells
     auto limits = [&](size_t p) {
-        const uint64_t n = (uint64_t)d->nx * d->ny * p, b = 4ull * esz, ps = psi_cells(d, p) * b;
+        const uint64_t n = (uint64_t)d->nx * d->ny * p, ps = psi_cells(d, p) * b;
         return (n * b > 0xffffffffull) | (n > (1ull << 30)) << 1 | (ps > 0xffffffffull) << 2 |
                (6 * n * b >= (1ull << 32)) << 3 | (2 * ps >= (1ull << 32)) << 4 |
                (3 * n * b >= (1ull << 32)) << 5 | (ps >= (1ull << 32)) << 6;
     };
     return limits(pz) == limits(d->nz) ? pz : d->nz;
+}
+
+// The row pitch of a context and its zeroed fields and psi slabs with it.
+static int lay_out(oem_ctx *c) {
+    const oem_dims *d = &c->dims;
+    const size_t pz = c->pz = row_pitch(d, c->pool != nullptr, c->form_req);
+    const size_t nc = c->nst = (size_t)d->nx * d->ny * pz;
+    const size_t slab[3] = {(size_t)(d->pml_lo[0] + d->pml_hi[0]) * d->ny * pz,
+                            (size_t)d->nx * (d->pml_lo[1] + d->pml_hi[1]) * pz,
+                            (size_t)d->nx * d->ny * (d->pml_lo[2] + d->pml_hi[2])};
+    size_t total = 0;
+    for (int a = 0; a < 3; ++a)
+        for (int m = 0; m < 2; ++m) {
+            c->psi.off[2 * a + m] = (uint32_t)total;
+            total += slab[a];
+        }
+    if (total * 4 * c->esz > 0xffffffffull) return fail(OEM_ENOTSUP, "CPML slabs exceed 4 GiB per side");
+    c->psi.total = (uint32_t)(total ? total : 1);
+    // E and H in one allocation (H right after E): a kernel then reaches a whole field set
+    // through one buffer descriptor
+    TRY(c->alloc(&c->E, 6 * nc * c->esz, true));
+    c->H = c->E + 3 * nc * c->esz;
+    float *pp = nullptr;
+    TRY(c->alloc(&pp, 2 * (size_t)c->psi.total * c->esz, true));
+    c->psi.h = pp;
+    c->psi.e = pp + (size_t)c->psi.total * c->esz;
+    c->n_laid = c->allocs.size();
+    HIP_OK(hipStreamSynchronize(c->stream));
+    return OEM_OK;
+}
+
+// The fields laid out anew; without the memory for both they stay as they are.
+static int lay_out_again(oem_ctx *c) {
+    float *E = c->E, *H = c->H;
+    const PsiDev psi = c->psi;
+    const int pz = c->pz;
+    const size_t nst = c->nst, n = c->allocs.size();
+    if (lay_out(c)) {
+        while (c->allocs.size() > n) TRY(c->release(c->allocs.back()));
+        c->E = E;
+        c->H = H;
+        c->psi = psi;
+        c->pz = pz;
+        c->nst = nst;
+    } else {
+        TRY(c->release(E));
+        TRY(c->release(psi.h));
+    }
+    c->n_laid = c->allocs.size();
+    return OEM_OK;
 }
 
 int ctx_init(oem_ctx *c, const oem_dims *d, int32_t device) {
@@ -108,30 +164,8 @@ int ctx_init(oem_ctx *c, const oem_dims *d, int32_t device) {
     if (c->ncell * 4 * c->esz > 0xffffffffull)
         return fail(OEM_ENOTSUP, "%zu cells: one field component exceeds 4 GiB (limit 2^%d cells)",
                     c->ncell, c->cplx ? 29 : 30);
-    const size_t pz = c->pz = row_pitch(d, c->pool != nullptr);
-    const size_t nc = c->nst = (size_t)d->nx * d->ny * pz;
-    const size_t slab[3] = {(size_t)(d->pml_lo[0] + d->pml_hi[0]) * d->ny * pz,
-                            (size_t)d->nx * (d->pml_lo[1] + d->pml_hi[1]) * pz,
-                            (size_t)d->nx * d->ny * (d->pml_lo[2] + d->pml_hi[2])};
-    size_t total = 0;
-    for (int a = 0; a < 3; ++a)
-        for (int m = 0; m < 2; ++m) {
-            c->psi.off[2 * a + m] = (uint32_t)total;
-            total += slab[a];
-        }
-    if (total * 4 * c->esz > 0xffffffffull) return fail(OEM_ENOTSUP, "CPML slabs exceed 4 GiB per side");
-    c->psi.total = (uint32_t)(total ? total : 1);
-    // E and H in one allocation (H right after E): a kernel then reaches a whole field set
-    // through one buffer descriptor
-    TRY(c->alloc(&c->E, 6 * nc * c->esz, true));
-    c->H = c->E + 3 * nc * c->esz;
-    float *pp = nullptr;
-    TRY(c->alloc(&pp, 2 * (size_t)c->psi.total * c->esz, true));
-    c->psi.h = pp;
-    c->psi.e = pp + (size_t)c->psi.total * c->esz;
     TRY(c->alloc(&c->d_step, 2, true));
-    HIP_OK(hipStreamSynchronize(c->stream));
-    return OEM_OK;
+    return lay_out(c);
 }
 
 extern "C" int oem_ctx_create(const oem_dims *d, int32_t device, oem_ctx **out) {
@@ -170,6 +204,10 @@ extern "C" int oem_set_step_form(oem_ctx *ctx, int32_t form) {
     if (form < 0 || form > 2) return fail(OEM_EINVAL, "step form %d", form);
     if (form == 2 && ctx->pool) return fail(OEM_ENOTSUP, "a pooled context steps with the two sweeps");
     ctx->form_req = form;
+    // while nothing is on the device but the zeroed fields their rows follow the form
+    if (ctx->allocs.size() == ctx->n_laid && !ctx->written &&
+        row_pitch(&ctx->dims, ctx->pool != nullptr, form) != ctx->pz)
+        TRY(lay_out_again(ctx));
     return OEM_OK;
 }
 
@@ -1612,5 +1650,6 @@ extern "C" int oem_write_field(oem_ctx *ctx, int32_t comp, const float *in, size
     TRY(field_ptr(ctx, comp, count, &p));
     if (!in) return fail(OEM_EINVAL, "null input");
     if (ctx->attached) return fail(OEM_ESTATE, "context is stepped by its pool");
+    ctx->written = true;
     return copy_field(ctx, p, const_cast<float *>(in), true);
 }
