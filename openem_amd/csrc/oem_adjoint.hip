@@ -1398,19 +1398,13 @@ extern "C" int oem_adjoint_forward(oem_ctx *ctx, int64_t n_steps) {
     if (n_steps < 1 || n_steps > a->max_seg) return fail(OEM_EINVAL, "segment of %lld steps", (long long)n_steps);
     if (ctx->step + n_steps > ctx->dims.n_steps) return fail(OEM_EINVAL, "beyond the step tables");
     // the cached step graph is captured with or without the recording: drop it on both sides
-    if (ctx->graph) {
-        (void)hipGraphExecDestroy(ctx->graph);
-        ctx->graph = nullptr;
-    }
+    ctx->drop_graphs();
     const int64_t s0 = ctx->step;
     gather_design(ctx, a, 0);
     record_hook(ctx, a, s0);
     const int rc = oem_run(ctx, n_steps);
     ctx->rec_hook.on = false;
-    if (ctx->graph) {
-        (void)hipGraphExecDestroy(ctx->graph);
-        ctx->graph = nullptr;
-    }
+    ctx->drop_graphs();
     TRY(rc);
     a->rec_s0 = s0;
     a->rec_n = (int)n_steps;

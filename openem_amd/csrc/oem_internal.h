@@ -186,7 +186,13 @@ struct oem_ctx {
         BlkTab tab{};               // its entries by work-group of the E sweep (n = 0: a launch)
     } rec_hook;
     struct oem_adjoint_state *adj = nullptr;
-    hipGraphExec_t graph = nullptr;
+    hipGraphExec_t graph[2] = {nullptr, nullptr};   // a block's steps, by the parity of its first
+    void drop_graphs() {
+        for (hipGraphExec_t &g : graph) {
+            if (g) (void)hipGraphExecDestroy(g);
+            g = nullptr;
+        }
+    }
     std::vector<void *> allocs;
     oem_reduce_state *red = nullptr;
 
@@ -197,7 +203,7 @@ struct oem_ctx {
     int64_t retire_after = -1;  // memory is reclaimed once this pool block has completed
 
     ~oem_ctx() {
-        if (graph) (void)hipGraphExecDestroy(graph);
+        drop_graphs();
         if (red) oemi::reduce_state_free(red);
         if (adj) oemi::adjoint_state_free(adj);
         // arena ranges before the capture lock: the pool's lock is never taken under it

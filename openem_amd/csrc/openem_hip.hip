@@ -11,8 +11,9 @@
 // with the DFT flushed every dft_batch steps.  Outside a serving pool, update_h and update_e run
 // as one fused kernel (update_he) that ping-pongs between two field sets, the H-side point
 // corrections added to the old H just before it.  Blocks of dft_batch steps aligned to the batch
-// are captured once into a hipGraph and replayed; the device-side step counter lets one graph
-// serve every block (the reference does the same with a CUDA graph, `openem/solver.py:1165-1182`).
+// are captured once into a hipGraph (for odd dft_batch the fused path has one for each field set that a
+// block starts from) and replayed; the device-side step counter lets one graph serve every block (the
+// reference does the same with a CUDA graph, `openem/solver.py:1165-1182`).
 
 #include "oem_internal.h"
 
@@ -1448,9 +1449,10 @@ static int run_steps(oem_ctx *ctx, int64_t n) {
     int64_t left = n;
     while (left > 0) {
         const bool disp_ok = !ctx->has_disp || ctx->pre_ready;
-        if (use_graph && ctx->pending == 0 && ctx->step % T == 0 && left > T && disp_ok &&
-            !(ctx->fused && (T & 1))) {
-            if (!ctx->graph) {
+        if (use_graph && ctx->pending == 0 && ctx->step % T == 0 && left > T && disp_ok) {
+            // on the fused path a block of odd T ends with the other field set: its graphs alternate
+            hipGraphExec_t &graph = ctx->graph[ctx->fused ? ctx->step & 1 : 0];
+            if (!graph) {
                 // no other thread synchronises the device while this stream captures
                 std::lock_guard<std::mutex> hold(oemi::device_sync_mutex());
                 hipGraph_t gr = nullptr;
@@ -1470,14 +1472,14 @@ static int run_steps(oem_ctx *ctx, int64_t n) {
                     return rc;
                 }
                 if (ec != hipSuccess) return fail(OEM_EHIP, "graph capture: %s", hipGetErrorString(ec));
-                hipError_t ei = hipGraphInstantiate(&ctx->graph, gr, nullptr, nullptr, 0);
+                hipError_t ei = hipGraphInstantiate(&graph, gr, nullptr, nullptr, 0);
                 (void)hipGraphDestroy(gr);
                 if (ei != hipSuccess) {
-                    ctx->graph = nullptr;
+                    graph = nullptr;
                     return fail(OEM_EHIP, "graph instantiate: %s", hipGetErrorString(ei));
                 }
             }
-            HIP_OK(hipGraphLaunch(ctx->graph, ctx->stream));
+            HIP_OK(hipGraphLaunch(graph, ctx->stream));
             ctx->step += T;
             left -= T;
         } else {
