@@ -26,9 +26,13 @@ import numpy as np
 
 from . import tables as tables_mod
 
-#: chunk candidates per form (x planes per work-group); the library's defaults are 12 (fused,
-#: real fields), 16 (fused, complex) and a size rule for the sweeps
+#: chunk candidates per form (x planes per work-group), beside the library's own choice for the scene
+#: (size rules: 2 to 12 planes fused on real fields, to 16 on complex ones, 4 and more for the sweeps)
 CHUNKS = {"fused": (8, 12, 16, 24), "sweeps": (16, 32, 64)}
+#: and those of a march under SMALL_CELLS cells, which needs its work-groups (64^3: 17.6 us a step with
+#: 2 planes, 18.5 with 4, 24.9 with 8; 512^3: 2000 us with 8, 1930 with 12)
+SMALL_CHUNKS = (2, 4, 6)
+SMALL_CELLS = 10 << 20
 
 _cache: dict = {}
 _lock = threading.Lock()
@@ -73,9 +77,10 @@ def _store_file(key: str, plan: dict) -> None:
         pass
 
 
-def candidates(tabs: tables_mod.StepTables, default_form: str) -> list:
+def candidates(tabs: tables_mod.StepTables, default_form: str, default_chunk: int = 0) -> list:
     """``(form, chunk)`` pairs to time.  Both forms when they give the same bits, else only the
-    library's default form; the fused march only while a field set fits 32-bit offsets."""
+    library's default form; the fused march only while a field set fits 32-bit offsets; the library's
+    own plan in any case (``default_chunk``: its chunk)."""
     n = int(np.prod(tabs.shape))
     esz = 2 if tabs.bloch else 1
     fused_ok = 6 * n * 4 * esz < (1 << 32)
@@ -85,12 +90,9 @@ def candidates(tabs: tables_mod.StepTables, default_form: str) -> list:
     nx = tabs.shape[0]
     out = []
     for f in forms:
-        seen = set()
-        for c in CHUNKS[f]:
-            c = min(c, nx)
-            if c not in seen:
-                seen.add(c)
-                out.append((f, c))
+        small = SMALL_CHUNKS if f == "fused" and n < SMALL_CELLS else ()
+        own = (default_chunk,) if f == default_form and default_chunk else ()
+        out += [(f, c) for c in dict.fromkeys(min(c, nx) for c in small + CHUNKS[f] + own)]
     return out
 
 
@@ -119,7 +121,7 @@ def tune(tabs: tables_mod.StepTables, device: int = 0, dft_batch: int = 16, step
     if tabs.n_total < need:
         raise ValueError(f"the tables hold {tabs.n_total} steps; tuning steps {need}")
     timings = {}
-    for form, chunk in candidates(tabs, default["form"]):
+    for form, chunk in candidates(tabs, default["form"], default["chunk"]):
         st = Stepper(tabs, device=device, dft_batch=dft_batch, form=form, chunk=chunk)
         try:
             st.run(warmup)
