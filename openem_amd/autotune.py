@@ -38,10 +38,17 @@ _cache: dict = {}
 _lock = threading.Lock()
 
 
+#: of the kernels and rules that plans are timed with; stored plans of another version are not used
+PLAN_VERSION = 2
+
+
 def shape_key(tabs: tables_mod.StepTables) -> str:
-    """What the launch plan depends on: the grid, real or complex fields, the CPML widths."""
+    """What the launch plan depends on: the grid, real or complex fields, the CPML widths, whether a
+    point list corrects H (the step form then decides the rounding, so such scenes share no plan with
+    others) and whether the coefficients are classes or dense (the march's tiles differ)."""
     pml = tuple((a.pml_lo, a.pml_hi) for a in tabs.axes)
-    return f"{tuple(tabs.shape)}|{'c' if tabs.bloch else 'r'}|{pml}"
+    kind = f"{'h' if has_h_points(tabs) else '-'}{'d' if tabs.material_classes() is None else 'l'}"
+    return f"v{PLAN_VERSION}|{tuple(tabs.shape)}|{'c' if tabs.bloch else 'r'}|{pml}|{kind}"
 
 
 def has_h_points(tabs: tables_mod.StepTables) -> bool:
