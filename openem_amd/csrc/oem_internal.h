@@ -279,25 +279,28 @@ struct oem_ctx {
         HIP_OK(hipSetDevice((c)->device));                                     \
     } while (0)
 
-// The work-groups the chip holds at once, and the share of a larger launch's that may have a tail
-// (build_blk).
+// The work-groups the chip holds at once, the share of a larger launch's that may have a tail, and the
+// most items of a table (build_blk).
 #define OEM_BLK_RESIDENT 1024
 #define OEM_BLK_SHARE 8
-
+#define OEM_BLK_ITEMS 320000
 // Tables of the items of several lists by the work-group that owns them: blk(l, t) of the n[l]
 // items of list l.  False, and the lists keep their own launches, when out of memory or when too
 // many work-groups would end with a tail of dependent loads: a grid whose work-groups all run at
 // once hides them behind each other (120 x 120 x 44, mode source, planes and design: E sweep 11.2
 // us with 11.8 us of launches after it, 12.5 with the lists), a larger one pays them per round
 // (160^3 with a z plane, in every work-group: 42.7 us against 35.6 and a launch of 5; 400 x 400 x
-// 48 with a 160 x 160 design, in a sixth of them: 99.9 against 79.3 and 5.2).
+// 48 with a 160 x 160 design, in a sixth of them: 99.9 against 79.3 and 5.2).  Nor with more than
+// OEM_BLK_ITEMS items: a step saves a launch, 3 us whatever its size, and the tables cost the context
+// 4 to 8 ns an item (TF/SF box of 100^3 with a box monitor of 593,000 points: 49.2 against 46.4 us a
+// step, oem_prepare 4.5 against 10.2 ms; 120^3 with three of 1.1 M 109.7 / 112.5 us, 6.3 / 34.5 ms).
 template <typename Fn>
 bool build_blk(oem_ctx *ctx, int nblocks, const std::vector<int> &n, Fn blk, BlkTab *out,
                int resident = OEM_BLK_RESIDENT) {
     const size_t nl = n.size();
     size_t total = 0;
     for (size_t l = 0; l < nl; ++l) total += (size_t)n[l];
-    if (total > 0x7fffffff) return false;
+    if (total > OEM_BLK_ITEMS) return false;
     // a few thousand of the items first: they mostly tell when there are too many work-groups
     for (const size_t step : {std::max<size_t>(1, total >> 13), (size_t)1}) {
         if (nblocks <= resident) break;
@@ -311,13 +314,18 @@ bool build_blk(oem_ctx *ctx, int nblocks, const std::vector<int> &n, Fn blk, Blk
             }
         if (touched > nblocks / OEM_BLK_SHARE) return false;
     }
-    std::vector<int> ofs((size_t)nblocks * nl + 1, 0);
+    std::vector<int> ofs((size_t)nblocks * nl + 1, 0), row, idx(total);
+    row.reserve(total);
     for (size_t l = 0; l < nl; ++l)
-        for (int t = 0; t < n[l]; ++t) ++ofs[(size_t)blk((int)l, t) * nl + l + 1];
+        for (int t = 0; t < n[l]; ++t) {
+            row.push_back((int)((size_t)blk((int)l, t) * nl + l));
+            ++ofs[(size_t)row.back() + 1];
+        }
     for (size_t q = 1; q < ofs.size(); ++q) ofs[q] += ofs[q - 1];
-    std::vector<int> at(ofs.begin(), ofs.end() - 1), idx(total);
+    std::vector<int> at(ofs.begin(), ofs.end() - 1);
+    size_t q = 0;
     for (size_t l = 0; l < nl; ++l)
-        for (int t = 0; t < n[l]; ++t) idx[at[(size_t)blk((int)l, t) * nl + l]++] = t;
+        for (int t = 0; t < n[l]; ++t) idx[at[row[q++]]++] = t;
     int *d_ofs = nullptr, *d_idx = nullptr;
     if (ctx->upload(&d_ofs, ofs.data(), ofs.size()) || ctx->upload(&d_idx, idx.data(), idx.size()))
         return false;

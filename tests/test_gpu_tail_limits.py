@@ -96,3 +96,45 @@ def test_fused_transposes_past_the_caches(gpu_lib, monkeypatch):
                            lorentz_on=False, pml_xy=True)
     assert 48 * np.prod(sc.shape) > 200 << 20
     _gradients(monkeypatch, sc, "T", 60)
+
+
+# 303,000 points go with the sweeps' work-groups, 343,000 (more than 320,000 items) keep their launch,
+# and so do many of a design (3 x 110,592) in the fused transposes
+@pytest.mark.parametrize("side,own_launch", [(67, False), (70, True)])
+def test_most_points_of_a_table(gpu_lib, monkeypatch, side, own_launch):
+    monkeypatch.delenv("OEM_CHUNK", raising=False)
+    sc = scenes.mini_scene(shape=(80, 78, 76), num_steps=N, pml_xy=True, lorentz_on=False,
+                           field_box=False)
+    f = np.array([2.5e14])
+    sc = replace(sc, flux_monitors=[], field_monitors=[FieldMonitor("b", f, (2, 2, 2), (side,) * 3)])
+    tabs = tables.build(sc)
+    out = []
+    for tail in ("1", "0"):
+        monkeypatch.setenv("OEM_TAIL", tail)
+        st = Stepper(tabs, dft_batch=8, form="sweeps")
+        try:
+            calls = st.profile_run(5)["dft_snap"][1]
+            st.run(N - 5)
+            out.append([st.read_field(c) for c in range(6)] + [st.read_monitor(0)])
+        finally:
+            st.close()
+        assert (calls > 0) == (own_launch or tail == "0")
+    for a, b in zip(*out):
+        assert np.abs(b).max() > 0 and np.array_equal(a, b)
+
+
+def test_large_design_of_the_fused_transposes(gpu_lib, monkeypatch):
+    sc = scenes.mini_scene(shape=(60, 56, 60), num_steps=100, nf=2, field_box=False, lorentz_on=False)
+    t = tables.build(sc)
+    m = t.monitors[[m.name for m in t.monitors].index("T")]
+    rng = np.random.default_rng(4)
+    K = rng.standard_normal((4, m.n1, m.n2)) + 1j * rng.standard_normal((4, m.n1, m.n2))
+    i, j, k = np.meshgrid(*[np.arange(4, 52)] * 3, indexing="ij")
+    cell = np.tile(((i * 56 + j) * 60 + k).ravel(), 3)
+    comp = np.repeat(np.arange(3), i.size)
+    assert cell.size > 320000
+    out = []
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("OEM_ADJ_FUSE", fuse)
+        out.append(adjoint.overlap_power_gradient(sc, "T", K, comp, cell))
+    assert np.abs(out[1].grad).max() > 0 and np.array_equal(out[0].grad, out[1].grad)
