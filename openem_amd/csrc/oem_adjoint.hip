@@ -1269,8 +1269,8 @@ extern "C" int oem_checkpoint_load(oem_ctx *ctx, int32_t slot) {
         return fail(OEM_EINVAL, "checkpoint slot %d is empty", slot);
     ctx->step = a->ckpt_step[slot];
     TRY(copy_state(ctx, a->ckpt + (size_t)slot * state_floats(ctx), false));
-    const int st[2] = {(int)ctx->step, (int)ctx->step};
-    HIP_OK(hipMemcpyAsync(ctx->d_step, st, sizeof(st), hipMemcpyHostToDevice, ctx->stream));
+    const int st = (int)ctx->step;
+    HIP_OK(hipMemcpyAsync(ctx->d_step, &st, sizeof(st), hipMemcpyHostToDevice, ctx->stream));
     HIP_OK(hipStreamSynchronize(ctx->stream));
     ctx->pending = 0;
     ctx->pre_ready = false;

@@ -167,7 +167,7 @@ struct oem_ctx {
     std::vector<Monitor> mons;
     std::vector<TimeMonitor> tmons;
     std::vector<FluxTimeMonitor> ftmons;
-    int *d_step = nullptr;      // [0] steps taken, [1] steps flushed into the DFT accumulators
+    int *d_step = nullptr;      // steps taken, up to the captured or pooled block under way
     int64_t step = 0;
     int pending = 0;
     bool pre_ready = false;     // ADE: hist/P already advanced by the previous fused step

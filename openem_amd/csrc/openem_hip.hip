@@ -8,12 +8,13 @@
 //   update_e (+ plane-wave E correction) -> TF/SF E faces -> electric dipoles -> ADE post
 //   (fused with the next pre) -> DFT snapshots -> step++
 //
-// with the DFT flushed every dft_batch steps.  Outside a serving pool, update_h and update_e run
-// as one fused kernel (update_he) that ping-pongs between two field sets, the H-side point
-// corrections added to the old H just before it.  Blocks of dft_batch steps aligned to the batch
-// are captured once into a hipGraph (for odd dft_batch the fused path has one for each field set that a
-// block starts from) and replayed; the device-side step counter lets one graph serve every block (the
-// reference does the same with a CUDA graph, `openem/solver.py:1165-1182`).
+// with the DFT flushed every dft_batch steps.  Where it is the faster form (march_pays, never in a
+// serving pool) update_h and update_e run as one fused kernel (update_he) that ping-pongs between two
+// field sets, the H-side point corrections added to the old H just before it.  Blocks of dft_batch
+// steps aligned to the batch are captured once into a hipGraph (for odd dft_batch the fused path has
+// one for each field set that a block starts from) and replayed; the device-side step counter lets one
+// graph serve every block (the reference does the same with a CUDA graph,
+// `openem/solver.py:1165-1182`).
 
 #include "oem_internal.h"
 
@@ -165,7 +166,7 @@ int ctx_init(oem_ctx *c, const oem_dims *d, int32_t device) {
     if (c->ncell * 4 * c->esz > 0xffffffffull)
         return fail(OEM_ENOTSUP, "%zu cells: one field component exceeds 4 GiB (limit 2^%d cells)",
                     c->ncell, c->cplx ? 29 : 30);
-    TRY(c->alloc(&c->d_step, 2, true));
+    TRY(c->alloc(&c->d_step, 1, true));
     return lay_out(c);
 }
 
