@@ -1134,17 +1134,18 @@ static int fuse_rows(const oem_ctx *c) {
     return std::min({OEM_ADJ_WG / c->dims.nz, OEM_ADJ_ROWS, c->dims.ny + 1});
 }
 static int fuse_tiles(const oem_ctx *c, int rows) { return (c->dims.ny + rows - 2) / (rows - 1); }
-// And a share of its lanes with a cell of their own of at least a half, or few lanes (a tile has at
-// most OEM_ADJ_ROWS rows, one of them a halo: rows of few cells, or few rows, leave the rest idle).
+// And a share of its lanes with a cell of their own of at least three fifths, or few lanes (a tile has
+// at most OEM_ADJ_ROWS rows, one of them a halo: rows of few cells, or few rows, leave the rest idle).
 // A backward step with one kernel / two (us) by that share: 0.12 (1000 x 1000 x 1) 72 / 35; 0.23 (700
 // x 700 x 2) 47 / 39; 0.25 (8000 x 1 x 128) 48 / 38; 0.37 (1000 x 1000 x 3) 77 / 67; 0.49 (1500 x
-// 1500 x 4) 183 / 138; 0.50 (4000 x 2 x 128) 27 / 34; 0.58 (1200 x 1200 x 5) 143 / 143; 0.73 (500 x
-// 500 x 6) 27 / 48.  Up to two million lanes the single launch wins whatever it idles: 300 x 300 x 1
-// (0.8 M) 13 / 20, 400 x 400 x 2 (1.4 M) 18 / 26, 450 x 450 x 1 (1.8 M) 20.8 / 21.2.
+// 1500 x 4) 183 / 138; 0.58 (1200 x 1200 x 5, adjoint fields everywhere) 152 / 147; 0.73 (500 x 500 x
+// 6) 27 / 48; 0.74 (300 x 300 x 127, fields everywhere) 235 / 269.  Up to two million lanes the single
+// launch wins whatever it idles: 300 x 300 x 1 (0.8 M) 13 / 20, 400 x 400 x 2 (1.4 M) 18 / 26, 450 x
+// 450 x 1 (1.8 M) 20.8 / 21.2.
 #define OEM_ADJ_LANES (2u << 20)
 static bool fuse_fills(const oem_ctx *c) {
     const uint64_t lanes = (uint64_t)fuse_tiles(c, fuse_rows(c)) * OEM_ADJ_WG * (uint64_t)c->dims.nx;
-    return lanes <= OEM_ADJ_LANES || 2 * (uint64_t)c->ncell >= lanes;
+    return lanes <= OEM_ADJ_LANES || 5 * (uint64_t)c->ncell >= 3 * lanes;
 }
 static bool adj_fuses(const oem_ctx *ctx) {
     const char *e = std::getenv("OEM_ADJ_FUSE");

@@ -984,18 +984,20 @@ static uint64_t march_bytes(const oem_ctx *c) {
 // or 14 rows, the sweeps number the columns of a plane without a gap, so a thin or flat scene idles
 // most of a march: step times march / sweeps (us) by the share of lanes used: 0.03 (1000 x 1000 x 1)
 // 229 / 19, (300 x 300 x 1) 34 / 14; 0.14 (1000 x 1 x 1000) 60 / 19; 0.15 (700 x 700 x 4) 122 / 37;
-// 0.25 (500 x 500 x 8) 68 / 34; 0.37 (400 x 400 x 12) 49 / 32; 0.51 (200 x 200 x 33) 32.6 / 26.9;
-// 0.74 (200 x 200 x 48) 42.8 / 41.5; 0.87 (250 x 250 x 28) 29.4 / 32.4; 0.99 (250 x 250 x 32) 30.4 /
-// 34.9.  From a half on it beats the two launches it replaced with their point, snapshot and counter
-// launches (200 x 200 x 33: 35.2).  Up to half a million lanes a step is launches and latency and
-// the march's single launch wins whatever it idles: 64 x 64 x 1 9.2 / 12.9, 120 x 120 x 16 13.4 /
-// 14.5, 50 x 50 x 33 9.6 / 15.3; 150 x 150 x 8 (0.74 M lanes) 16.6 / 13.1.
+// 0.25 (500 x 500 x 8) 68 / 34; 0.37 (400 x 400 x 12) 49 / 32; 0.51 (200 x 200 x 33) 32.9 / 26.9, dense
+// 32.7 / 31.1, (180 x 180 x 65, dense) 60 / 52; 0.60 (112 x 57 x 66, ADE) 26.2 / 25.9.  From three
+// fifths on it goes either way by a tenth (0.65, 160 x 120 x 65, ADE 46.4 / 42.9; 120 x 134 x 131, dense
+// 52 / 57; 0.72, 140 x 100 x 97, dense 37 / 40; 0.74, 95 x 106 x 100, ADE 40.5 / 36.7; 0.79, 97 x 89 x
+// 103, ADE 35.6 / 35.5), then to the march (0.87, 250 x 250 x 28 29.4 / 32.4, 140^3 47 / 55).  Up to half a
+// million lanes a step is launches and latency and the march's single launch wins whatever it idles: 64
+// x 64 x 1 9.2 / 12.9, 120 x 120 x 16 13.4 / 14.5, 50 x 50 x 33 9.6 / 15.3; 150 x 150 x 8 (0.74 M lanes)
+// 16.6 / 13.1.
 #define OEM_MARCH_LANES 500000
 static bool march_fills(const oem_ctx *c) {
     GridDev g = c->g;
     march_tiles(g, mat_kind(c->mat) == 2);
     const uint64_t lanes = (uint64_t)g.tiles * OEM_CT * (uint64_t)g.nx;
-    return lanes <= OEM_MARCH_LANES || 2 * (uint64_t)c->ncell >= lanes;
+    return lanes <= OEM_MARCH_LANES || 5 * (uint64_t)c->ncell >= 3 * lanes;
 }
 
 // Whether the fused H+E step is the faster form.  It moves two thirds of the sweeps' bytes but

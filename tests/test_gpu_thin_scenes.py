@@ -32,11 +32,12 @@ def _scene(shape, steps=40):
                                                   np.ones(1), wf)])
 
 
-# the share of the march's lanes in use: 0.03, 0.24, 0.25, 0.37, 0.14 with over half a million of
-# them; under that, and above a half
+# the share of the march's lanes in use: 0.03, 0.24, 0.25, 0.37, 0.14, 0.51 with over half a million of
+# them; under that, and above three fifths
 @pytest.mark.parametrize("shape,form", [
     ((300, 300, 1), "sweeps"), ((150, 150, 8), "sweeps"), ((500, 500, 8), "sweeps"),
     ((400, 400, 12), "sweeps"), ((1000, 1, 1000), "sweeps"),
+    ((200, 200, 33), "sweeps"),
     ((64, 64, 1), "fused"), ((48, 1, 48), "fused"), ((50, 50, 33), "fused"),
     ((250, 250, 28), "fused"), ((80, 70, 66), "fused")])
 def test_default_form_by_lane_use(gpu_lib, monkeypatch, shape, form):
